@@ -153,8 +153,13 @@ struct AttnLaunch {
   uint32_t* stamp_workgroups;  // out: workgroups launched
 };
 
-// Causal prefill attention on MFMA (a prefill whose positions all see [0,
-// position] in their own slots; int8 cache).  Workgroup = (block of 64 query
+// Causal prefill attention on MFMA (a prefill whose positions sit in their
+// own slots; int8 cache).  With a window, a row sees the sinks [0, sink) and
+// the last `window` positions up to its own, and the workgroup walks only the
+// key blocks one of its rows sees: those of the sinks, then those from the
+// first row's window on.  Keys of these blocks that no row sees may hold
+// anything: their scales are taken as zero and their scores masked.
+// Workgroup = (block of 64 query
 // rows, query head h, KV head h / rep), 16 waves in four groups: wave w
 // takes rows [z0 + 16 (w % 4), +16), lane l the row 16 (w % 4) + l % 16, and
 // group g = w / 4 the key blocks g, g + 4, ... (64 keys each), so each group
@@ -190,18 +195,23 @@ struct PfBuf {
   float vs[kPfKeys];  // v_scale * 2^f
 };
 
+// WIN: the launch has a window to mask (without one the masks and the walk
+// over block pieces fold away: 2048 positions, 8 layers, cost 1.4% more with
+// them).
+template <bool WIN>
 __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     const int8_t* __restrict__ Kc, const int8_t* __restrict__ Vc, const float* __restrict__ Ks,
     const float* __restrict__ Vs, const float* __restrict__ Q, float* __restrict__ out,
     const float* __restrict__ gate, uint32_t gate_ld, uint32_t layer, uint32_t kv_heads,
-    uint32_t alloc, const uint32_t* __restrict__ positions, uint32_t qrows, uint32_t q_heads,
-    uint32_t rep, float score_scale) {
+    uint32_t alloc, uint32_t sink, uint32_t window, const uint32_t* __restrict__ positions,
+    uint32_t qrows, uint32_t q_heads, uint32_t rep, float score_scale) {
   using nd::half8;
   using nd::float4v;
   using nd::u32x2;
   typedef _Float16 half4 __attribute__((ext_vector_type(4)));
   __shared__ __align__(16) PfBuf s_buf[kPfGroups][2];  // [group][buffer]
-  __shared__ uint32_t s_top[kPfThreads / 64];
+  __shared__ uint32_t s_top;
+  __shared__ uint32_t s_low;
   __shared__ float s_vmax[kPfThreads / 64];
   const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const uint32_t grp = wave >> 2, wq = wave & 3, tg = t & 255;
@@ -210,12 +220,22 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
   const uint32_t z0 = blockIdx.x * kPfRows;
   const size_t head_base = ((size_t)layer * kv_heads + kvh) * alloc;
 
-  // Keys [0, top): top = 1 + the largest position of the block's rows.
-  uint32_t my_top = 0;
-  if (t < kPfRows && z0 + t < qrows) my_top = positions[z0 + t] + 1;
+  // Keys below top = 1 + the largest position of the block's rows and, past
+  // the sinks, from low = the first position a row's window holds.
+  if (wave == 0) {
+    const bool in = z0 + t < qrows;
+    const uint32_t p1 = in ? positions[z0 + t] + 1 : 0;
+    [[maybe_unused]] uint32_t my_top = p1, my_low = in ? (WIN && p1 > window ? p1 - window : 0) : 0xffffffffu;
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) my_top = max(my_top, (uint32_t)__shfl_xor((int)my_top, o, 64));
-  if (lane == 0) s_top[wave] = my_top;
+    for (int o = 32; o >= 1; o >>= 1) {
+      my_top = max(my_top, (uint32_t)__shfl_xor((int)my_top, o, 64));
+      if constexpr (WIN) my_low = min(my_low, (uint32_t)__shfl_xor((int)my_low, o, 64));
+    }
+    if (lane == 0) {
+      s_top = my_top;
+      s_low = my_low;
+    }
+  }
   // This lane's query row and its q values: dims 32 s + 8 kb + [0, 8).
   const uint32_t zq = z0 + 16 * wq + r16;
   const bool q_ok = zq < qrows;
@@ -229,17 +249,27 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     qv[s2][0] = a.x; qv[s2][1] = a.y; qv[s2][2] = a.z; qv[s2][3] = a.w;
     qv[s2][4] = b.x; qv[s2][5] = b.y; qv[s2][6] = b.z; qv[s2][7] = b.w;
   }
-  // The smallest position of the wave's rows: blocks wholly below it need no mask.
-  uint32_t wmin = q_ok ? pos : 0;
+  // The row's first windowed position; the smallest position and the largest
+  // such of the wave's rows: blocks wholly between them need no mask.
+  const uint32_t row_low = WIN && pos + 1 > window ? pos + 1 - window : 0;
+  uint32_t wmin = q_ok ? pos : 0, wlow = row_low;
 #pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) wmin = min(wmin, (uint32_t)__shfl_xor((int)wmin, o, 64));
+  for (int o = 8; o >= 1; o >>= 1) {
+    wmin = min(wmin, (uint32_t)__shfl_xor((int)wmin, o, 64));
+    if constexpr (WIN) wlow = max(wlow, (uint32_t)__shfl_xor((int)wlow, o, 64));
+  }
   wmin = __builtin_amdgcn_readfirstlane(wmin);
+  wlow = __builtin_amdgcn_readfirstlane(wlow);
   __syncthreads();
-  uint32_t top = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < kPfThreads / 64; ++w) top = max(top, s_top[w]);
+  const uint32_t top = s_top, low = WIN ? s_low : 0;
   if (top > alloc || top == 0) return;  // validated on entry; stay in bounds
-  const uint32_t nblocks = (top + kPfKeys - 1) / kPfKeys;
+  // Step i walks the keys of block i (i < sblocks: the sinks) or i + skip.
+  uint32_t sblocks = WIN ? (min(sink, top) + kPfKeys - 1) / kPfKeys : 0;
+  if (low / kPfKeys <= sblocks) sblocks = low / kPfKeys;  // contiguous
+  const uint32_t skip = low / kPfKeys - sblocks;
+  const uint32_t nblocks = (top + kPfKeys - 1) / kPfKeys - skip;
+  auto block_key = [&](uint32_t b) { return (b < sblocks ? b : b + skip) * kPfKeys; };
+  auto seen = [&](uint32_t key) { return !WIN || key >= low || key < sink; };
 
   // The split of q: the row maximum over the four lanes holding the row.
   float qmax = 0.f;
@@ -265,7 +295,14 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
 
   // The largest v_scale of the visible keys sets the p' scale 2^f.
   float vmax = 0.f;
-  for (uint32_t k = t; k < top; k += kPfThreads) vmax = fmaxf(vmax, Vs[head_base + k]);
+  if constexpr (WIN) {
+    for (uint32_t i = t; i < nblocks * kPfKeys; i += kPfThreads) {
+      const uint32_t k = block_key(i / kPfKeys) + i % kPfKeys;
+      if (k < top && seen(k)) vmax = fmaxf(vmax, Vs[head_base + k]);
+    }
+  } else {
+    for (uint32_t k = t; k < top; k += kPfThreads) vmax = fmaxf(vmax, Vs[head_base + k]);
+  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
   if (lane == 0) s_vmax[wave] = vmax;
@@ -285,14 +322,16 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
   uint4 kreg, vreg;
   float ksr = 0.f, vsr = 0.f;
   auto load_block = [&](uint32_t b) {
-    const uint32_t key = min(b * kPfKeys + lkey, top - 1);
+    const uint32_t kb0 = block_key(b);
+    const uint32_t key = min(kb0 + lkey, top - 1);
     const size_t row = head_base + key;
     kreg = *reinterpret_cast<const uint4*>(Kc + row * kHeadDim + 16 * lpart);
     vreg = *reinterpret_cast<const uint4*>(Vc + row * kHeadDim + 16 * lpart);
     if (tg < kPfKeys) {
-      const size_t srow = head_base + min(b * kPfKeys + tg, top - 1);
-      ksr = Ks[srow];
-      vsr = Vs[srow];
+      const uint32_t skey = min(kb0 + tg, top - 1);
+      const float kk = Ks[head_base + skey], vv = Vs[head_base + skey];
+      ksr = seen(skey) ? kk : 0.f;
+      vsr = seen(skey) ? vv : 0.f;
     }
   };
   auto store_block = [&](PfBuf& B) {
@@ -327,7 +366,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     PfBuf& B = s_buf[grp][i & 1];
     if (has_next) load_block(b + kPfGroups);
     if (has) {
-      const uint32_t k0 = b * kPfKeys;
+      const uint32_t k0 = block_key(b);
       // S^T tiles j: keys k0 + 16 j + 4 kb + c of this lane's row.
       float4v sc[4];
 #pragma unroll
@@ -341,7 +380,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
           sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[s2], sc[j], 0, 0, 0);
         }
       }
-      const bool masked = k0 + kPfKeys - 1 > wmin;  // uniform over the wave
+      const bool masked = k0 + kPfKeys - 1 > wmin || (WIN && k0 < wlow);  // uniform over the wave
       float bmax = -INFINITY;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -350,7 +389,10 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           float v = (sc[j][c] * ksv[c]) * qup;
-          if (masked) v = (q_ok && k0 + 16 * j + 4 * kb + c <= pos) ? v : -INFINITY;
+          if (masked) {
+            const uint32_t key = k0 + 16 * j + 4 * kb + c;
+            v = (q_ok && key <= pos && (!WIN || key >= row_low || key < sink)) ? v : -INFINITY;
+          }
           sc[j][c] = v;
           bmax = fmaxf(bmax, v);
         }
@@ -486,24 +528,15 @@ hipError_t launch_attention(const AttnLaunch& a, hipStream_t s) {
   }
   if constexpr ((REP == 1 || REP == 2) && !F32) {
     if (a.qblock) {
-      hipLaunchKernelGGL(prefill_attention_mfma_kernel,
+      const uint32_t window = nd_kv_linear(a.kv) ? a.kv->window : 0u;
+      hipLaunchKernelGGL(window ? prefill_attention_mfma_kernel<true>
+                                : prefill_attention_mfma_kernel<false>,
                          dim3((a.batch + kPfRows - 1) / kPfRows, a.seq_kv_heads * REP),
                          dim3(kPfThreads), 0, s, reinterpret_cast<const int8_t*>(a.kv->k),
                          reinterpret_cast<const int8_t*>(a.kv->v), a.kv->ks, a.kv->vs, a.q, a.out,
-                         a.gate, a.gate_ld, a.layer, a.kv->kv_heads, a.kv->alloc, a.positions,
-                         a.batch, a.seq_kv_heads * REP, (uint32_t)REP, 0.125f);
-      return hipGetLastError();
-    }
-    // Query blocks: 4 rows per workgroup (4 positions x 1 head, or 2 x 2).
-    if (a.qblock) {
-      constexpr int kQb = 4;
-      hipLaunchKernelGGL((attention_kernel<kQb, false, true>),
-                         dim3(1, a.seq_kv_heads, (a.batch + kQb / REP - 1) / (kQb / REP)),
-                         dim3(64 * kWaves), 0, s, a.kv->k, a.kv->v, a.kv->ks, a.kv->vs, a.q,
-                         a.out, a.gate, a.gate_ld, nullptr, nullptr, nullptr, a.layer,
-                         a.kv->kv_heads, a.kv->alloc, a.kv->sink, a.kv->window, a.vis,
-                         a.positions, 0u, a.seq_kv_heads, 0u, a.max_count, 1u, 0.125f, a.batch,
-                         (uint32_t)REP, nullptr);
+                         a.gate, a.gate_ld, a.layer, a.kv->kv_heads, a.kv->alloc, a.kv->sink,
+                         window, a.positions, a.batch, a.seq_kv_heads * REP, (uint32_t)REP,
+                         0.125f);
       return hipGetLastError();
     }
   }
@@ -739,9 +772,9 @@ hipError_t nd_launch_attention_batch(const nd_kv* kv, uint32_t layer, const uint
   a.rep = rep;
   a.batch = batch;
   a.max_count = nv.count;
-  // Every position sees [0, position] when no window is outgrown (positions
-  // below the window also sit in their own slots).
-  a.qblock = kv_stride_z == 0 && (kv->window == 0 || max_position < kv->window) &&
+  // Positions sit in their own slots while no window is outgrown (they then
+  // also see all of [0, position]) and in a linear cache.
+  a.qblock = kv_stride_z == 0 && (nd_kv_linear(kv) || max_position < kv->window) &&
              (rep == 1 || rep == 2) && kv->mode != ND_KV_FLOAT32 && batch >= 64;
   return kv->mode == ND_KV_FLOAT32 ? launch_rep<true>(a, s) : launch_rep<false>(a, s);
 }

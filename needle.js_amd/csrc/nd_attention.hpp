@@ -47,13 +47,16 @@ struct Tile {
 // else r0 + wrap(b0 + t - prefix), wrap(x) = x >= w ? x - w : x.  A sliding
 // window (kv_slot) gives r0 = sink, b0 = (recent_low - sink) % window, w =
 // window -- the recent indices span fewer than `window` positions, so one
-// subtraction wraps them -- and no window r0 = recent_low, b0 = 0, w = 2^32 - 1.
+// subtraction wraps them -- and no window, or a linear cache (kv_linear),
+// r0 = recent_low, b0 = 0, w = 2^32 - 1.
 struct Ring {
   uint32_t r0, b0, w;
 };
 
-__device__ __forceinline__ Ring ring_of(const Visible& vis, uint32_t sink, uint32_t window) {
-  if (window == 0 || vis.recent_low < sink) return Ring{vis.recent_low, 0u, 0xffffffffu};
+__device__ __forceinline__ Ring ring_of(const Visible& vis, uint32_t sink, uint32_t window,
+                                        uint32_t alloc) {
+  if (window == 0 || vis.recent_low < sink || alloc > sink + window)
+    return Ring{vis.recent_low, 0u, 0xffffffffu};
   return Ring{sink, (vis.recent_low - sink) % window, window};
 }
 
@@ -377,7 +380,8 @@ __device__ __forceinline__ void attention_body(
     }
   };
   constexpr uint32_t kStride = (uint32_t)KW * kWavePositions;
-  const Ring ring = ring_of(vis, sink, window);
+  // In slot order every index is its slot (below the prefix: ring_slot).
+  const Ring ring = slot_space ? Ring{0u, 0u, 0xffffffffu} : ring_of(vis, sink, window, alloc);
   const uint32_t t_first = c_begin + wave * kWavePositions;
   // Tiles t_first + kStride j, j < n (n uniform), two per round: both tiles'
   // loads are in flight before the first tile's math.  TILES = 1 or 2: the

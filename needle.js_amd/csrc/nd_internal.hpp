@@ -163,6 +163,13 @@ struct nd_visible {
   uint32_t count;       // prefix + position - recent_low + 1
 };
 nd_visible nd_kv_visible(const nd_kv* kv, uint32_t position);
+// A cache whose slot is the position itself although it has a window: a ring
+// never holds more than sink + window slots, so more of them mean one slot
+// per position (the prompt cache of a Needle 2 prefill that outgrows its
+// ring).  Positions the window has passed stay in their slots, unread.
+inline bool nd_kv_linear(const nd_kv* kv) {
+  return kv->window == 0 || kv->alloc > kv->sink + kv->window;
+}
 uint32_t nd_attention_chunks(uint32_t count, uint32_t kv_heads);
 size_t nd_attention_partial_floats(uint32_t q_heads, uint32_t kv_heads, uint32_t count);
 constexpr uint32_t kMaxAttentionKvHeads = 1024;

@@ -37,7 +37,10 @@ namespace {
 constexpr uint32_t kHd = 64;
 constexpr int kWg = 1024;
 constexpr int kMixWg = 512;  // mix kernel: dim <= 512 values per thread role
-constexpr uint32_t kPrefillRows = 512;  // positions per batched prefill pass
+constexpr uint32_t kPrefillRows = 1024;  // positions per batched prefill pass
+// Prompt positions past the ring that take steps instead of a pass over the
+// prompt cache (run_prompt).
+constexpr uint32_t kStepRest = 4;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 using nd::half8;
@@ -2107,8 +2110,12 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
 // one-workgroup parts become one workgroup per position, and causal
 // attention reads the int8 cache, which holds every earlier position because
 // each position's K/V is appended before any attention of the layer runs.
-// It applies while the prompt's cache slots do not wrap (positions < slots),
-// which keeps every position a later query can see in the cache.
+// While the prompt's cache slots do not wrap (positions < slots) the passes
+// work on the ring itself, which keeps every position a later query can see.
+// A prompt that outgrows the ring works on a linear prompt cache, one slot
+// per position and layer: the ring's rows are copied in once, every pass
+// appends to it and attends over each query's own window of it, and the rows
+// the ring keeps are copied back once after the last pass.
 
 // Per position: token from the prompt in `history`, engram hashes, scaled
 // embedding in every lane, concatenated engram rows; workgroup 0 advances the
@@ -2224,6 +2231,33 @@ __global__ __launch_bounds__(64) void n2_rope_store_batch_kernel(
   head_epilogue(val, lane, role, sn, cs, role == 0 ? q_norm[lane] : k_norm[lane],
                 q_out + ((size_t)m * heads + h) * kHd, Kc, Vc, Ks, Vs,
                 ((size_t)layer * kv_heads + h) * alloc, kv_slot(pos, sink, window), alloc, f32);
+}
+
+// Cache rows between the ring and the linear prompt cache: one wave per
+// (row i, KV head, layer), codes (or float32 rows) as `words` 32-bit words
+// and both scales.  Row i of `sinks` is position i, the others positions
+// recent + (i - sinks); to_ring selects the direction.
+__global__ __launch_bounds__(64) void n2_ring_copy_kernel(nd_kv ring, nd_kv lin, uint32_t first,
+                                                          uint32_t sinks, uint32_t recent,
+                                                          uint32_t words, bool to_ring) {
+  const uint32_t i = blockIdx.x, h = blockIdx.y, layer = blockIdx.z, lane = threadIdx.x;
+  const uint32_t pos = i < sinks ? first + i : recent + (i - sinks);
+  const size_t head = (size_t)layer * ring.kv_heads + h;
+  const size_t rr = head * ring.alloc + kv_slot(pos, ring.sink, ring.window);
+  const size_t lr = head * lin.alloc + pos;
+  const nd_kv& src = to_ring ? lin : ring;
+  const nd_kv& dst = to_ring ? ring : lin;
+  const size_t sr = to_ring ? lr : rr, dr = to_ring ? rr : lr;
+  if (lane < words) {
+    reinterpret_cast<uint32_t*>(dst.k)[dr * words + lane] =
+        reinterpret_cast<const uint32_t*>(src.k)[sr * words + lane];
+    reinterpret_cast<uint32_t*>(dst.v)[dr * words + lane] =
+        reinterpret_cast<const uint32_t*>(src.v)[sr * words + lane];
+  }
+  if (lane == 0) {
+    dst.ks[dr] = src.ks[sr];
+    dst.vs[dr] = src.vs[sr];
+  }
 }
 
 // Confidence pool state (OnlineProbePool, runtime.ts:48-62) for up to
@@ -2530,6 +2564,10 @@ struct nd_needle {
   int8_t* pf_digits = nullptr;
   uint32_t *pf_positions = nullptr, *pf_counters = nullptr;
   uint32_t* pf_cq_lookup = nullptr;  // CQ model: each position's engram lookups and token
+  // The linear prompt cache (first prompt that outgrows its ring): max_length
+  // slots per layer and KV head, pf_kv.mode the widest row it holds so far.
+  char* pf_kv_arena = nullptr;
+  nd_kv pf_kv{};
   // Step graphs, valid for (graph_alloc, graph_sink).
   hipGraphExec_t graphs[3] = {nullptr, nullptr, nullptr};
   uint32_t graph_kernels[3] = {0, 0, 0};  // kernel launches each graph holds
@@ -3188,11 +3226,12 @@ nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
 }
 
 // Enqueues `count` prompt tokens (already in history at [position, position
-// + count)) as one batched pass; the host checks that the slots do not wrap
-// and that count <= pf_cap.  want_logits / select: the last position's
-// logits (and selection over all ids) as a step would produce them.
-hipError_t enqueue_prefill(nd_needle* n, uint32_t count, bool want_logits, bool select,
-                           hipStream_t s) {
+// + count)) as one batched pass over the cache kv (the ring, whose slots the
+// host checks not to wrap, or the linear prompt cache); count <= pf_cap.
+// want_logits / select: the last position's logits (and selection over all
+// ids) as a step would produce them.
+hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool want_logits,
+                           bool select, hipStream_t s) {
   const nd_needle_desc& d = n->d;
   const uint32_t D = d.dim, ln = d.lanes, qw = d.heads * kHd, kw = d.kv_heads * kHd;
   const uint32_t M = count, p0 = n->position, N = ln * D;
@@ -3335,11 +3374,10 @@ hipError_t enqueue_prefill(nd_needle* n, uint32_t count, bool want_logits, bool 
     hipLaunchKernelGGL(n2_rope_store_batch_kernel, dim3(d.heads + 2 * d.kv_heads, M), dim3(64), 0,
                        s, n->pf_qkvg, qkv_ld, d.heads, d.kv_heads,
                        n->params + n->o_qn + (size_t)l * kHd, n->params + n->o_kn + (size_t)l * kHd,
-                       n->inv_freq, p0, n->pf_q, n->kv.k, n->kv.v, n->kv.ks, n->kv.vs, l,
-                       n->kv.alloc, n->kv.sink, n->kv.window,
-                       n->kv.mode == ND_KV_FLOAT32 ? 1u : 0u);
+                       n->inv_freq, p0, n->pf_q, kv.k, kv.v, kv.ks, kv.vs, l, kv.alloc, kv.sink,
+                       nd_kv_linear(&kv) ? 0u : kv.window, kv.mode == ND_KV_FLOAT32 ? 1u : 0u);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    e = nd_launch_attention_batch(&n->kv, l, n->pf_positions, M, d.kv_heads, 0u,
+    e = nd_launch_attention_batch(&kv, l, n->pf_positions, M, d.kv_heads, 0u,
                                   d.heads / d.kv_heads, p0 + M - 1, n->pf_q, n->pf_att,
                                   n->pf_partials, n->pf_counters, s, n->pf_qkvg + qw + 2 * kw,
                                   qkv_ld);
@@ -3355,27 +3393,96 @@ hipError_t enqueue_prefill(nd_needle* n, uint32_t count, bool want_logits, bool 
   return nd_launch_select_list(n->logits, d.vocab, nullptr, 0, n->sel_id, n->sel_lp, s);
 }
 
-// Runs the prompt tokens already in history at [position, position + count):
-// batched passes while the cache slots do not wrap, steps after that.  The
-// last token produces logits (and a selection over all ids when select).
+// The linear prompt cache for this reset's cache mode.
+nd_status ensure_prompt_cache(nd_ctx* ctx, nd_needle* n) {
+  const nd_needle_desc& d = n->d;
+  const bool f32 = n->kv.mode == ND_KV_FLOAT32;
+  if (!n->pf_kv_arena || (f32 && n->pf_kv.mode != ND_KV_FLOAT32)) {
+    const size_t rows = (size_t)d.layers * d.kv_heads * d.max_length;
+    const size_t code_bytes = al(rows * kHd * (f32 ? 4 : 1)), scale_bytes = al(rows * 4);
+    if (n->pf_kv_arena) {  // earlier prompts may still read it
+      ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      hipFree(n->pf_kv_arena);
+      n->pf_kv_arena = nullptr;
+    }
+    ND_HIP(ctx, hipMalloc(&n->pf_kv_arena, 2 * (code_bytes + scale_bytes)));
+    n->pf_kv.k = n->pf_kv_arena;
+    n->pf_kv.v = n->pf_kv_arena + code_bytes;
+    n->pf_kv.ks = reinterpret_cast<float*>(n->pf_kv_arena + 2 * code_bytes);
+    n->pf_kv.vs = reinterpret_cast<float*>(n->pf_kv_arena + 2 * code_bytes + scale_bytes);
+    n->pf_kv.mode = n->kv.mode;
+  }
+  return ND_OK;
+}
+
+// Copies rows between the ring and the linear prompt cache lin: positions
+// [first, sink) and the window's last ones, of those below `end`.
+hipError_t enqueue_ring_copy(nd_needle* n, const nd_kv& lin, uint32_t first, uint32_t end,
+                             bool to_ring, hipStream_t s) {
+  const nd_kv& kv = n->kv;
+  const uint32_t sink_end = std::min(kv.sink, end);
+  const uint32_t sinks = sink_end > first ? sink_end - first : 0;
+  const uint32_t recent = std::max(std::max(first, sink_end), end > kv.window ? end - kv.window : 0);
+  const uint32_t rows = sinks + (end - recent);
+  if (!rows) return hipSuccess;
+  const uint32_t words = kv.mode == ND_KV_FLOAT32 ? kHd : kHd / 4;
+  hipLaunchKernelGGL(n2_ring_copy_kernel, dim3(rows, n->d.kv_heads, n->d.layers), dim3(64), 0, s,
+                     kv, lin, first, sinks, recent, words, to_ring);
+  return hipGetLastError();
+}
+
+// Runs the prompt tokens already in history at [position, position + count).
+// The last token produces logits (and a selection over all ids when select).
+// A prompt whose positions fit the ring's slots runs as passes over the ring;
+// one that outgrows it by more than kStepRest positions as passes over the
+// linear prompt cache, with the rows the ring keeps copied back at the end.
+// A rest of up to kStepRest positions takes steps: a pass costs its launches
+// and one trip through the layers however few its rows (about 1.5 ms at 27
+// layers, against 0.46-0.55 ms a step).  640 CQ4 tokens over a 256-position
+// window, 27 layers: 5.3 ms as one pass, 206 ms with the 384 positions past
+// the ring as steps.
 nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits, bool select,
                      bool graphs) {
   nd_status st = ensure_prefill(ctx, n);
   if (st != ND_OK) return st;
   hipStream_t s = ctx->stream;
   uint32_t done = 0;
+  const uint32_t fit = n->kv.alloc > n->position ? n->kv.alloc - n->position : 0;
+  if (count > fit && count - fit > kStepRest) {
+    if ((st = ensure_prompt_cache(ctx, n)) != ND_OK) return st;
+    nd_kv lin = n->kv;
+    lin.k = n->pf_kv.k;
+    lin.v = n->pf_kv.v;
+    lin.ks = n->pf_kv.ks;
+    lin.vs = n->pf_kv.vs;
+    // More than sink + window slots, the mark of a linear cache: the prompt
+    // outgrows the ring, so max_length does too.
+    lin.alloc = n->d.max_length;
+    const uint32_t first = n->position;
+    if (first) ND_HIP(ctx, enqueue_ring_copy(n, lin, 0, first, false, s));
+    const uint32_t passes = (count + n->pf_cap - 1) / n->pf_cap;
+    for (uint32_t i = 0; i < passes; ++i) {  // even passes: no short last one
+      const uint32_t chunk = (count - done + (passes - i) - 1) / (passes - i);
+      const bool last = i + 1 == passes;
+      ND_HIP(ctx, enqueue_prefill(n, lin, chunk, last && want_logits, last && select, s));
+      n->position += chunk;
+      done += chunk;
+    }
+    ND_HIP(ctx, enqueue_ring_copy(n, lin, first, n->position, true, s));
+    return ND_OK;
+  }
   while (done < count) {
     const uint32_t left = count - done;
     const uint32_t room = n->kv.alloc > n->position ? n->kv.alloc - n->position : 0;
     const uint32_t chunk = std::min(std::min(left, n->pf_cap), room);
     const bool last_pass = chunk == left;
     if (chunk > 0) {
-      ND_HIP(ctx, enqueue_prefill(n, chunk, last_pass && want_logits, last_pass && select, s));
+      ND_HIP(ctx, enqueue_prefill(n, n->kv, chunk, last_pass && want_logits, last_pass && select, s));
       n->position += chunk;
       done += chunk;
       continue;
     }
-    // Slots wrap from here on: one step per token.
+    // The few positions past the ring: one step per token.
     const bool last = left == 1;
     if (graphs) {
       if ((st = launch_graph(ctx, n, last && (want_logits || select) ? kGraphPromptSelect
@@ -3706,6 +3813,7 @@ nd_status nd_needle_free(nd_ctx* ctx, nd_needle* n) {
   drop_graphs(n);
   if (n->arena) hipFree(n->arena);
   if (n->pf_arena) hipFree(n->pf_arena);
+  if (n->pf_kv_arena) hipFree(n->pf_kv_arena);
   for (auto* v : {&n->wqkvg, &n->ekv, &n->owned_parts})
     for (auto& m : *v) {
       if (m.w) hipFree(m.w);

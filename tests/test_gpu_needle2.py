@@ -549,3 +549,56 @@ def test_batched_prefill_then_steps(hip, window, sink, n_prompt, max_length, cq_
         close_confidence(rt.resolve_confidence(), ref.confidence(), "confidence after steps")
     finally:
         model.dispose()
+
+
+@pytest.mark.parametrize("window,sink,prompts,mode,cq_bits",
+                         [(8, 3, (15,), "int8", 0), (8, 3, (16,), "int8", 0),
+                          (8, 0, (3, 10, 20), "int8", 4), (64, 0, (200,), "int8", 0),
+                          (100, 70, (400,), "int8", 0), (96, 5, (150, 130), "int8", 4),
+                          (96, 5, (150, 130), "float32", 0), (256, 3, (1100,), "int8", 0)])
+def test_prompt_that_outgrows_the_ring(hip, window, sink, prompts, mode, cq_bits):
+    """Prompts whose positions outgrow the ring run as passes over the linear
+    prompt cache (a rest of up to 4 positions as steps: 15 against 16 over 11
+    slots): logits, the rows the ring keeps, the confidence and the following
+    steps against a step per token -- the oracle's for the int8 cache, the
+    device's own for the float32 one.  A window narrower and wider than a
+    64-key block, sinks past one block, prompts that begin on a wrapped ring,
+    and 1100 positions over two passes."""
+    say("needle2 prompt past the ring", window, sink, prompts, mode, cq_bits)
+    total = sum(prompts)
+    g = Needle2Geometry(**{**SMALL.__dict__, "kv_window": window, "max_length": total + 8})
+    w = Needle2Weights(g, 43, cq_bits=cq_bits)
+    model = NeedleModel(hip, w)
+    try:
+        rt, resident = model.create_resident_runtime(), model.resident
+        tokens = synth.Stream(13, f"n2ring{window}").integers(total + 4, 0, g.vocab - 1)
+        if mode == "float32":
+            resident.reset(g.max_length, sink, "float32")
+            want = [rt.step(int(t)) for t in tokens]
+            rows = [resident.kv_read(l, h) for l in range(g.layers) for h in range(g.kv_heads)]
+            resident.reset(g.max_length, sink, "float32")
+        else:
+            ref = oracle.Needle2(w).runtime(g.max_length, sink)
+            ref.capture_kv(0, g.max_length)
+            rt.reset(g.max_length, sink)
+        at = 0
+        for n in prompts:
+            got = rt.prefill(tokens[at:at + n])
+            if mode == "int8":
+                for t in tokens[at:at + n]:
+                    step = ref.step(int(t))
+            at += n
+            close(got, want[at - 1] if mode == "float32" else step, ("prompt", at))
+        if mode == "int8":
+            check_kv(model, ref, g, total, sink, "prompt past the ring")
+            close_confidence(rt.resolve_confidence(), ref.confidence(), "prompt past the ring")
+        for t in tokens[total:]:
+            close(rt.step(int(t)), want[at] if mode == "float32" else ref.step(int(t)), ("step", at))
+            at += 1
+        if mode == "float32":
+            after = [resident.kv_read(l, h) for l in range(g.layers) for h in range(g.kv_heads)]
+            for got, ref_rows in zip(after, rows):
+                for a, b in zip(got, ref_rows):
+                    close(a, b, "float32 rows")
+    finally:
+        model.dispose()
