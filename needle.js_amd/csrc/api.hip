@@ -357,6 +357,7 @@ nd_status nd_mat_upload_cq(nd_ctx* ctx, const uint8_t* packed, const uint16_t* n
   } else {
     for (uint32_t i = 0; i < (1u << bits); ++i) m->cb[i] = codebook[i];
   }
+  if (!nd_split_codebook(m->cb, bits, &m->planes, &m->cb_factor)) m->cb_factor = 0.0;
   const size_t pbytes = (size_t)n * m->row_bytes, nbytes = (size_t)n * (kstore / g) * 2;
   const void* psrc = packed;
   const void* nsrc = norms;
@@ -373,7 +374,7 @@ nd_status nd_mat_upload_cq(nd_ctx* ctx, const uint8_t* packed, const uint16_t* n
     psrc = ppad.data();
     nsrc = npad.data();
   }
-  hipError_t e = hipMalloc(&m->packed, pbytes);
+  hipError_t e = hipMalloc(&m->packed, pbytes + kCqSlack);
   if (e == hipSuccess) e = hipMalloc(&m->norms, nbytes);
   if (e == hipSuccess) e = hipMemcpyAsync(m->packed, psrc, pbytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->norms, nsrc, nbytes, hipMemcpyHostToDevice, ctx->stream);

@@ -408,12 +408,25 @@ hipError_t nd_launch_cq_matvec(const nd_mat* m, const float* x, uint32_t batch, 
           ? 1u
           : kRacc;
   const uint32_t blocks = (row_count + rpp * racc - 1) / (rpp * racc);
+  const bool vec = (m->k & 3) == 0 && (x_stride & 3) == 0 &&
+                   (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  if (nd_batch_matvec_fits(m, batch)) {
+    // The batched form when it should be a tenth faster: a round of 256
+    // workgroups here takes about 1.6 us at kRacc rows a thread and 0.6 at
+    // one, 3.3 times that with scalar loads of x (measured at 1536 x 512, 512
+    // x 512, 8192 x 512, 4096 x 1024, 16384 x 2048, 4096 x 4096 and 300 x 777,
+    // 2 to 300 batch rows: the faster form, or one within a tenth of it, at
+    // every point).
+    const uint64_t rounds = ((uint64_t)blocks * batch + 255) / 256;
+    const float here = (float)rounds * (racc == 1 ? 0.6f : 1.6f) * (vec ? 1.f : 3.3f);
+    if (nd_batch_matvec_us(m, row_count, batch) < 0.9f * here)
+      return nd_launch_batch_matvec(m, x, batch, x_stride, row_start, row_count, y, y_stride, s,
+                                    nullptr);
+  }
   uint32_t g_log2 = 0;
   while ((1u << g_log2) < m->g) ++g_log2;
   const uint32_t lanes_per_group = m->g > 32 ? m->g / 32 : 1;
   if (m->g <= kMaxRotateGroup) {
-    const bool vec = (m->k & 3) == 0 && (x_stride & 3) == 0 &&
-                     (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     const CqFn f = vec ? pick<true, true>(m, racc) : pick<true, false>(m, racc);
     hipLaunchKernelGGL(f, dim3(blocks, batch), dim3(kCqThreads), 0, s, m->packed,
                        m->norms, codebook_of(m), x, x_stride, y, y_stride, m->k, m->kpad, g_log2,

@@ -684,7 +684,8 @@ VecPlan plan_vector(const nd_mat* m, uint32_t left, uint32_t row_count) {
 // Host-side checks that the kernel's geometry fits the matrix were done by
 // the caller (k = 16 * 2^j with 128 <= k <= 8192, g % 16 == 0, k % g == 0).
 // With `split` (kMatvecSplitBytes of device memory), batches of 3 or more
-// rows of a matrix with g % 32 == 0 run on MFMA, 8 rows per launch: k <=
+// rows of a matrix with g % 32 == 0 run on MFMA: more than 8 rows, or a tall
+// matrix, in nd_launch_batch_matvec; up to 8 rows in the forms here, k <=
 // 2048 in one fused launch, k >= 4096 as k-slices summed by the last slice
 // of each row block (9.2 vs 10.7 us for the fused form at 4096 x 4096 and
 // 12.9 vs 17.4 at 4096 x 8192, batch 8; at 4096 x 2048 the fused form wins,
@@ -694,6 +695,16 @@ hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uin
                             uint32_t row_start, uint32_t row_count, float* y, uint32_t y_stride,
                             hipStream_t s, void* split) {
   if (row_count == 0 || batch == 0) return hipSuccess;
+  // More than eight rows (the forms below then launch once for every eight:
+  // 12 rows of 4096 x 4096, 15.8 us against 8.5), or more than 256 of the
+  // fused form's workgroups, one to a CU (8 rows of 6000 x 2048, 9.3 against
+  // 8.1 us; at 4096 rows or fewer the fused form is the faster one, 4.7
+  // against 5.3 us at 4096 x 1024): the batched form, all rows in one launch.
+  const bool rounds = m->k <= kFusedMaxK && row_count > 16 * 256;
+  if (split && (batch > kSplitRows || rounds) && nd_batch_matvec_fits(m, batch) &&
+      (x_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0)
+    return nd_launch_batch_matvec(m, x, batch, x_stride, row_start, row_count, y, y_stride, s,
+                                  split);
   if (split && batch >= kMfmaMinBatch && m->g % 32 == 0) {
     uint32_t gshift = 0;  // g = 32 << gshift (g divides k, a power of two)
     while ((32u << gshift) < m->g) ++gshift;
@@ -719,7 +730,7 @@ hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uin
       const size_t cap = kMatvecPartialBytes / sizeof(float) / ((size_t)slices * kSplitRows);
       // Row blocks per launch: within the partials and within the counters
       // (one 32-word line per row block in the split's last 64 KB).
-      constexpr size_t kCounterBlocks = (kMatvecSplitBytes - kMatvecPartialBytes) / (32 * 4);
+      constexpr size_t kCounterBlocks = kMatvecCounters;
       const uint32_t block = (uint32_t)(std::min(cap / 64, kCounterBlocks) * 64);
       float* P = reinterpret_cast<float*>(split);
       uint32_t* counters = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(split) +

@@ -11,6 +11,15 @@
 #include "needle_hip.h"
 #include "nd_rope.hpp"
 
+// A codebook as byte planes for v_perm_b32: plane 2 h + q holds byte q of the
+// fp16 hi (h = 0) or lo (h = 1) half of entries 4 i .. 4 i + 3 in word i.
+struct nd_code_planes {
+  uint32_t v[4][4];
+};
+
+// Bytes past the last packed row that a 16-byte read of it may touch.
+constexpr size_t kCqSlack = 16;
+
 struct nd_mat {
   int8_t* w = nullptr;      // [n][k] int8 codes, row-major
   float* scales = nullptr;  // [n][k / g]
@@ -22,6 +31,9 @@ struct nd_mat {
   uint8_t* packed = nullptr;
   uint16_t* norms = nullptr;
   float cb[16] = {};
+  // The codebook times cb_factor as fp16 halves (0: it has no such form).
+  nd_code_planes planes = {};
+  double cb_factor = 0.0;
 };
 // Prepared (rotated) input rows of a Cactus-Quant matvec: the context holds
 // kCqPreparedRows rows of up to kCqMaxKpad floats, reused in stream order.
@@ -128,8 +140,9 @@ void nd_xcd_override(bool off);
 // arrival counters, zero at allocation and left zero by every launch);
 // nullptr keeps the vector kernel.  Launches sharing one `split` must be ordered
 // (one stream).
-constexpr size_t kMatvecPartialBytes = (size_t(4) << 20) - (size_t(64) << 10);
-constexpr size_t kMatvecSplitBytes = kMatvecPartialBytes + (size_t(64) << 10);  // + counters
+constexpr uint32_t kMatvecCounters = 512;  // a 128-byte line each
+constexpr size_t kMatvecPartialBytes = size_t(16) << 20;
+constexpr size_t kMatvecSplitBytes = kMatvecPartialBytes + kMatvecCounters * 128;
 hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uint32_t x_stride,
                             uint32_t row_start, uint32_t row_count, float* y, uint32_t y_stride,
                             hipStream_t s, void* split = nullptr);
@@ -155,6 +168,19 @@ hipError_t nd_launch_cq_matvec(const nd_mat* m, const float* x, uint32_t batch, 
                                float* prepared, uint32_t row_start, uint32_t row_count, float* y,
                                uint32_t y_stride, hipStream_t s);
 hipError_t nd_launch_cq_row(const nd_mat* m, uint32_t row, float* out, hipStream_t s);
+
+// Batched rows on MFMA for group-scaled matrices (csrc/batch_matvec.hip):
+// batches of 3 or more, int8 with g % 32 == 0 (16-byte aligned rows of x) or
+// Cactus-Quant with g in 32..256 (nd_batch_matvec_fits).  `split` (as above)
+// lets an int8 product that leaves the GPU idle slice k; nullptr keeps it
+// whole.  nd_batch_matvec_us: about what a Cactus-Quant launch takes beyond a
+// launch's fixed cost, for the choice against one workgroup per batch row.
+bool nd_split_codebook(const float* cb, uint32_t bits, nd_code_planes* out, double* factor);
+bool nd_batch_matvec_fits(const nd_mat* m, uint32_t batch);
+float nd_batch_matvec_us(const nd_mat* m, uint32_t row_count, uint32_t batch);
+hipError_t nd_launch_batch_matvec(const nd_mat* m, const float* x, uint32_t batch,
+                                  uint32_t x_stride, uint32_t row_start, uint32_t row_count,
+                                  float* y, uint32_t y_stride, hipStream_t s, void* split);
 
 // Visible-position arithmetic of the attention window (runtime.ts:723-728).
 struct nd_visible {

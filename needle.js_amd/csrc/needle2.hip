@@ -3669,8 +3669,10 @@ nd_status nd_needle_create(nd_ctx* ctx, const nd_needle_desc* d, nd_needle** out
       m.kpad = p0->kpad;
       m.row_bytes = p0->row_bytes;
       for (int i = 0; i < 16; ++i) m.cb[i] = p0->cb[i];
+      m.planes = p0->planes;
+      m.cb_factor = p0->cb_factor;
       const size_t nb = (size_t)(m.kpad / m.g) * 2;  // norm bytes per row
-      if (e == hipSuccess) e = hipMalloc(&m.packed, (size_t)m.n * m.row_bytes);
+      if (e == hipSuccess) e = hipMalloc(&m.packed, (size_t)m.n * m.row_bytes + kCqSlack);
       if (e == hipSuccess) e = hipMalloc(&m.norms, (size_t)m.n * nb);
       size_t row = 0;
       for (size_t i = 0; i < count; ++i) {

@@ -206,3 +206,42 @@ def test_needle2_archive_matrices_on_device(hip):
             assert_close(hip.matvec(m, xx), ref_matvec(m, xx), RTOL, ATOL, f"archive b{bits}")
         for tok in (0, 255):
             assert np.array_equal(hip.row(w.embedding, tok), ref_row(w.embedding, tok))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+@pytest.mark.parametrize("n,k,g,batch", [(300, 777, 32, 64), (200, 513, 128, 81),
+                                         (400, 1030, 256, 97), (1536, 512, 32, 300),
+                                         (2001, 300, 64, 500)])
+def test_cq_many_rows(hip, bits, n, k, g, batch):
+    """Batches that take the MFMA form: 16, 32 and 64 rows a tile, rows of x
+    of any alignment, a last chunk of one unit, groups narrower than a chunk
+    and as wide; a row of zeros, one of subnormals and one of large values.
+    Bound per output: x and the codebook keep 2^-24 and 2^-23 in their fp16
+    halves, the rotation's log2(g) additions and at most 57 more follow, each
+    2^-24 of the absolute sum over the rotation's absolute values: 2^-18."""
+    say("cq many rows", n, k, g, bits, batch)
+    m = cq(9, n, k, g, bits)
+    x = np.random.default_rng(n + k + batch).standard_normal((batch, k)).astype(np.float32)
+    x[0] = 0.0
+    x[1] *= np.float32(1e-41)
+    x[2] *= np.float32(1e30)
+    kpad = -(-k // g) * g
+    levels = (np.array([0.0, 1.2240064, 0.0, -1.2240064]) / np.sqrt(g) if bits == TERNARY
+              else BOOKS[bits].astype(np.float64))
+    h = np.ones((1, 1))
+    while h.shape[0] < g:
+        h = np.block([[h, h], [h, -h]])
+    xp = np.zeros((batch, kpad))
+    xp[:, :k] = x
+    rot = (xp.reshape(batch, -1, g) @ h).reshape(batch, kpad) / np.sqrt(g)
+    spread = (np.abs(xp).reshape(batch, -1, g) @ np.abs(h)).reshape(batch, kpad) / np.sqrt(g)
+    pb = 2 if bits == TERNARY else bits
+    raw = np.unpackbits(m.packed.reshape(n, -1), axis=1, bitorder="little")[:, :kpad * pb]
+    codes = (raw.reshape(n, kpad, pb) * (1 << np.arange(pb))).sum(-1)
+    norms = np.asarray(m.norms).view(np.float16).astype(np.float64).reshape(n, -1)[:, :kpad // g]
+    w = levels[codes] * np.repeat(norms, g, axis=1)
+    for lo, count in ((0, n), (1, n - 2)):
+        got = hip.matvec(m, x, MatrixRowRange(lo, count)).astype(np.float64)
+        want = rot @ w[lo:lo + count].T
+        bound = 2.0 ** -18 * (spread @ np.abs(w[lo:lo + count]).T) + 1e-43
+        assert np.all(np.abs(got - want) <= bound), (lo, np.max(np.abs(got - want) / bound))

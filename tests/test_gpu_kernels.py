@@ -392,3 +392,28 @@ def test_select_random_bit_exact_ids(hip, vocab):
         hip.select(np.zeros(10, np.float32), np.array([10], np.uint32))
     with pytest.raises(NeedleError):
         hip.select(np.zeros(10, np.float32), np.array([], np.uint32))
+
+
+@pytest.mark.parametrize("n,k,g,batch", [(65, 128, 32, 9), (64, 256, 256, 16), (130, 512, 64, 17),
+                                         (300, 2048, 2048, 33), (200, 4096, 32, 70),
+                                         (96, 8192, 128, 65), (4100, 512, 32, 3)])
+def test_matvec_many_rows(hip, n, k, g, batch):
+    """Batches above eight (and three rows of a tall matrix) in one launch: a
+    half chunk, one chunk, k slices, one row past a tile in each direction,
+    batch rows of zeros, of subnormals and near the largest float, and a row
+    range.  Bound per output: the hi/lo split keeps x to 2^-24 and at most 57
+    fp32 additions follow (32 products, 8 units, up to 16 chunks of a group,
+    a slice), each 2^-24 of the absolute sum: 2^-18 of it."""
+    say("matvec many rows", n, k, g, batch)
+    w, s = synth.int8_matrix(61, f"many{n}x{k}", n, k, g)
+    x = synth.Stream(61, f"xm{k}b{batch}").normal((batch, k))
+    x[0] = 0.0
+    x[1] *= np.float32(1e-41)
+    x[2] *= np.float32(1e33)
+    m = Int8Matrix(w, s, g)
+    full = w.astype(np.float64) * np.repeat(s.astype(np.float64), g, axis=1)
+    for lo, count in ((0, n), (1, n - 2)):
+        got = hip.matvec(m, x, MatrixRowRange(lo, count)).astype(np.float64)
+        want = x.astype(np.float64) @ full[lo:lo + count].T
+        bound = 2.0 ** -18 * (np.abs(x).astype(np.float64) @ np.abs(full[lo:lo + count]).T) + 1e-43
+        assert np.all(np.abs(got - want) <= bound), (lo, np.max(np.abs(got - want) / bound))
