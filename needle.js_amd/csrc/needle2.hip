@@ -1595,8 +1595,14 @@ __device__ __forceinline__ void attention_role(const MixArgs& a, uint32_t ah,
   w.release();
 }
 
-template <bool CQ, bool WO = false, bool PU = true, bool STAMP = false>
-__global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
+// ROWS (a prefill pass: one workgroup per position): the phi weights are
+// loaded where they are used instead of with the first operands.  One row
+// alone waits for its loads, so it issues all of them at entry and holds them
+// in registers; with hundreds of rows the CU's other workgroups fill the wait
+// and registers decide how many there are (149 a thread: one workgroup a CU
+// and 38 us a layer for 640 CQ4 rows; at most 128: two, 31 us).
+template <bool CQ, bool WO = false, bool PU = true, bool STAMP = false, bool ROWS = false>
+__global__ __launch_bounds__(kMixWg, ROWS ? 4 : 1) void n2_mix_kernel(MixArgs a) {
   static_assert(kQkvWg == kMixWg, "the fused projection runs on mix-sized workgroups");
   uint64_t stamp[16] = {};
   if constexpr (STAMP) stamp[0] = wall_clock64();
@@ -1717,13 +1723,16 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
   // rows past the phi rows are zeroed there.
   __builtin_amdgcn_sched_barrier(0);
   u32x4 pw[kPhiPairs];
-  if constexpr (!CQ) {
+  auto load_phi = [&]() __attribute__((always_inline)) {
+    if constexpr (!CQ) {
 #pragma unroll
-    for (int i = 0; i < kPhiPairs; ++i) {
-      const uint32_t pp = min(kq * ppw + i, pairs - 1);
-      pw[i] = *reinterpret_cast<const u32x4*>(wrow + (size_t)pp * 64);
+      for (int i = 0; i < kPhiPairs; ++i) {
+        const uint32_t pp = min(kq * ppw + i, pairs - 1);
+        pw[i] = *reinterpret_cast<const u32x4*>(wrow + (size_t)pp * 64);
+      }
     }
-  }
+  };
+  if constexpr (!ROWS) load_phi();
   __builtin_amdgcn_sched_barrier(0);
   const uint32_t tr = min(t, nrows - 1);
   const float norm_in = a.norm_input[tc], ekey = a.ekey[tc], evalue = a.evalue[tc],
@@ -1741,7 +1750,7 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
   // (bits of them) and the norms of its groups -- loaded here with the
   // other operands, each row in its own matrix's format.
   uint32_t cw[3][4] = {}, cn[3][4] = {};
-  if constexpr (CQ) {
+  auto load_cq_phi = [&]() __attribute__((always_inline)) {
     if (t == 0) {  // constant indices into the argument block
 #pragma unroll
       for (int m = 0; m < (PU ? 1 : 3); ++m)
@@ -1772,7 +1781,8 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
         if ((uint32_t)k < gpu) cn[j][k] = nrow[k];
       }
     }
-  }
+  };
+  if constexpr (CQ && !ROWS) load_cq_phi();
 
   if constexpr (WO) {
     // Every operand above is in flight; wait for the Wo workgroups' count
@@ -1908,6 +1918,7 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
     // as cq_rotate_unit, done once instead of once per wave.
     const uint32_t g0 = a.cq_g[0];
     const bool lanes_rot = PU && (D & 63u) == 0;
+    if constexpr (ROWS) load_cq_phi();
     if (col) {
 #pragma unroll
       for (int l = 0; l < 4; ++l)
@@ -1985,6 +1996,7 @@ __global__ __launch_bounds__(kMixWg) void n2_mix_kernel(MixArgs a) {
     }
     pre_phi = phi[min(lane, L - 1)];
   } else {
+    if constexpr (ROWS) load_phi();
     if (col) {
   #pragma unroll
       for (int l = 0; l < 4; ++l)
@@ -3362,9 +3374,9 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
       m.r_b_post = n->params + n->o_bpost + (size_t)l * ln;
       m.r_b_res = n->params + n->o_bres + (size_t)l * ln * ln;
     }
-    auto mix = !n->cq ? &n2_mix_kernel<false>
-               : n->phi_uniform ? &n2_mix_kernel<true, false, true>
-                                : &n2_mix_kernel<true, false, false>;
+    auto mix = !n->cq ? &n2_mix_kernel<false, false, true, false, true>
+               : n->phi_uniform ? &n2_mix_kernel<true, false, true, false, true>
+                                : &n2_mix_kernel<true, false, false, false, true>;
     hipLaunchKernelGGL(mix, dim3(rows), dim3(kMixWg), 0, s, m);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!pre) break;
