@@ -2134,10 +2134,17 @@ __global__ __launch_bounds__(kMixWg, ROWS ? 4 : 1) void n2_mix_kernel(MixArgs a)
 // position counters past the batch.
 __global__ __launch_bounds__(kWg) void n2_begin_batch_kernel(BeginArgs a, uint32_t p0,
                                                              uint32_t count,
-                                                             uint32_t* __restrict__ positions) {
+                                                             uint32_t* __restrict__ positions,
+                                                             const double* __restrict__ inv_freq,
+                                                             double2* __restrict__ rope) {
   __shared__ uint32_t s_idx[16], s_valid[16];
   const uint32_t m = blockIdx.x, t = threadIdx.x, pos = p0 + m;
   const uint32_t tok = a.history[pos];
+  if (t >= kWg - 32) {  // the row's RoPE angles, shared by every layer and head
+    double sn, cs;
+    sincos((double)pos * inv_freq[t & 31], &sn, &cs);
+    rope[(size_t)m * 32 + (t & 31)] = make_double2(sn, cs);
+  }
   if (t == 0) {
     positions[m] = pos;
     if (m == 0) {
@@ -2226,21 +2233,25 @@ __global__ void n2_ring_store_kernel(const float* __restrict__ ekv, float* __res
 }
 
 // Query/key norm + RoPE and the K/V append of every batch position: one wave
-// per (head, position); qkvg rows [q | k | v | gate] with stride ld.
-__global__ __launch_bounds__(64) void n2_rope_store_batch_kernel(
+// per (head, position), four heads of a position to a workgroup (a workgroup
+// per head took the dispatcher longer than the work, and every head its own
+// float64 sincos: 6.7 us at 640 positions of 16 heads); qkvg rows [q | k | v |
+// gate] with stride ld.
+__global__ __launch_bounds__(256) void n2_rope_store_batch_kernel(
     const float* __restrict__ qkvg, uint32_t ld, uint32_t heads, uint32_t kv_heads,
     const float* __restrict__ q_norm, const float* __restrict__ k_norm,
-    const double* __restrict__ inv_freq, uint32_t p0, float* __restrict__ q_out,
+    const double2* __restrict__ rope, uint32_t p0, float* __restrict__ q_out,
     void* __restrict__ Kc, void* __restrict__ Vc, float* __restrict__ Ks,
     float* __restrict__ Vs, uint32_t layer, uint32_t alloc, uint32_t sink, uint32_t window,
     uint32_t f32) {
-  const uint32_t b = blockIdx.x, m = blockIdx.y, lane = threadIdx.x, pos = p0 + m;
+  const uint32_t b = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t m = blockIdx.y, lane = threadIdx.x & 63, pos = p0 + m;
+  if (b >= heads + 2 * kv_heads) return;
   const int role = b < heads ? 0 : (b < heads + kv_heads ? 1 : 2);
   const uint32_t h = role == 0 ? b : (role == 1 ? b - heads : b - heads - kv_heads);
   const float val = qkvg[(size_t)m * ld + (size_t)b * kHd + lane];
-  double sn, cs;
-  sincos((double)pos * inv_freq[lane & 31], &sn, &cs);
-  head_epilogue(val, lane, role, sn, cs, role == 0 ? q_norm[lane] : k_norm[lane],
+  const double2 sc = rope[(size_t)m * 32 + (lane & 31)];
+  head_epilogue(val, lane, role, sc.x, sc.y, role == 0 ? q_norm[lane] : k_norm[lane],
                 q_out + ((size_t)m * heads + h) * kHd, Kc, Vc, Ks, Vs,
                 ((size_t)layer * kv_heads + h) * alloc, kv_slot(pos, sink, window), alloc, f32);
 }
@@ -2330,72 +2341,135 @@ __global__ __launch_bounds__(256) void n2_probe_scores_kernel(const float* __res
   }
 }
 
-constexpr uint32_t kPoolThreads = 1024;  // 16 waves, each on every 16th cell
+// The pool update for a prefill pass's cells (runtime.ts:74-105) in its closed
+// form: with M' = max(M, scores), the sums so far are rescaled by exp(M - M')
+// (0 before the first cell) and cell c enters with weight exp(s_c - M').  Two
+// launches.  The first reads every cell once: workgroup (slice, j) takes the
+// slice's cells and columns [128 j, +128), with weights relative to the
+// slice's own maximum m, for all probes at once (thread: one column of every
+// fourth cell), and leaves the weighted sums, m and the sum of weights.  The
+// second rescales the slices by exp(m - M') and adds them in slice order.  A
+// workgroup per probe and 64 columns reads the cells once for each probe and
+// ran on 64 CUs: 235 us for 640 positions of 28 cells.
+constexpr uint32_t kPoolSlices = 64, kPoolCols = 128, kPoolThreads = 512;
+constexpr uint32_t kPoolSubs = kPoolThreads / kPoolCols;
+struct PoolSlice {
+  double max[kMaxProbes], den[kMaxProbes];
+};
+__global__ __launch_bounds__(kPoolThreads) void n2_probe_pool_kernel(
+    const float* __restrict__ cells, uint32_t C, uint32_t D, uint32_t P,
+    const double* __restrict__ scores, uint32_t per, double* __restrict__ part,
+    PoolSlice* __restrict__ slices) {
+  constexpr uint32_t kChunk = 64;
+  __shared__ double e[kChunk][kMaxProbes];
+  __shared__ double red[kPoolSubs - 1][kMaxProbes][kPoolCols];
+  __shared__ double s_max[kMaxProbes];
+  const uint32_t t = threadIdx.x, slice = blockIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t col = blockIdx.y * kPoolCols + t % kPoolCols, sub = t / kPoolCols;
+  const uint32_t cc = col < D ? col : D - 1;
+  const uint32_t c_begin = slice * per, c_end = C - c_begin < per ? C : c_begin + per;
+  if (wave < kMaxProbes) {  // wave p: the slice's maximum of probe p
+    double mx = -INFINITY;
+    if (wave < P)
+      for (uint32_t c = c_begin + lane; c < c_end; c += 64)
+        mx = fmax(mx, scores[(size_t)c * kMaxProbes + wave]);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) s_max[wave] = mx;
+  }
+  __syncthreads();
+  double acc[kMaxProbes] = {}, den = 0.0;
+  const uint32_t ep = t % kMaxProbes, ec = t / kMaxProbes;  // this thread's weight of a chunk
+  static_assert(kPoolThreads == kChunk * kMaxProbes, "one weight a thread");
+  for (uint32_t c0 = c_begin; c0 < c_end; c0 += kChunk) {
+    const uint32_t n = c_end - c0 < kChunk ? c_end - c0 : kChunk;
+    // The chunk's cells of this thread, in flight while the weights are taken.
+    float v[kChunk / kPoolSubs];
+#pragma unroll
+    for (uint32_t i = 0; i < kChunk / kPoolSubs; ++i) {
+      const uint32_t c = sub + kPoolSubs * i;
+      v[i] = cells[(size_t)(c0 + (c < n ? c : 0)) * D + cc];
+    }
+    double w = 0.0;
+    if (ec < n && ep < P) w = exp(scores[(size_t)(c0 + ec) * kMaxProbes + ep] - s_max[ep]);
+    e[ec][ep] = w;
+    den += w;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kChunk / kPoolSubs; ++i) {
+      const double x = sub + kPoolSubs * i < n ? (double)v[i] : 0.0;
+#pragma unroll
+      for (uint32_t p = 0; p < kMaxProbes; ++p)
+        acc[p] += e[sub + kPoolSubs * i][p] * x;
+    }
+    __syncthreads();
+  }
+  if (sub > 0)
+#pragma unroll
+    for (uint32_t p = 0; p < kMaxProbes; ++p) red[sub - 1][p][t % kPoolCols] = acc[p];
+  __syncthreads();
+  if (sub == 0 && col < D)
+#pragma unroll
+    for (uint32_t p = 0; p < kMaxProbes; ++p) {
+      double sum = acc[p];
+#pragma unroll
+      for (uint32_t q = 0; q + 1 < kPoolSubs; ++q) sum += red[q][p][t];
+      part[((size_t)slice * kMaxProbes + p) * D + col] = sum;
+    }
+  __syncthreads();
+  double* dr = &red[0][0][0];
+  dr[t] = den;
+  __syncthreads();
+  if (t < kMaxProbes && blockIdx.y == 0) {
+    double sum = 0.0;
+    for (uint32_t q = 0; q < kChunk; ++q) sum += dr[q * kMaxProbes + t];
+    slices[slice].max[t] = s_max[t];
+    slices[slice].den[t] = sum;
+  }
+}
 
-// The online update of runtime.ts:73-90 over C cells at once, in its closed
-// form: M' = max(M, max_c s_c); every earlier term is rescaled by
-// exp(M - M') (0 before the first cell) and cell c enters with weight
-// exp(s_c - M').  Workgroup (p, j) updates probe p's weighted sums of
-// columns [64 j, 64 j + 64) and its copy of (M, denominator).
-__global__ __launch_bounds__(kPoolThreads) void n2_probe_pool_kernel(const float* __restrict__ cells,
-                                                            uint32_t C, uint32_t D,
-                                                            const double* __restrict__ scores,
-                                                            PoolState ps) {
-  constexpr uint32_t kChunk = 1024;
-  __shared__ double e[kChunk];
-  __shared__ double red[kPoolThreads];
-  constexpr uint32_t kSlices = kPoolThreads / 64;
-  const uint32_t p = blockIdx.x, j = blockIdx.y, t = threadIdx.x;
-  const uint32_t col = j * 64 + (t & 63), slice = t >> 6;
+// Workgroup (p, j): probe p's columns [64 j, +64) over all slices, four
+// quarters of them at a time.
+__global__ __launch_bounds__(256) void n2_probe_merge_kernel(const double* __restrict__ part,
+                                                             const PoolSlice* __restrict__ slices,
+                                                             uint32_t n, uint32_t D, PoolState ps) {
+  __shared__ double f[kPoolSlices], red[4][64];
+  const uint32_t p = blockIdx.x, j = blockIdx.y, t = threadIdx.x, lane = t & 63, q = t >> 6;
+  const uint32_t col = j * 64 + lane;
   double* const my_max = ps.max + p * kMaxChunks + j;
   double* const my_den = ps.den + p * kMaxChunks + j;
   const double den_old = *my_den;
   const double m_old = den_old > 0.0 ? *my_max : -INFINITY;
-  double mx = -INFINITY;
-  for (uint32_t c = t; c < C; c += kPoolThreads) mx = fmax(mx, scores[(size_t)c * kMaxProbes + p]);
-  red[t] = mx;
-  __syncthreads();
-  for (uint32_t w = kPoolThreads / 2; w > 0; w >>= 1) {
-    if (t < w) red[t] = fmax(red[t], red[t + w]);
-    __syncthreads();
-  }
-  const double m_new = fmax(m_old, red[0]);
-  const double factor = m_old > -INFINITY ? exp(m_old - m_new) : 0.0;
-  __syncthreads();
-  double acc = 0.0, esum = 0.0;
-  for (uint32_t c0 = 0; c0 < C; c0 += kChunk) {
-    const uint32_t n = C - c0 < kChunk ? C - c0 : kChunk;
-    for (uint32_t c = t; c < n; c += kPoolThreads) {
-      const double w = exp(scores[(size_t)(c0 + c) * kMaxProbes + p] - m_new);
-      e[c] = w;
-      esum += w;
-    }
-    __syncthreads();
-    if (col < D) {
-#pragma unroll 16
-      for (uint32_t c = slice; c < n; c += kSlices)
-        acc += e[c] * (double)cells[(size_t)(c0 + c) * D + col];
-    }
-    __syncthreads();
-  }
-  red[t] = acc;
-  __syncthreads();
-  if (t < 64 && col < D) {
-    double sum = red[t];
+  const double ms = lane < n ? slices[lane].max[p] : -INFINITY;
+  double m_new = fmax(m_old, ms);
 #pragma unroll
-    for (uint32_t q = 1; q < kSlices; ++q) sum += red[t + 64 * q];
-    double* w = ps.weighted + (size_t)p * D + col;
-    *w = *w * factor + sum;
+  for (int o = 32; o >= 1; o >>= 1) m_new = fmax(m_new, __shfl_xor(m_new, o, 64));
+  const double factor = m_old > -INFINITY ? exp(m_old - m_new) : 0.0;
+  const double fs = lane < n ? exp(ms - m_new) : 0.0;
+  if (q == 0) f[lane] = fs;
+  double den = lane < n ? slices[lane].den[p] * fs : 0.0;
+  den = nd::wave_sum(den);
+  __syncthreads();
+  double v[kPoolSlices / 4];
+#pragma unroll
+  for (uint32_t i = 0; i < kPoolSlices / 4; ++i) {
+    const uint32_t s = q * (kPoolSlices / 4) + i;
+    v[i] = part[((size_t)(s < n ? s : 0) * kMaxProbes + p) * D + (col < D ? col : D - 1)];
   }
+  double sum = 0.0;
+#pragma unroll
+  for (uint32_t i = 0; i < kPoolSlices / 4; ++i) {
+    const uint32_t s = q * (kPoolSlices / 4) + i;
+    sum += s < n ? v[i] * f[s] : 0.0;
+  }
+  red[q][lane] = sum;
   __syncthreads();
-  red[t] = esum;
-  __syncthreads();
-  for (uint32_t w = kPoolThreads / 2; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
+  if (q == 0 && col < D) {
+    double* w = ps.weighted + (size_t)p * D + col;
+    *w = *w * factor + (((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
   }
   if (t == 0) {
-    *my_den = den_old * factor + red[0];
+    *my_den = den_old * factor + den;
     *my_max = m_new;
   }
 }
@@ -2575,6 +2649,7 @@ struct nd_needle {
         *pf_ekv = nullptr, *pf_evals = nullptr, *pf_fm = nullptr, *pf_partials = nullptr;
   int8_t* pf_digits = nullptr;
   uint32_t *pf_positions = nullptr, *pf_counters = nullptr;
+  double2* pf_rope = nullptr;        // (sin, cos) of each position's RoPE angles [cap][32]
   uint32_t* pf_cq_lookup = nullptr;  // CQ model: each position's engram lookups and token
   // The linear prompt cache (first prompt that outgrows its ring): max_length
   // slots per layer and KV head, pf_kv.mode the widest row it holds so far.
@@ -2596,6 +2671,8 @@ struct nd_needle {
   PoolState pool{};
   float *cells = nullptr, *pf_cells = nullptr;
   double *scores = nullptr, *pf_scores = nullptr, *conf_out = nullptr;
+  double* pf_pool = nullptr;  // the pass's slices: weighted sums [slice][8][d]
+  PoolSlice* pf_pool_slices = nullptr;
   // Which calls drive the runtime since the last reset: 0 none yet, 1 whole
   // steps (nd_needle_step, _prefill, _step_select, _generate), 2 the session
   // methods (ResidentExecutionSession, backends/backend.ts:65-80).
@@ -2644,8 +2721,14 @@ hipError_t enqueue_pool(nd_needle* n, const float* cells, uint32_t C, double* sc
                      probes, n->probe_count, scale, scores);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(n2_probe_pool_kernel, grid, dim3(kPoolThreads), 0, s, cells, C, D, scores,
-                     n->pool);
+  const uint32_t per = std::max((C + kPoolSlices - 1) / kPoolSlices, 32u);
+  const uint32_t slices = (C + per - 1) / per;
+  hipLaunchKernelGGL(n2_probe_pool_kernel, dim3(slices, (D + kPoolCols - 1) / kPoolCols),
+                     dim3(kPoolThreads), 0, s, cells, C, D, n->probe_count, scores, per,
+                     n->pf_pool, n->pf_pool_slices);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(n2_probe_merge_kernel, grid, dim3(256), 0, s, n->pf_pool, n->pf_pool_slices,
+                     slices, D, n->pool);
   return hipGetLastError();
 }
 
@@ -3194,6 +3277,9 @@ nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
                           al((size_t)cap * d.kv_heads * kAttnCounterStride * 4),
                           n->conf ? al((size_t)cap * (d.layers + 1) * D * 4) : 0,
                           n->conf ? al((size_t)cap * (d.layers + 1) * kMaxProbes * 8) : 0,
+                          n->conf ? al((size_t)kPoolSlices * kMaxProbes * D * 8) : 0,
+                          n->conf ? al(kPoolSlices * sizeof(PoolSlice)) : 0,
+                          al((size_t)cap * 32 * 16),
                           n->cq ? al((size_t)cap * (2 * d.engram_tables + 1) * 4) : 0};
   size_t total = 0;
   for (size_t v : sizes) total += v;
@@ -3232,6 +3318,9 @@ nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
   take(&n->pf_counters);
   take(&n->pf_cells);
   take(&n->pf_scores);
+  take(&n->pf_pool);
+  take(&n->pf_pool_slices);
+  take(&n->pf_rope);
   take(&n->pf_cq_lookup);
   n->pf_cap = cap;
   return ND_OK;
@@ -3274,7 +3363,8 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
   b.cell0 = pool_on(n) ? n->pf_cells : nullptr;
   b.cell_ld = cell_ld;
   b.cq_lookup = n->cq ? n->pf_cq_lookup : nullptr;
-  hipLaunchKernelGGL(n2_begin_batch_kernel, dim3(M), dim3(kWg), 0, s, b, p0, M, n->pf_positions);
+  hipLaunchKernelGGL(n2_begin_batch_kernel, dim3(M), dim3(kWg), 0, s, b, p0, M, n->pf_positions,
+                     n->inv_freq, n->pf_rope);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const uint32_t lk = 2 * d.engram_tables + 1;
@@ -3383,10 +3473,10 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
     if ((e = parts_product(n->wqkvg[l], n->cq ? n->qkv_part[l].data() : nullptr, 4, n->pf_ain, D,
                            D, n->pf_qkvg, qkv_ld)) != hipSuccess)
       return e;
-    hipLaunchKernelGGL(n2_rope_store_batch_kernel, dim3(d.heads + 2 * d.kv_heads, M), dim3(64), 0,
-                       s, n->pf_qkvg, qkv_ld, d.heads, d.kv_heads,
+    hipLaunchKernelGGL(n2_rope_store_batch_kernel, dim3((d.heads + 2 * d.kv_heads + 3) / 4, M),
+                       dim3(256), 0, s, n->pf_qkvg, qkv_ld, d.heads, d.kv_heads,
                        n->params + n->o_qn + (size_t)l * kHd, n->params + n->o_kn + (size_t)l * kHd,
-                       n->inv_freq, p0, n->pf_q, kv.k, kv.v, kv.ks, kv.vs, l, kv.alloc, kv.sink,
+                       n->pf_rope, p0, n->pf_q, kv.k, kv.v, kv.ks, kv.vs, l, kv.alloc, kv.sink,
                        nd_kv_linear(&kv) ? 0u : kv.window, kv.mode == ND_KV_FLOAT32 ? 1u : 0u);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     e = nd_launch_attention_batch(&kv, l, n->pf_positions, M, d.kv_heads, 0u,
