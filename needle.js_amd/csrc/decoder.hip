@@ -56,12 +56,11 @@ __device__ __forceinline__ void qk_rope_store_item(
     uint32_t m, uint32_t slot, uint32_t lane,
     const float* __restrict__ qkv, uint32_t ld, uint32_t heads, uint32_t kv_heads,
     const float* __restrict__ q_norm, const float* __restrict__ k_norm,
-    const double* __restrict__ inv_freq, const double2* __restrict__ rope_tab,
-    const uint32_t* __restrict__ positions,
-    uint32_t position0, float* __restrict__ q_out, int8_t* __restrict__ Kc,
-    int8_t* __restrict__ Vc, float* __restrict__ Ks, float* __restrict__ Vs, uint32_t layer,
-    uint32_t cache_heads, uint32_t alloc, uint32_t kv_head_stride) {
-  const uint32_t pos = positions ? positions[m] : position0 + m;
+    const double* __restrict__ inv_freq, const uint32_t* __restrict__ positions,
+    float* __restrict__ q_out, int8_t* __restrict__ Kc, int8_t* __restrict__ Vc,
+    float* __restrict__ Ks, float* __restrict__ Vs, uint32_t layer, uint32_t cache_heads,
+    uint32_t alloc, uint32_t kv_head_stride) {
+  const uint32_t pos = positions[m];
   const bool is_q = slot < heads;
   const uint32_t h = is_q ? slot : slot - heads;
   const float* src = qkv + (size_t)m * ld + (is_q ? h * kHd : heads * kHd + h * kHd);
@@ -70,13 +69,7 @@ __device__ __forceinline__ void qk_rope_store_item(
   // Half-split RoPE: pair (j, j + 32), angle = pos * theta^(-2j/64).
   const uint32_t j = lane & 31;
   double sn, cs;
-  if (rope_tab) {  // rope_table_kernel's values for row m: the same sincos
-    const double2 sc = rope_tab[(size_t)m * 32 + j];
-    sn = sc.x;
-    cs = sc.y;
-  } else {
-    sincos((double)pos * inv_freq[j], &sn, &cs);
-  }
+  sincos((double)pos * inv_freq[j], &sn, &cs);
   const float rot = nd::norm_rope(x, scale, lane, sn, cs);
   if (is_q) {
     q_out[((size_t)m * heads + h) * kHd + lane] = rot;
@@ -95,14 +88,53 @@ __device__ __forceinline__ void qk_rope_store_item(
 __global__ __launch_bounds__(64) void qk_rope_store_kernel(
     const float* __restrict__ qkv, uint32_t ld, uint32_t heads, uint32_t kv_heads,
     const float* __restrict__ q_norm, const float* __restrict__ k_norm,
-    const double* __restrict__ inv_freq, const double2* __restrict__ rope_tab,
-    const uint32_t* __restrict__ positions,
-    uint32_t position0, float* __restrict__ q_out, int8_t* __restrict__ Kc,
-    int8_t* __restrict__ Vc, float* __restrict__ Ks, float* __restrict__ Vs, uint32_t layer,
-    uint32_t cache_heads, uint32_t alloc, uint32_t kv_head_stride) {
+    const double* __restrict__ inv_freq, const uint32_t* __restrict__ positions,
+    float* __restrict__ q_out, int8_t* __restrict__ Kc, int8_t* __restrict__ Vc,
+    float* __restrict__ Ks, float* __restrict__ Vs, uint32_t layer, uint32_t cache_heads,
+    uint32_t alloc, uint32_t kv_head_stride) {
   qk_rope_store_item(blockIdx.y, blockIdx.x, threadIdx.x, qkv, ld, heads, kv_heads, q_norm,
-                     k_norm, inv_freq, rope_tab, positions, position0, q_out, Kc, Vc, Ks, Vs,
-                     layer, cache_heads, alloc, kv_head_stride);
+                     k_norm, inv_freq, positions, q_out, Kc, Vc, Ks, Vs, layer, cache_heads,
+                     alloc, kv_head_stride);
+}
+
+// The prompt's form: workgroup (column head, 16 rows), four rows a wave
+// (nd_rope.hpp).  Row m sits at position position0 + m with the angles
+// rope_tab[m].  Bound by the float64 of the norms and the store: a wave per
+// row and head took 15.9 us at 2048 rows of 16 + 8 heads.
+__global__ __launch_bounds__(256) void rope_store_rows_kernel(const float* __restrict__ qkv,
+                                                              uint32_t ld, uint32_t position0,
+                                                              uint32_t M, nd::RopeStore p) {
+  const uint32_t slot = blockIdx.x, lane = threadIdx.x & 63, l16 = lane & 15;
+  const uint32_t m = blockIdx.y * 16 + 4 * (threadIdx.x >> 6) + (lane >> 4);
+  const bool live = m < M;
+  const uint32_t mc = live ? m : M - 1;
+  const float* src = qkv + (size_t)mc * ld + slot * kHd + 2 * l16;
+  const float2 a = *reinterpret_cast<const float2*>(src);
+  const float2 b = *reinterpret_cast<const float2*>(src + 32);
+  nd::Head16 v{{a.x, a.y, b.x, b.y}};
+  const bool is_q = slot < p.heads;
+  if (slot < p.heads + p.kv_heads) {
+    const float* w = (is_q ? p.q_norm : p.k_norm) + 2 * l16;
+    const float2 wa = *reinterpret_cast<const float2*>(w);
+    const float2 wb = *reinterpret_cast<const float2*>(w + 32);
+    const double2* tab = p.rope_tab + (size_t)mc * 32 + 2 * l16;
+    const float scale[4] = {wa.x, wa.y, wb.x, wb.y};
+    const double2 sc[2] = {tab[0], tab[1]};
+    nd::norm_rope16(v, scale, sc);
+  }
+  if (is_q) {
+    if (!live) return;
+    float* q = p.q_out + ((size_t)m * p.heads + slot) * kHd + 2 * l16;
+    *reinterpret_cast<float2*>(q) = make_float2(v.x[0], v.x[1]);
+    *reinterpret_cast<float2*>(q + 32) = make_float2(v.x[2], v.x[3]);
+    return;
+  }
+  const bool is_k = slot < p.heads + p.kv_heads;
+  const uint32_t h = slot - p.heads - (is_k ? 0 : p.kv_heads), pos = position0 + mc;
+  if (!live || pos >= p.alloc) return;  // positions are validated on entry
+  const size_t row =
+      ((size_t)p.layer * p.cache_heads + (size_t)m * p.kv_head_stride + h) * p.alloc + pos;
+  nd::quant_store16(v, row, l16, is_k ? p.Kc : p.Vc, is_k ? p.Ks : p.Vs);
 }
 
 // (sin, cos) of the RoPE angles pos * inv_freq[j], j < 32, of rows [0, M)
@@ -574,7 +606,7 @@ nd_status nd_batch_step(nd_ctx* ctx, nd_batch* b, uint32_t max_position, uint32_
       ND_HIP(ctx, product(&dec->wqkv[l], b->x, attn_norm, b->qkv, qkv_rows, 0));
       hipLaunchKernelGGL(qk_rope_store_kernel, dim3(dec->heads + dec->kv_heads, B), dim3(64), 0,
                          s, b->qkv, qkv_rows, dec->heads, dec->kv_heads, q_norm, k_norm,
-                         dec->inv_freq, nullptr, b->positions, 0u, b->q, (int8_t*)b->kv.k,
+                         dec->inv_freq, b->positions, b->q, (int8_t*)b->kv.k,
                          (int8_t*)b->kv.v, b->kv.ks, b->kv.vs, l, b->kv.kv_heads, b->kv.alloc,
                          dec->kv_heads);
       ND_HIP(ctx, hipGetLastError());
@@ -768,12 +800,12 @@ static nd_status enqueue_prefill(nd_ctx* ctx, nd_prefill* p, nd_kv* kv, hipStrea
     ND_HIP(ctx, mark(O));
     ND_HIP(ctx, nd_launch_gemm(&dec->wqkv[l], p->digits, p->fm, p->qkv, qkv_rows, M, 0, s));
     ND_HIP(ctx, mark(G));
-    hipLaunchKernelGGL(qk_rope_store_kernel, dim3(dec->heads + dec->kv_heads, M), dim3(64), 0, s,
-                       p->qkv, qkv_rows, dec->heads, dec->kv_heads,
-                       dec->norms + dec->q_off + (size_t)l * kHd,
-                       dec->norms + dec->k_off + (size_t)l * kHd, dec->inv_freq, p->rope,
-                       nullptr, p->position0, p->q, (int8_t*)kv->k, (int8_t*)kv->v, kv->ks,
-                       kv->vs, l, kv->kv_heads, kv->alloc, 0u);
+    const nd::RopeStore rs{dec->heads, dec->kv_heads, dec->norms + dec->q_off + (size_t)l * kHd,
+                           dec->norms + dec->k_off + (size_t)l * kHd, p->rope, nullptr, p->q,
+                           (int8_t*)kv->k, (int8_t*)kv->v, kv->ks, kv->vs, l, kv->kv_heads,
+                           kv->alloc, 0u};
+    hipLaunchKernelGGL(rope_store_rows_kernel, dim3(dec->heads + 2 * dec->kv_heads, (M + 15) / 16),
+                       dim3(256), 0, s, p->qkv, qkv_rows, p->position0, M, rs);
     ND_HIP(ctx, hipGetLastError());
     ND_HIP(ctx, mark(O));
     ND_HIP(ctx, nd_launch_attention_batch(kv, l, p->positions, M, dec->kv_heads, 0u, rep, last,

@@ -45,6 +45,17 @@ __device__ __forceinline__ float norm_rope(double x, const float* __restrict__ s
   return lane < 32 ? (float)(mine * cs - other * sn) : (float)(mine * cs + other * sn);
 }
 
+// rint(x / s) of a #storeKV code, inv = 1 / s: x inv is within |x / s| 2^-51 of
+// x / s, below 6e-14 for the codes' range, so unless it lies within 1e-12 of a
+// half-integer both round to the same code; there (and for NaN) the division
+// decides.
+__device__ __forceinline__ int8_t kv_code(double x, double s, double inv) {
+  const double q = x * inv;
+  double c = rint(q);
+  if (!(fabs(fabs(q - c) - 0.5) > 1e-12)) c = rint(x / s);
+  return c != c ? (int8_t)0 : (int8_t)(int)c;
+}
+
 // #storeKV of one row: m = max(1e-12, max|x|), s = m / 127 in float64, scale
 // f32(s), code = roundTiesToEven(x / s) (NaN -> 0).
 __device__ __forceinline__ void quant_store(float val, size_t row, uint32_t lane,
@@ -109,6 +120,56 @@ __device__ __forceinline__ void rope_store_rows(const float (&x)[R], const uint3
         pos[r];
     quant_store(x[r], row, lane, p.Vc, p.Vs);
   }
+}
+
+// Four rows of one column head on a wave, 16 lanes a row: lane l holds
+// dimensions 2 (l % 16) + {0, 1} and 32 more of each (x[0..1], x[2..3]), the two
+// pairs a rotation mixes, so the row's float64 square root, divisions and
+// scale are taken once for four rows instead of once for each.
+struct Head16 {
+  float x[4];
+};
+
+__device__ __forceinline__ float row_max_js(float v) {
+  v = js_max(v, dpp<kQuadXor1>(v));
+  v = js_max(v, dpp<kQuadXor2>(v));
+  v = js_max(v, dpp<kHalfMirror>(v));
+  return js_max(v, dpp<kRowMirror>(v));
+}
+
+// Norm and rotation of the row (scale: the norm weights of the lane's
+// dimensions; sc: (sin, cos) of its two pairs).
+__device__ __forceinline__ void norm_rope16(Head16& v, const float (&scale)[4],
+                                            const double2 (&sc)[2]) {
+  double ss = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ss += (double)v.x[i] * (double)v.x[i];
+  const double inv = 1.0 / sqrt(row_sum(ss) / kRopeHd + 1e-6);
+  double n[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) n[i] = (float)((1.0 + (double)scale[i]) * (double)v.x[i] * inv);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    v.x[i] = (float)(n[i] * sc[i].y - n[i + 2] * sc[i].x);
+    v.x[i + 2] = (float)(n[i + 2] * sc[i].y + n[i] * sc[i].x);
+  }
+}
+
+// #storeKV of the row into `row` of codes and scales.
+__device__ __forceinline__ void quant_store16(const Head16& v, size_t row, uint32_t l16,
+                                              int8_t* __restrict__ codes,
+                                              float* __restrict__ scales) {
+  const float a = row_max_js(js_max(js_max(fabsf(v.x[0]), fabsf(v.x[1])),
+                                    js_max(fabsf(v.x[2]), fabsf(v.x[3]))));
+  const double mm = (a != a) ? (double)a : fmax(1e-12, (double)a);
+  const double sc = mm / 127.0, inv = 1.0 / sc;
+  uint32_t c[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c[i] = (uint8_t)kv_code((double)v.x[i], sc, inv);
+  uint16_t* at = reinterpret_cast<uint16_t*>(codes + row * kRopeHd) + l16;
+  at[0] = (uint16_t)(c[0] | c[1] << 8);
+  at[16] = (uint16_t)(c[2] | c[3] << 8);
+  if (l16 == 0) scales[row] = (float)sc;
 }
 
 }  // namespace nd

@@ -30,6 +30,7 @@
 #include "nd_cq.hpp"
 #include "nd_attention.hpp"
 #include "nd_internal.hpp"
+#include "nd_rope.hpp"
 #include "nd_wave.hpp"
 
 namespace {
@@ -2232,28 +2233,49 @@ __global__ void n2_ring_store_kernel(const float* __restrict__ ekv, float* __res
       ekv[((size_t)m * n_sites + s) * 2 * d + d + i];
 }
 
-// Query/key norm + RoPE and the K/V append of every batch position: one wave
-// per (head, position), four heads of a position to a workgroup (a workgroup
-// per head took the dispatcher longer than the work, and every head its own
-// float64 sincos: 6.7 us at 640 positions of 16 heads); qkvg rows [q | k | v |
-// gate] with stride ld.
+// Query/key norm + RoPE and the K/V append of every batch position: 16 lanes
+// per (head, position) (nd_rope.hpp), a column head of 16 positions to a
+// workgroup; qkvg rows [q | k | v | gate] with stride ld.
 __global__ __launch_bounds__(256) void n2_rope_store_batch_kernel(
     const float* __restrict__ qkvg, uint32_t ld, uint32_t heads, uint32_t kv_heads,
     const float* __restrict__ q_norm, const float* __restrict__ k_norm,
-    const double2* __restrict__ rope, uint32_t p0, float* __restrict__ q_out,
+    const double2* __restrict__ rope, uint32_t p0, uint32_t M, float* __restrict__ q_out,
     void* __restrict__ Kc, void* __restrict__ Vc, float* __restrict__ Ks,
     float* __restrict__ Vs, uint32_t layer, uint32_t alloc, uint32_t sink, uint32_t window,
     uint32_t f32) {
-  const uint32_t b = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t m = blockIdx.y, lane = threadIdx.x & 63, pos = p0 + m;
-  if (b >= heads + 2 * kv_heads) return;
+  const uint32_t b = blockIdx.x, lane = threadIdx.x & 63, l16 = lane & 15;
+  const uint32_t m = blockIdx.y * 16 + 4 * (threadIdx.x >> 6) + (lane >> 4);
+  const bool live = m < M;
+  const uint32_t mc = live ? m : M - 1;
   const int role = b < heads ? 0 : (b < heads + kv_heads ? 1 : 2);
   const uint32_t h = role == 0 ? b : (role == 1 ? b - heads : b - heads - kv_heads);
-  const float val = qkvg[(size_t)m * ld + (size_t)b * kHd + lane];
-  const double2 sc = rope[(size_t)m * 32 + (lane & 31)];
-  head_epilogue(val, lane, role, sc.x, sc.y, role == 0 ? q_norm[lane] : k_norm[lane],
-                q_out + ((size_t)m * heads + h) * kHd, Kc, Vc, Ks, Vs,
-                ((size_t)layer * kv_heads + h) * alloc, kv_slot(pos, sink, window), alloc, f32);
+  const float* src = qkvg + (size_t)mc * ld + (size_t)b * kHd + 2 * l16;
+  const float2 lo = *reinterpret_cast<const float2*>(src);
+  const float2 hi = *reinterpret_cast<const float2*>(src + 32);
+  nd::Head16 v{{lo.x, lo.y, hi.x, hi.y}};
+  if (role != 2) {
+    const float* w = (role == 0 ? q_norm : k_norm) + 2 * l16;
+    const float scale[4] = {w[0], w[1], w[32], w[33]};
+    const double2* tab = rope + (size_t)mc * 32 + 2 * l16;
+    const double2 sc[2] = {tab[0], tab[1]};
+    nd::norm_rope16(v, scale, sc);
+  }
+  if (!live) return;
+  const size_t slot = kv_slot(p0 + m, sink, window);
+  float* dst = q_out + ((size_t)m * heads + h) * kHd;
+  if (role != 0) {
+    if (slot >= alloc) return;  // the host keeps positions below the runtime limit
+    const size_t row = ((size_t)layer * kv_heads + h) * alloc + slot;
+    if (!f32) {
+      nd::quant_store16(v, row, l16, reinterpret_cast<int8_t*>(role == 1 ? Kc : Vc),
+                        role == 1 ? Ks : Vs);
+      return;
+    }
+    dst = reinterpret_cast<float*>(role == 1 ? Kc : Vc) + row * kHd;
+    if (l16 == 0) (role == 1 ? Ks : Vs)[row] = 1.f;
+  }
+  *reinterpret_cast<float2*>(dst + 2 * l16) = make_float2(v.x[0], v.x[1]);
+  *reinterpret_cast<float2*>(dst + 32 + 2 * l16) = make_float2(v.x[2], v.x[3]);
 }
 
 // Cache rows between the ring and the linear prompt cache: one wave per
@@ -3473,10 +3495,10 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
     if ((e = parts_product(n->wqkvg[l], n->cq ? n->qkv_part[l].data() : nullptr, 4, n->pf_ain, D,
                            D, n->pf_qkvg, qkv_ld)) != hipSuccess)
       return e;
-    hipLaunchKernelGGL(n2_rope_store_batch_kernel, dim3((d.heads + 2 * d.kv_heads + 3) / 4, M),
+    hipLaunchKernelGGL(n2_rope_store_batch_kernel, dim3(d.heads + 2 * d.kv_heads, (M + 15) / 16),
                        dim3(256), 0, s, n->pf_qkvg, qkv_ld, d.heads, d.kv_heads,
                        n->params + n->o_qn + (size_t)l * kHd, n->params + n->o_kn + (size_t)l * kHd,
-                       n->pf_rope, p0, n->pf_q, kv.k, kv.v, kv.ks, kv.vs, l, kv.alloc, kv.sink,
+                       n->pf_rope, p0, M, n->pf_q, kv.k, kv.v, kv.ks, kv.vs, l, kv.alloc, kv.sink,
                        nd_kv_linear(&kv) ? 0u : kv.window, kv.mode == ND_KV_FLOAT32 ? 1u : 0u);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     e = nd_launch_attention_batch(&kv, l, n->pf_positions, M, d.kv_heads, 0u,
