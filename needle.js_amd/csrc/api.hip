@@ -130,6 +130,7 @@ void nd_xcd_override(bool off) {
 
 static void free_mat_buffers(nd_mat* m) {
   hipFree(m->w);
+  hipFree(m->wt);
   hipFree(m->scales);
   hipFree(m->packed);
   hipFree(m->norms);
@@ -281,11 +282,10 @@ static nd_status upload(nd_ctx* ctx, const void* w, const void* s, uint32_t n, u
   if (e == hipSuccess) e = hipMalloc(&m->scales, sb);
   if (e == hipSuccess) e = hipMemcpyAsync(m->w, w, wb, kind, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->scales, s, sb, kind, ctx->stream);
+  if (e == hipSuccess) e = nd_tile_weights(m->w, n, k, &m->wt, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
-    hipFree(m->w);
-    hipFree(m->scales);
-    delete m;
+    free_mat_buffers(m);
     return nd_hip_fail(ctx, e, "matrix upload");
   }
   ctx->mats.insert(m);

@@ -65,7 +65,7 @@ constexpr uint32_t kTernaryBits = 5;
 
 
 struct BatchArgs {
-  const uint8_t* w;      // int8 codes [n][k] or packed codes [n][row_bytes]
+  const uint8_t* w;      // int8 codes (nd_tile_weights) or packed codes [n][row_bytes]
   const void* s;         // fp32 scales or binary16 norms [n][groups]
   const float* x;
   float* y;
@@ -201,12 +201,11 @@ __global__ __launch_bounds__(64 * kWaves * KW) void batch_matvec_kernel(BatchArg
   auto load_w = [&](Weights& w, uint32_t chunk) {
     const uint32_t u0 = chunk * kUnits;
     if constexpr (!kCq) {
-      const int8_t* base = reinterpret_cast<const int8_t*>(a.w) + (size_t)wrow * a.k +
-                           (kb & 1) * 16 + (kb >> 1) * 32;
+      const uint8_t* base = a.w + nd_tile_row(wrow, a.k) + kb * 256;
 #pragma unroll
       for (uint32_t p = 0; p < kUnits / 2; ++p)
         w.q[p] = *reinterpret_cast<const u32x4*>(
-            base + (size_t)(u0 + 2 * p < a.units ? u0 + 2 * p : 0) * 32);
+            base + (size_t)(u0 + 2 * p < a.units ? u0 / 2 + p : 0) * 1024);
     } else {
       // 16-byte pieces of the rows' chunk; one that starts past the row
       // rereads its start, one that straddles its end runs into the next row
@@ -646,7 +645,7 @@ hipError_t nd_launch_batch_matvec(const nd_mat* m, const float* x, uint32_t batc
   if (!nd_batch_matvec_fits(m, batch)) return hipErrorInvalidValue;
   BatchArgs a{};
   const uint32_t width = m->bits ? m->kpad : m->k;
-  a.w = m->bits ? m->packed : reinterpret_cast<const uint8_t*>(m->w);
+  a.w = m->bits ? m->packed : reinterpret_cast<const uint8_t*>(m->wt);
   a.s = m->bits ? (const void*)m->norms : (const void*)m->scales;
   a.x = x;
   a.y = y;

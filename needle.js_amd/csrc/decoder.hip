@@ -318,6 +318,7 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
                            ctx->stream);
       row += p->n;
     }
+    if (e == hipSuccess) e = nd_tile_weights(m.w, m.n, m.k, &m.wt, ctx->stream);
     dec->wo.push_back(d->wo[l]);
     dec->wup.push_back(d->wup[l]);
     dec->wdown.push_back(d->wdown[l]);
@@ -354,6 +355,7 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
   if (e != hipSuccess) {
     for (auto& m : dec->wqkv) {
       hipFree(m.w);
+      hipFree(m.wt);
       hipFree(m.scales);
     }
     hipFree(dec->norms);
@@ -371,6 +373,7 @@ nd_status nd_decoder_free(nd_ctx* ctx, nd_decoder* dec) {
   ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
   for (auto& m : dec->wqkv) {
     hipFree(m.w);
+    hipFree(m.wt);
     hipFree(m.scales);
   }
   hipFree(dec->norms);
@@ -794,10 +797,18 @@ static nd_status enqueue_prefill(nd_ctx* ctx, nd_prefill* p, nd_kv* kv, hipStrea
                      p->position0, M, p->rope);
   ND_HIP(ctx, hipGetLastError());
   ND_HIP(ctx, mark(O));
+  // Wo and Wdown as whole-row products that digitize their own inputs and
+  // leave the next norm's digits, or as digitize and GEMM launches.
+  const bool wide_o = nd_gemm_wide_fits(dec->wo[0], D, D, M);
+  const bool wide_d = nd_gemm_wide_fits(dec->wdown[0], F, D, M);
+  bool have = false;  // p->digits hold the next product's rows
   for (uint32_t l = 0; l < dec->layers; ++l) {
-    ND_HIP(ctx, nd_launch_digitize(p->x, D, dec->norms + dec->attn_off + (size_t)l * D, nullptr,
-                                   p->digits, p->fm, M, D, s));
-    ND_HIP(ctx, mark(O));
+    const float* attn_norm = dec->norms + dec->attn_off + (size_t)l * D;
+    const float* ffn_norm = dec->norms + dec->ffn_off + (size_t)l * D;
+    if (!have) {
+      ND_HIP(ctx, nd_launch_digitize(p->x, D, attn_norm, nullptr, p->digits, p->fm, M, D, s));
+      ND_HIP(ctx, mark(O));
+    }
     ND_HIP(ctx, nd_launch_gemm(&dec->wqkv[l], p->digits, p->fm, p->qkv, qkv_rows, M, 0, s));
     ND_HIP(ctx, mark(G));
     const nd::RopeStore rs{dec->heads, dec->kv_heads, dec->norms + dec->q_off + (size_t)l * kHd,
@@ -811,18 +822,28 @@ static nd_status enqueue_prefill(nd_ctx* ctx, nd_prefill* p, nd_kv* kv, hipStrea
     ND_HIP(ctx, nd_launch_attention_batch(kv, l, p->positions, M, dec->kv_heads, 0u, rep, last,
                                           p->q, p->o, p->partials, p->counters, s));
     ND_HIP(ctx, mark(A));
-    ND_HIP(ctx, nd_launch_digitize(p->o, D, nullptr, nullptr, p->digits, p->fm, M, D, s));
-    ND_HIP(ctx, mark(O));
-    ND_HIP(ctx, nd_launch_gemm(dec->wo[l], p->digits, p->fm, p->x, D, M, 1, s));
-    ND_HIP(ctx, mark(G));
-    ND_HIP(ctx, nd_launch_digitize(p->x, D, dec->norms + dec->ffn_off + (size_t)l * D, nullptr,
-                                   p->digits, p->fm, M, D, s));
-    ND_HIP(ctx, mark(O));
+    if (wide_o) {
+      ND_HIP(ctx, nd_launch_gemm_wide(dec->wo[l], p->o, D, p->x, D, M, ffn_norm, p->digits, p->fm, s));
+      ND_HIP(ctx, mark(G));
+    } else {
+      ND_HIP(ctx, nd_launch_digitize(p->o, D, nullptr, nullptr, p->digits, p->fm, M, D, s));
+      ND_HIP(ctx, mark(O));
+      ND_HIP(ctx, nd_launch_gemm(dec->wo[l], p->digits, p->fm, p->x, D, M, 1, s));
+      ND_HIP(ctx, mark(G));
+      ND_HIP(ctx, nd_launch_digitize(p->x, D, ffn_norm, nullptr, p->digits, p->fm, M, D, s));
+      ND_HIP(ctx, mark(O));
+    }
     ND_HIP(ctx, nd_launch_gemm(dec->wup[l], p->digits, p->fm, p->h, F, M, 2, s));
     ND_HIP(ctx, mark(G));
-    ND_HIP(ctx, nd_launch_digitize(p->h, F, nullptr, nullptr, p->digits, p->fm, M, F, s));
-    ND_HIP(ctx, mark(O));
-    ND_HIP(ctx, nd_launch_gemm(dec->wdown[l], p->digits, p->fm, p->x, D, M, 1, s));
+    have = wide_d && l + 1 < dec->layers;
+    if (wide_d) {
+      ND_HIP(ctx, nd_launch_gemm_wide(dec->wdown[l], p->h, F, p->x, D, M,
+                                      have ? attn_norm + D : nullptr, p->digits, p->fm, s));
+    } else {
+      ND_HIP(ctx, nd_launch_digitize(p->h, F, nullptr, nullptr, p->digits, p->fm, M, F, s));
+      ND_HIP(ctx, mark(O));
+      ND_HIP(ctx, nd_launch_gemm(dec->wdown[l], p->digits, p->fm, p->x, D, M, 1, s));
+    }
     ND_HIP(ctx, mark(G));
   }
   ND_HIP(ctx, nd_launch_digitize(p->x + (size_t)(M - 1) * D, D, dec->norms + dec->final_off,

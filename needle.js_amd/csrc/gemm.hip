@@ -16,8 +16,10 @@
 // MFMA operand layout (16x16x64 i8): lane l supplies 16 consecutive k of row
 // l%16 of each operand, k in [16*(l/16), +16) of the 64-wide step; the
 // accumulator's element i of lane l is row 4*(l/16)+i (weight row n) and
-// column l%16 (activation row m).  Any k order shared by both operands gives
-// the same sum, so both are read straight from row-major memory.
+// column l%16 (activation row m).  Weights come from the matrix's copy in that
+// order (nd_tile_weights), one contiguous KiB a load.
+#include <type_traits>
+
 #include "nd_internal.hpp"
 #include "nd_rope.hpp"
 #include "nd_wave.hpp"
@@ -31,6 +33,7 @@ constexpr int kKChunk = 256;             // k per LDS stage
 constexpr int kLdsRow = kKChunk + 16;    // padded row stride (bank spread)
 constexpr int kMaxSplit = 8;             // k slices of a split launch
 constexpr uint32_t kMaxNormK = 1024;     // rows the fused norm reads whole
+constexpr uint32_t kWideMinRows = 256;
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.f + __expf(-v)); }
 
@@ -109,9 +112,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_digits_kernel(
       const uint32_t ks = (uint32_t)q * 64 < kw ? q * 64 : 0;  // clamped past kw, never used
 #pragma unroll
       for (int a = 0; a < NS; ++a) {
-        const uint32_t n = n0 + a * 16 + lrow;
-        const uint32_t nn = n < N ? n : N - 1;
-        wa[q][a] = *reinterpret_cast<const v4i*>(W + (size_t)nn * K + kc + ks + lk);
+        const uint32_t n = n0 + a * 16;
+        wa[q][a] = *reinterpret_cast<const v4i*>(
+            W + ((size_t)((n < N ? n : N - 1) / 16) * (K / 64) + (kc + ks) / 64) * 1024 + lane * 16);
       }
     }
 #pragma unroll
@@ -391,13 +394,13 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
   // Weights of the chunks first.
   v4i wa[CPW][kKChunk / 64];
   {
-    const uint32_t n = n0 + lrow;
-    const int8_t* wr = W + (size_t)(n < N ? n : N - 1) * K + kc0 + lk;
+    const int8_t* wr =
+        W + ((size_t)((n0 < N ? n0 : N - 1) / 16) * (K / 64) + kc0 / 64) * 1024 + lane * 16;
 #pragma unroll
     for (int c = 0; c < CPW; ++c)
 #pragma unroll
       for (int q = 0; q < kKChunk / 64; ++q)
-        wa[c][q] = *reinterpret_cast<const v4i*>(wr + c * kKChunk + q * 64);
+        wa[c][q] = *reinterpret_cast<const v4i*>(wr + (c * (kKChunk / 64) + q) * 1024);
   }
   // Activations: row r of the tile, 16 values of each chunk (and the row's
   // other chunks for the norm; K <= kMaxNormK then).
@@ -701,10 +704,10 @@ __global__ __launch_bounds__(512) void gemm_i8_astat_kernel(
     for (int q = 0; q < (int)(kAsMaxK / 64); ++q)
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        const uint32_t n = nb + 16 * a + lrow;
+        const uint32_t n = nb + 16 * a;
         const uint32_t qs = (uint32_t)q < steps ? q : 0;
-        wa[q][a] = *reinterpret_cast<const v4i*>(W + (size_t)(n < N ? n : N - 1) * K + qs * 64 +
-                                                 lk * 16);
+        wa[q][a] = *reinterpret_cast<const v4i*>(
+            W + ((size_t)((n < N ? n : N - 1) / 16) * steps + qs) * 1024 + lane * 16);
       }
     v4i acc[2][4][3];
 #pragma unroll
@@ -764,6 +767,207 @@ __global__ __launch_bounds__(512) void gemm_i8_astat_kernel(
   }
 }
 
+// Prompt-sized product whose outputs are whole rows (N = 128 NS <= 512
+// columns, M rows in tiles of 16): y += A W^T on fp32 rows A that the
+// workgroup digitizes itself, and, with DOUT, the zero-centred RMS norm of the
+// new rows and their digits for the next product.  A tile of all N columns
+// digitizes each row once and has the row's sum of squares and maximum at
+// hand, so the two digitize launches around such a product (5.4 and 7.7 us at
+// 2048 rows of 512 and 2048) and the fp32 round trips between them go away;
+// 16 rows keep 2048 of them on 128 workgroups.
+//
+// 8 waves: wave w digitizes rows 2 w and 2 w + 1 (digitize_rows_kernel's
+// split, the same bits) into LDS, then takes columns [16 NS w, +16 NS) over
+// all of K: weights straight from memory to registers, 256 k ahead of the
+// products (the first 256 k and the addends issued at entry), digits from LDS
+// (row stride K + 16 bytes: 16 rows cover all banks).  Lane l holds columns 4
+// (l / 16) + i of row l % 16.  Bound by the weights entering each CU: N K
+// bytes a workgroup.
+template <int NS, int KMAX, bool DOUT>
+__global__ __launch_bounds__(512) void gemm_i8_wide_kernel(
+    const int8_t* __restrict__ W, const float* __restrict__ sw, const float* __restrict__ X,
+    uint32_t ldx, float* __restrict__ Y, uint32_t ldy, uint32_t M, uint32_t K,
+    const float* __restrict__ norm, int8_t* __restrict__ Dout, float* __restrict__ fm_out) {
+  constexpr uint32_t N = 128 * NS;
+  constexpr int VEC = KMAX / 256;
+  constexpr int kQ = 4;  // 64-wide k steps per weight stage
+  constexpr uint32_t kOutLd = N + 16;
+  __shared__ __attribute__((aligned(16))) int8_t lds[3 * 16 * (KMAX + 16)];
+  static_assert(sizeof(lds) >= 3 * 16 * kOutLd, "the output digits fit");
+  __shared__ float s_fm[16], s_red[2][8][16];
+  const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const uint32_t lrow = lane & 15, lk = lane >> 4;
+  const uint32_t m0 = blockIdx.x * 16, n0 = wave * 16 * NS;
+  const uint32_t kld = K + 16;
+  const uint32_t steps = K / 64;
+
+  // The rows, then the first weights, then the addends.
+  float4 v[2][VEC];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t m = m0 + 2 * wave + r;
+    const float4* x = reinterpret_cast<const float4*>(X + (size_t)(m < M ? m : M - 1) * ldx);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const uint32_t u = lane + 64 * i;
+      v[r][i] = x[u < K / 4 ? u : 0];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  v4i wn[kQ][NS];
+  auto load_w = [&](uint32_t q0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+#pragma unroll
+      for (int a = 0; a < NS; ++a) {
+        const uint32_t qs = q0 + q < steps ? q0 + q : 0;  // clamped, never used
+        wn[q][a] = *reinterpret_cast<const v4i*>(W + ((size_t)(n0 / 16 + a) * steps + qs) * 1024 +
+                                                 lane * 16);
+      }
+  };
+  load_w(0);
+  const uint32_t mo = m0 + lrow;
+  const float* yrow = Y + (size_t)(mo < M ? mo : M - 1) * ldy + n0 + 4 * lk;
+  float4 add[NS];
+#pragma unroll
+  for (int a = 0; a < NS; ++a) add[a] = *reinterpret_cast<const float4*>(yrow + 16 * a);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t lr = 2 * wave + r;
+    const bool live = m0 + lr < M;  // rows past M multiply as zeros
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      if (!live || lane + 64 * i >= K / 4) v[r][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[r][i].x), fabsf(v[r][i].y)),
+                               fmaxf(fabsf(v[r][i].z), fabsf(v[r][i].w))));
+    }
+    amax = nd::row_max(amax);
+    amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
+                 fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
+    int e = 0;
+    if (amax > 0.f) {
+      frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
+      e -= 1;
+    }
+    const float up = ldexpf(1.f, 21 - e);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const uint32_t u = lane + 64 * i;
+      if (u >= K / 4) continue;
+      uint32_t d0, d1, d2;
+      digit_words(digit_bias(v[r][i].x, up), digit_bias(v[r][i].y, up),
+                  digit_bias(v[r][i].z, up), digit_bias(v[r][i].w, up), d0, d1, d2);
+      int8_t* at = lds + lr * kld + 4 * u;
+      *reinterpret_cast<uint32_t*>(at) = d0;
+      *reinterpret_cast<uint32_t*>(at + 16 * kld) = d1;
+      *reinterpret_cast<uint32_t*>(at + 32 * kld) = d2;
+    }
+    if (lane == 0) s_fm[lr] = ldexpf(1.f, e - 21);
+  }
+  nd::lds_barrier();
+
+  v4i acc[NS][3];
+#pragma unroll
+  for (int a = 0; a < NS; ++a)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) acc[a][j] = v4i{0, 0, 0, 0};
+  for (uint32_t q0 = 0; q0 < steps; q0 += kQ) {
+    v4i w[kQ][NS];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+#pragma unroll
+      for (int a = 0; a < NS; ++a) w[q][a] = wn[q][a];
+    if (q0 + kQ < steps) load_w(q0 + kQ);
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const uint32_t qs = q0 + q;
+      if (qs >= steps) break;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const v4i db = *reinterpret_cast<const v4i*>(lds + (j * 16 + lrow) * kld + qs * 64 + lk * 16);
+#pragma unroll
+        for (int a = 0; a < NS; ++a)
+          acc[a][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[q][a], db, acc[a][j], 0, 0, 0);
+      }
+    }
+  }
+
+  const float f = s_fm[lrow];
+  float y[NS][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int a = 0; a < NS; ++a) {
+    const float4 s4 = *reinterpret_cast<const float4*>(sw + n0 + 16 * a + 4 * lk);
+    const float swv[4] = {s4.x, s4.y, s4.z, s4.w};
+    const float o[4] = {add[a].x, add[a].y, add[a].z, add[a].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float c = (float)acc[a][0][i] + 256.f * (float)acc[a][1][i] +
+                      65536.f * (float)acc[a][2][i];
+      y[a][i] = o[i] + swv[i] * (f * c);
+      ss = fmaf(y[a][i], y[a][i], ss);
+    }
+    if (mo < M)
+      *reinterpret_cast<float4*>(Y + (size_t)mo * ldy + n0 + 16 * a + 4 * lk) =
+          make_float4(y[a][0], y[a][1], y[a][2], y[a][3]);
+  }
+  if constexpr (!DOUT) return;
+  // The new rows' norm and digits: row sums and maxima over the lanes of a
+  // row and the waves.
+  ss = nd::sum_xor<16>(ss);
+  ss = nd::sum_xor<32>(ss);
+  if (lk == 0) s_red[0][wave][lrow] = ss;
+  nd::lds_barrier();  // also: every wave is done with the digits
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) total += s_red[0][w][lrow];
+  const float inv = 1.f / sqrtf(total / (float)N + 1e-6f);
+  float amax = 0.f;
+#pragma unroll
+  for (int a = 0; a < NS; ++a) {
+    const float4 w4 = *reinterpret_cast<const float4*>(norm + n0 + 16 * a + 4 * lk);
+    const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      y[a][i] = (1.f + wv[i]) * y[a][i] * inv;
+      amax = fmaxf(amax, fabsf(y[a][i]));
+    }
+  }
+  amax = nd::max_xor<16>(amax);
+  amax = nd::max_xor<32>(amax);
+  if (lk == 0) s_red[1][wave][lrow] = amax;
+  nd::lds_barrier();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) amax = fmaxf(amax, s_red[1][w][lrow]);
+  int e = 0;
+  if (amax > 0.f) {
+    frexpf(amax, &e);
+    e -= 1;
+  }
+  const float up = ldexpf(1.f, 21 - e);
+#pragma unroll
+  for (int a = 0; a < NS; ++a) {
+    uint32_t d0, d1, d2;
+    digit_words(digit_bias(y[a][0], up), digit_bias(y[a][1], up), digit_bias(y[a][2], up),
+                digit_bias(y[a][3], up), d0, d1, d2);
+    int8_t* at = lds + lrow * kOutLd + n0 + 16 * a + 4 * lk;
+    *reinterpret_cast<uint32_t*>(at) = d0;
+    *reinterpret_cast<uint32_t*>(at + 16 * kOutLd) = d1;
+    *reinterpret_cast<uint32_t*>(at + 32 * kOutLd) = d2;
+  }
+  if (wave == 0 && lk == 0 && mo < M) fm_out[mo] = ldexpf(1.f, e - 21);
+  nd::lds_barrier();
+  const size_t plane = (size_t)M * N;
+  for (uint32_t u = t; u < 3 * 16 * N / 16; u += 512) {
+    const uint32_t j = u / N, r = u % N / (N / 16), c = u % (N / 16) * 16;
+    if (m0 + r < M)
+      *reinterpret_cast<uint4*>(Dout + j * plane + (size_t)(m0 + r) * N + c) =
+          *reinterpret_cast<const uint4*>(lds + (j * 16 + r) * kOutLd + c);
+  }
+}
+
 using F32aFn = void (*)(const int8_t*, const float*, const float*, uint32_t, const float*, float*,
                         uint32_t, uint32_t, uint32_t, uint32_t, float*, uint32_t*, nd::RopeStore,
                         uint32_t);
@@ -793,6 +997,29 @@ GemmFn pick(uint32_t ms, uint32_t ns, bool pf) {
 }
 
 }  // namespace
+
+namespace {
+// Thread e: 16 bytes of block e / 64.
+__global__ __launch_bounds__(256) void tile_weights_kernel(const int8_t* __restrict__ w, uint32_t n,
+                                                           uint32_t k, uint64_t units,
+                                                           uint4* __restrict__ wt) {
+  const uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= units) return;
+  const uint32_t l = (uint32_t)e & 63, q = (uint32_t)((e >> 6) % (k / 64));
+  const uint64_t row = (e >> 6) / (k / 64) * 16 + (l & 15);
+  wt[e] = row < n ? *reinterpret_cast<const uint4*>(w + row * k + q * 64 + (l >> 4) * 16)
+                  : make_uint4(0, 0, 0, 0);
+}
+}  // namespace
+
+hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t** wt, hipStream_t s) {
+  const uint64_t units = ((uint64_t)n + 15) / 16 * k;
+  hipError_t e = hipMalloc(wt, units * 16);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(tile_weights_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, w,
+                     n, k, units, reinterpret_cast<uint4*>(*wt));
+  return hipGetLastError();
+}
 
 hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, float* norm_out,
                               int8_t* digits, float* fm, uint32_t M, uint32_t K, hipStream_t s) {
@@ -846,13 +1073,13 @@ hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm
     const uint32_t gc = (strips / groups) * kAsStrip;
     const dim3 grid(groups, mt);
     if (epilogue == 0)
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<0>, grid, dim3(512), 0, s, w->w, w->scales, digits,
+      hipLaunchKernelGGL(gemm_i8_astat_kernel<0>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
                          fm, y, M, w->n, w->k, ldy, gc);
     else if (epilogue == 1)
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<1>, grid, dim3(512), 0, s, w->w, w->scales, digits,
+      hipLaunchKernelGGL(gemm_i8_astat_kernel<1>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
                          fm, y, M, w->n, w->k, ldy, gc);
     else
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<2>, grid, dim3(512), 0, s, w->w, w->scales, digits,
+      hipLaunchKernelGGL(gemm_i8_astat_kernel<2>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
                          fm, y, M, w->n, w->k, ldy, gc);
     return hipGetLastError();
   }
@@ -883,9 +1110,43 @@ hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm
       S *= 2;
     grid.z = S;
   }
-  hipLaunchKernelGGL(f, grid, dim3(kGemmThreads), 0, s, w->w, w->scales, digits, fm, y, M, w->n,
+  hipLaunchKernelGGL(f, grid, dim3(kGemmThreads), 0, s, w->wt, w->scales, digits, fm, y, M, w->n,
                      w->k, ldy, w->k / grid.z, split ? split->partials : nullptr,
                      split ? split->counters : nullptr);
+  return hipGetLastError();
+}
+
+// The whole-row product above: true when it takes (w, M).  Prompts through 8
+// layers of 512 x 512 and 512 x 2048, whole-row against tiled products with
+// their digitize launches: 496 and 513 us at 256 rows, 557 and 598 at 512, 695
+// and 838 at 1024.
+bool nd_gemm_wide_fits(const nd_mat* w, uint32_t ldx, uint32_t ldy, uint32_t M) {
+  return M >= kWideMinRows && (w->n == 128 || w->n == 256 || w->n == 512) && w->k % 64 == 0 &&
+         w->k <= 2048 && ldx % 4 == 0 && ldy % 4 == 0;
+}
+
+hipError_t nd_launch_gemm_wide(const nd_mat* w, const float* x, uint32_t ldx, float* y,
+                               uint32_t ldy, uint32_t M, const float* norm, int8_t* digits,
+                               float* fm, hipStream_t s) {
+  if (!nd_gemm_wide_fits(w, ldx, ldy, M) ||
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
+        reinterpret_cast<uintptr_t>(norm) | reinterpret_cast<uintptr_t>(digits)) & 15))
+    return hipErrorInvalidValue;
+  using Fn = void (*)(const int8_t*, const float*, const float*, uint32_t, float*, uint32_t,
+                      uint32_t, uint32_t, const float*, int8_t*, float*);
+  auto pick = [&](auto ns, auto k) -> Fn {
+    constexpr int NS = decltype(ns)::value, KM = decltype(k)::value;
+    return norm ? &gemm_i8_wide_kernel<NS, KM, true> : &gemm_i8_wide_kernel<NS, KM, false>;
+  };
+  auto pick_k = [&](auto ns) -> Fn {
+    return w->k <= 512 ? pick(ns, std::integral_constant<int, 512>())
+                       : pick(ns, std::integral_constant<int, 2048>());
+  };
+  const Fn f = w->n == 512   ? pick_k(std::integral_constant<int, 4>())
+               : w->n == 256 ? pick_k(std::integral_constant<int, 2>())
+                             : pick_k(std::integral_constant<int, 1>());
+  hipLaunchKernelGGL(f, dim3((M + 15) / 16), dim3(512), 0, s, w->wt, w->scales, x, ldx, y, ldy, M,
+                     w->k, norm, digits, fm);
   return hipGetLastError();
 }
 
@@ -921,7 +1182,7 @@ hipError_t nd_launch_gemm_f32(const nd_mat* w, const float* x, uint32_t ldx, con
   const uint32_t S = pair ? chunks / 2 : chunks;
   const F32aFn f = pair ? (norm ? pick_f32a<true, 2>(epilogue) : pick_f32a<false, 2>(epilogue))
                         : (norm ? pick_f32a<true, 1>(epilogue) : pick_f32a<false, 1>(epilogue));
-  hipLaunchKernelGGL(f, dim3((w->n + 63) / 64, (M + 15) / 16, S), dim3(kGemmThreads), 0, s, w->w,
+  hipLaunchKernelGGL(f, dim3((w->n + 63) / 64, (M + 15) / 16, S), dim3(kGemmThreads), 0, s, w->wt,
                      w->scales, x, ldx, norm, y, M, w->n, w->k, ldy, split->partials,
                      split->counters, rope ? *rope : nd::RopeStore{}, nd_xcd_local() ? 1u : 0u);
   return hipGetLastError();

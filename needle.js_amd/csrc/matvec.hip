@@ -263,8 +263,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void matvec_mfma_fused_kernel(
   const uint32_t r16 = lane & 15, kb = lane >> 4;
   const uint32_t row0 = blockIdx.x * 16;
   const uint32_t row = row0 + r16;
-  const int8_t* wrow = W + (size_t)(row_start + (row < row_count ? row : row_count - 1)) * K +
-                       (kb & 1) * 16 + (kb >> 1) * 32;
+  const int8_t* wrow =
+      W + nd_tile_row(row_start + (row < row_count ? row : row_count - 1), K) + kb * 256;
   const uint32_t ng = K / 32, npairs = ng / 2;
   const uint32_t per_wave = (npairs + kMfmaWaves - 1) / kMfmaWaves;
 
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void matvec_mfma_fused_kernel(
     for (int i = 0; i < NP; ++i) {
       const uint32_t p = wave + kMfmaWaves * (base + i);
       const uint32_t pc = p < npairs ? p : 0;
-      wv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow + (size_t)pc * 64));
+      wv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow + (size_t)pc * 1024));
     }
   };
   auto compute = [&](uint32_t base) {
@@ -465,13 +465,13 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void matvec_mfma_slice_kernel(
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   const uint32_t row = row0 + 16 * tile + r16;
-  const int8_t* wrow = W + (size_t)(row_start + (row < row_count ? row : row_count - 1)) * K + k0 +
-                       (kb & 1) * 16 + (kb >> 1) * 32;
+  const int8_t* wrow = W + nd_tile_row(row_start + (row < row_count ? row : row_count - 1), K) +
+                       (size_t)(k0 / 64) * 1024 + kb * 256;
   u32x4 wv[NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i)
     wv[i] = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4*>(wrow + (size_t)(NP * wq + i) * 64));
+        reinterpret_cast<const u32x4*>(wrow + (size_t)(NP * wq + i) * 1024));
   __builtin_amdgcn_sched_barrier(0);
 
   // Slice maxima: a batch row spans kUnits / 64 waves.
@@ -716,7 +716,7 @@ hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uin
         const uint32_t pairs_per_wave = (m->k / 64 + kMfmaWaves - 1) / kMfmaWaves;
         const auto kern = pairs_per_wave >= 2 ? &matvec_mfma_fused_kernel<2>
                                               : &matvec_mfma_fused_kernel<1>;
-        hipLaunchKernelGGL(kern, dim3((row_count + 15) / 16), dim3(64 * kMfmaWaves), 0, s, m->w,
+        hipLaunchKernelGGL(kern, dim3((row_count + 15) / 16), dim3(64 * kMfmaWaves), 0, s, m->wt,
                            m->scales, xb, x_stride, yb, m->k, m->k / m->g, gshift, row_start,
                            row_count, bc, y_stride);
         hipError_t e = hipGetLastError();
@@ -739,7 +739,7 @@ hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uin
         const uint32_t rc = row_count - r0 < block ? row_count - r0 : block;
         const auto kern = wide ? &matvec_mfma_slice_kernel<4> : &matvec_mfma_slice_kernel<2>;
         const uint32_t rpx = ((rc + 63) / 64 + 7) / 8;  // row blocks per XCD
-        hipLaunchKernelGGL(kern, dim3(8 * rpx * slices), dim3(64 * kMfmaWaves), 0, s, m->w,
+        hipLaunchKernelGGL(kern, dim3(8 * rpx * slices), dim3(64 * kMfmaWaves), 0, s, m->wt,
                            m->scales, xb, x_stride, P, counters, yb + r0, y_stride, m->k,
                            m->k / m->g, gshift, row_start + r0, rc, bc,
                            nd_xcd_local() ? 1u : 0u);

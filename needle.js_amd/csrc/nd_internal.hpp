@@ -22,6 +22,7 @@ constexpr size_t kCqSlack = 16;
 
 struct nd_mat {
   int8_t* w = nullptr;      // [n][k] int8 codes, row-major
+  int8_t* wt = nullptr;     // the same codes in MFMA operand order (nd_tile_weights)
   float* scales = nullptr;  // [n][k / g]
   uint32_t n = 0, k = 0, g = 0;
   // Cactus-Quant form (bits != 0; w and scales unused): packed codes
@@ -241,6 +242,17 @@ hipError_t nd_launch_select_mask(const float* logits, uint32_t batch, uint32_t v
 // digitize.
 hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, float* norm_out,
                               int8_t* digits, float* fm, uint32_t M, uint32_t K, hipStream_t s);
+// The codes w [n][k] (k % 64 == 0) in MFMA operand order, allocated into *wt:
+// 1 KiB blocks [row / 16][k / 64], lane l of a block holding row l % 16, k
+// [16 (l / 16), +16).  Consecutive lanes of an MFMA operand are different rows,
+// and a wave's load is served four adjacent lanes (64 contiguous bytes) a
+// cycle: read from row-major memory every lane is a request of its own, 34
+// KB/us into a CU against 105-117 from this order (a 1 MB matrix read by 64 to
+// 256 workgroups).  Rows past n are zero.
+hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t** wt, hipStream_t s);
+inline __host__ __device__ size_t nd_tile_row(uint32_t row, uint32_t k) {
+  return (size_t)(row >> 4) * (k / 64) * 1024 + (row & 15) * 16;
+}
 // Split-k workspace of nd_launch_gemm: partial sums (partial_floats floats)
 // and counter_count arrival counters, zero when first used and left zero by
 // every launch that completes.  Launches that share a workspace must be
@@ -254,6 +266,14 @@ struct nd_gemm_split {
 hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm, float* y,
                           uint32_t ldy, uint32_t M, int epilogue, hipStream_t s,
                           const nd_gemm_split* split = nullptr);
+// y += x W^T for prompt-sized M and n of 128, 256 or 512 (nd_gemm_wide_fits) on
+// fp32 rows x [M][ldx], digitized inside the launch; with `norm`, the new rows
+// of y are then RMS-normalized (math.ts:16-32) and their digits and factors
+// written for the next nd_launch_gemm.  Pointers 16-byte aligned.
+bool nd_gemm_wide_fits(const nd_mat* w, uint32_t ldx, uint32_t ldy, uint32_t M);
+hipError_t nd_launch_gemm_wide(const nd_mat* w, const float* x, uint32_t ldx, float* y,
+                               uint32_t ldy, uint32_t M, const float* norm, int8_t* digits,
+                               float* fm, hipStream_t s);
 // The same product on fp32 rows x [M][ldx] (optionally RMS-normalized with
 // `norm`, math.ts:16-32), digitized per 256-wide chunk inside the launch;
 // only for the shapes nd_gemm_f32_fits accepts.  Epilogue 3 (the q/k/v
