@@ -147,6 +147,7 @@ struct AttnLaunch {
   uint32_t rep;                // query heads per KV head
   uint32_t batch;
   uint32_t max_count;          // bound on every sequence's visible count
+  uint32_t first_position;     // qblock: the position of query row 0
   bool qblock;                 // query blocks of a prefill whose positions see [0, position]
   uint64_t* stamps;            // measurement form: 8 stamps per workgroup, or nullptr
   uint32_t stamp_capacity;     // workgroups the stamps hold
@@ -159,16 +160,22 @@ struct AttnLaunch {
 // key blocks one of its rows sees: those of the sinks, then those from the
 // first row's window on.  Keys of these blocks that no row sees may hold
 // anything: their scales are taken as zero and their scores masked.
-// Workgroup = (block of 64 query
-// rows, query head h, KV head h / rep), 16 waves in four groups: wave w
-// takes rows [z0 + 16 (w % 4), +16), lane l the row 16 (w % 4) + l % 16, and
-// group g = w / 4 the key blocks g, g + 4, ... (64 keys each), so each group
-// walks a quarter of the row block's keys (the causal triangle gives the
-// last row blocks the most); the four online-softmax states merge through
-// LDS at the end.  Each group streams its key blocks through its own pair of
-// LDS buffers, converting the codes to fp16 once on the way in (K as
-// stored, V transposed to [dim][key]), one barrier per step.  Per block and
-// wave:
+// Workgroup = (block of 32 query rows, query head h, KV head h / rep), 8
+// waves in four groups: wave w takes rows [z0 + 16 (w % 2), +16), lane l the row
+// 16 (w % 2) + l % 16, and group g = w / 2 the key blocks g, g + 4, ... (64 keys
+// each); the four online-softmax states merge through LDS at the end.  Each
+// group converts its key block's codes to fp16 once on the way into its LDS
+// buffer (K as stored, V transposed to [dim][key], the keys of each 32 in the
+// order a lane's A operand takes them: eight contiguous halves).
+//
+// Bound by the LDS traffic and the vector ALU (softmax, the fp16 halves of p',
+// the conversion): a thread converts four keys of eight dimensions, 12 wide
+// stores, where one dimension of V at a time took 36.  And by the causal
+// triangle: the last row blocks walk every key and the first one block.  A CU holds two workgroups, so a launch of up to 512 goes out heavy
+// blocks first, then the light ones in the opposite order, and each CU's pair
+// has about the same work; 64-row workgroups, one to a CU, left half of the
+// CUs' time idle (2048 positions, 8 heads: 33.7 us).
+// Per block and wave:
 //   S^T = K Q^T on v_mfma_f32_16x16x32_f16: A = K codes (row = key, exact in
 //   fp16), B = Q^T split into fp16 halves hi + lo of q * 2^-e (e: the row's
 //   largest magnitude, < 2^e), which hold q to 2^-24 of the row maximum; the
@@ -185,9 +192,10 @@ struct AttnLaunch {
 //   S^T product left in the lane (8 keys per lane, the A operand reads V^T at
 //   the same keys); A = V^T codes (row = dim).
 // The output row is O / (l 2^f), gated when `gate` is set (runtime.ts:503-507).
-constexpr uint32_t kPfRows = 64, kPfKeys = 64, kPfGroups = 4, kPfThreads = 256 * kPfGroups;
+constexpr uint32_t kPfRows = 32, kPfKeys = 64, kPfGroups = 4, kPfThreads = 128 * kPfGroups;
+constexpr uint32_t kPfResident = 512;  // workgroups the GPU holds, two to a CU
 constexpr uint32_t kKStrideH = 72;   // halves per key row of K in LDS (16-byte aligned rows)
-constexpr uint32_t kVtStrideH = 68;  // halves per dim row of V^T in LDS (8-byte aligned rows)
+constexpr uint32_t kVtStrideH = 72;  // halves per dim row of V^T in LDS
 struct PfBuf {
   _Float16 k[kPfKeys * kKStrideH];
   _Float16 vt[kHeadDim * kVtStrideH];
@@ -199,47 +207,75 @@ struct PfBuf {
 // over block pieces fold away: 2048 positions, 8 layers, cost 1.4% more with
 // them).
 template <bool WIN>
-__global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
+__global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
     const int8_t* __restrict__ Kc, const int8_t* __restrict__ Vc, const float* __restrict__ Ks,
     const float* __restrict__ Vs, const float* __restrict__ Q, float* __restrict__ out,
     const float* __restrict__ gate, uint32_t gate_ld, uint32_t layer, uint32_t kv_heads,
-    uint32_t alloc, uint32_t sink, uint32_t window, const uint32_t* __restrict__ positions,
-    uint32_t qrows, uint32_t q_heads, uint32_t rep, float score_scale) {
+    uint32_t alloc, uint32_t sink, uint32_t window, uint32_t p0, uint32_t qrows,
+    uint32_t q_heads, uint32_t rep, float score_scale) {
   using nd::half8;
   using nd::float4v;
   using nd::u32x2;
   typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-  __shared__ __align__(16) PfBuf s_buf[kPfGroups][2];  // [group][buffer]
-  __shared__ uint32_t s_top;
-  __shared__ uint32_t s_low;
+  __shared__ __align__(16) PfBuf s_buf[kPfGroups];
   __shared__ float s_vmax[kPfThreads / 64];
   const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const uint32_t grp = wave >> 2, wq = wave & 3, tg = t & 255;
+  const uint32_t grp = wave >> 1, wq = wave & 1, tg = t & 127;
   const uint32_t r16 = lane & 15, kb = lane >> 4;
-  const uint32_t h = blockIdx.y, kvh = h / rep;
-  const uint32_t z0 = blockIdx.x * kPfRows;
+  // Row block by rank of work (the last blocks walk the most keys): heaviest
+  // first, the second half of a launch that fits the GPU in reverse.
+  const uint32_t h = blockIdx.x % q_heads, kvh = h / rep, rank = blockIdx.x / q_heads;
+  const uint32_t blocks = gridDim.x / q_heads, heavy = (blocks + 1) / 2;
+  const uint32_t zb = gridDim.x <= kPfResident && rank >= heavy ? rank - heavy : blocks - 1 - rank;
+  const uint32_t z0 = zb * kPfRows;
   const size_t head_base = ((size_t)layer * kv_heads + kvh) * alloc;
 
-  // Keys below top = 1 + the largest position of the block's rows and, past
-  // the sinks, from low = the first position a row's window holds.
-  if (wave == 0) {
-    const bool in = z0 + t < qrows;
-    const uint32_t p1 = in ? positions[z0 + t] + 1 : 0;
-    [[maybe_unused]] uint32_t my_top = p1, my_low = in ? (WIN && p1 > window ? p1 - window : 0) : 0xffffffffu;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      my_top = max(my_top, (uint32_t)__shfl_xor((int)my_top, o, 64));
-      if constexpr (WIN) my_low = min(my_low, (uint32_t)__shfl_xor((int)my_low, o, 64));
-    }
-    if (lane == 0) {
-      s_top = my_top;
-      s_low = my_low;
-    }
-  }
-  // This lane's query row and its q values: dims 32 s + 8 kb + [0, 8).
-  const uint32_t zq = z0 + 16 * wq + r16;
+  // Row z sits at position p0 + z: keys below top = 1 + the position of the
+  // block's last row and, past the sinks, from low = the first position a row's
+  // window holds.
+  auto low_of = [&](uint32_t p) { return WIN && p + 1 > window ? p + 1 - window : 0; };
+  const uint32_t top = p0 + min(z0 + kPfRows, qrows), low = low_of(p0 + z0);
+  if (top > alloc) return;  // validated on entry; stay in bounds
+  // Step i walks the keys of block i (i < sblocks: the sinks) or i + skip.
+  uint32_t sblocks = WIN ? (min(sink, top) + kPfKeys - 1) / kPfKeys : 0;
+  if (low / kPfKeys <= sblocks) sblocks = low / kPfKeys;  // contiguous
+  const uint32_t skip = low / kPfKeys - sblocks;
+  const uint32_t nblocks = (top + kPfKeys - 1) / kPfKeys - skip;
+  auto block_key = [&](uint32_t b) { return (b < sblocks ? b : b + skip) * kPfKeys; };
+  auto seen = [&](uint32_t key) { return !WIN || key >= low || key < sink; };
+  // This lane's query row; the smallest position and the largest first
+  // windowed position of the wave's rows: blocks wholly between them need no
+  // mask.
+  const uint32_t zw = z0 + 16 * __builtin_amdgcn_readfirstlane(wq), zq = zw + r16;
   const bool q_ok = zq < qrows;
-  const uint32_t pos = q_ok ? positions[zq] : 0;
+  const uint32_t pos = q_ok ? p0 + zq : 0, row_low = low_of(pos);
+  const uint32_t wmin = zw + 15 < qrows ? p0 + zw : 0, wlow = low_of(p0 + zw + 15);
+
+  // Block loads of the group: thread tg takes keys 4 (tg / 8) + [0, 4), bytes
+  // [8 (tg % 8), +8) of their K and V rows (keys past top read the last visible
+  // slot; they are masked).
+  const uint32_t lkey = 4 * (tg >> 3), lpart = tg & 7;
+  uint2 kreg[4], vreg[4];
+  float ksr = 0.f, vsr = 0.f;
+  auto load_block = [&](uint32_t b) {
+    const uint32_t kb0 = block_key(b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const size_t row = head_base + min(kb0 + lkey + i, top - 1);
+      kreg[i] = *reinterpret_cast<const uint2*>(Kc + row * kHeadDim + 8 * lpart);
+      vreg[i] = *reinterpret_cast<const uint2*>(Vc + row * kHeadDim + 8 * lpart);
+    }
+    if (tg < kPfKeys) {
+      const uint32_t skey = min(kb0 + tg, top - 1);
+      const float kk = Ks[head_base + skey], vv = Vs[head_base + skey];
+      ksr = seen(skey) ? kk : 0.f;
+      vsr = seen(skey) ? vv : 0.f;
+    }
+  };
+
+  // Everything the first step needs is issued together, one round trip: q
+  // (dims 32 s + 8 kb + [0, 8) of the row), the visible keys' v scales for the
+  // p' scale, the group's first block.
   const float* qp = Q + ((size_t)(q_ok ? zq : 0) * q_heads + h) * kHeadDim + 8 * kb;
   float qv[2][8];
 #pragma unroll
@@ -249,27 +285,22 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     qv[s2][0] = a.x; qv[s2][1] = a.y; qv[s2][2] = a.z; qv[s2][3] = a.w;
     qv[s2][4] = b.x; qv[s2][5] = b.y; qv[s2][6] = b.z; qv[s2][7] = b.w;
   }
-  // The row's first windowed position; the smallest position and the largest
-  // such of the wave's rows: blocks wholly between them need no mask.
-  const uint32_t row_low = WIN && pos + 1 > window ? pos + 1 - window : 0;
-  uint32_t wmin = q_ok ? pos : 0, wlow = row_low;
+  constexpr uint32_t kVs = 4;  // v scales a thread loads at a time
+  float vmax = 0.f;
+  for (uint32_t i0 = 0; i0 < nblocks * kPfKeys; i0 += kVs * kPfThreads) {
+    float vs[kVs];
+    uint32_t key[kVs];
 #pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) {
-    wmin = min(wmin, (uint32_t)__shfl_xor((int)wmin, o, 64));
-    if constexpr (WIN) wlow = max(wlow, (uint32_t)__shfl_xor((int)wlow, o, 64));
+    for (uint32_t u = 0; u < kVs; ++u) {
+      const uint32_t i = i0 + u * kPfThreads + t;
+      key[u] = i < nblocks * kPfKeys ? block_key(i / kPfKeys) + i % kPfKeys : top;
+      vs[u] = Vs[head_base + min(key[u], top - 1)];
+    }
+    if (i0 == 0) load_block(grp);
+#pragma unroll
+    for (uint32_t u = 0; u < kVs; ++u)
+      if (key[u] < top && seen(key[u])) vmax = fmaxf(vmax, vs[u]);
   }
-  wmin = __builtin_amdgcn_readfirstlane(wmin);
-  wlow = __builtin_amdgcn_readfirstlane(wlow);
-  __syncthreads();
-  const uint32_t top = s_top, low = WIN ? s_low : 0;
-  if (top > alloc || top == 0) return;  // validated on entry; stay in bounds
-  // Step i walks the keys of block i (i < sblocks: the sinks) or i + skip.
-  uint32_t sblocks = WIN ? (min(sink, top) + kPfKeys - 1) / kPfKeys : 0;
-  if (low / kPfKeys <= sblocks) sblocks = low / kPfKeys;  // contiguous
-  const uint32_t skip = low / kPfKeys - sblocks;
-  const uint32_t nblocks = (top + kPfKeys - 1) / kPfKeys - skip;
-  auto block_key = [&](uint32_t b) { return (b < sblocks ? b : b + skip) * kPfKeys; };
-  auto seen = [&](uint32_t key) { return !WIN || key >= low || key < sink; };
 
   // The split of q: the row maximum over the four lanes holding the row.
   float qmax = 0.f;
@@ -294,15 +325,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     }
 
   // The largest v_scale of the visible keys sets the p' scale 2^f.
-  float vmax = 0.f;
-  if constexpr (WIN) {
-    for (uint32_t i = t; i < nblocks * kPfKeys; i += kPfThreads) {
-      const uint32_t k = block_key(i / kPfKeys) + i % kPfKeys;
-      if (k < top && seen(k)) vmax = fmaxf(vmax, Vs[head_base + k]);
-    }
-  } else {
-    for (uint32_t k = t; k < top; k += kPfThreads) vmax = fmaxf(vmax, Vs[head_base + k]);
-  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
   if (lane == 0) s_vmax[wave] = vmax;
@@ -315,36 +337,34 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
   const float pup = ldexpf(1.f, 15 - fe), pdown = ldexpf(1.f, fe - 15);
   const float ks_mul = score_scale * 1.4426950408889634f;  // scores in base 2
 
-  // Block loads of the group: thread tg takes key tg / 4, bytes [16 (tg %
-  // 4), +16) of its K and V rows (keys past top read the last visible slot;
-  // they are masked).
-  const uint32_t lkey = tg >> 2, lpart = tg & 3;
-  uint4 kreg, vreg;
-  float ksr = 0.f, vsr = 0.f;
-  auto load_block = [&](uint32_t b) {
-    const uint32_t kb0 = block_key(b);
-    const uint32_t key = min(kb0 + lkey, top - 1);
-    const size_t row = head_base + key;
-    kreg = *reinterpret_cast<const uint4*>(Kc + row * kHeadDim + 16 * lpart);
-    vreg = *reinterpret_cast<const uint4*>(Vc + row * kHeadDim + 16 * lpart);
-    if (tg < kPfKeys) {
-      const uint32_t skey = min(kb0 + tg, top - 1);
-      const float kk = Ks[head_base + skey], vv = Vs[head_base + skey];
-      ksr = seen(skey) ? kk : 0.f;
-      vsr = seen(skey) ? vv : 0.f;
-    }
-  };
   auto store_block = [&](PfBuf& B) {
-    const half8 k0 = nd::codes_to_half(u32x2{kreg.x, kreg.y});
-    const half8 k1 = nd::codes_to_half(u32x2{kreg.z, kreg.w});
-    *reinterpret_cast<half8*>(&B.k[lkey * kKStrideH + 16 * lpart]) = k0;
-    *reinterpret_cast<half8*>(&B.k[lkey * kKStrideH + 16 * lpart + 8]) = k1;
-    const half8 v0 = nd::codes_to_half(u32x2{vreg.x, vreg.y});
-    const half8 v1 = nd::codes_to_half(u32x2{vreg.z, vreg.w});
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      B.vt[(16 * lpart + e) * kVtStrideH + lkey] = v0[e];
-      B.vt[(16 * lpart + 8 + e) * kVtStrideH + lkey] = v1[e];
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<half8*>(&B.k[(lkey + i) * kKStrideH + 8 * lpart]) =
+          nd::codes_to_half(u32x2{kreg[i].x, kreg[i].y});
+    // V: the four keys' bytes of each dimension together (a 4 x 4 byte
+    // transpose of each word), then to halves: dimensions 8 lpart + 4 w + 2 p
+    // and + 1 a call.  Keys 4 g .. of a 32-key step are lane block g % 4 of
+    // 16-key tile g / 4: position 8 (g % 4) + 4 (g / 4).
+    const uint32_t g = (tg >> 3) & 7;
+    _Float16* vt = &B.vt[8 * lpart * kVtStrideH + 32 * (tg >> 6) + 8 * (g & 3) + 4 * (g >> 2)];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const uint32_t a = w ? vreg[0].y : vreg[0].x, b = w ? vreg[1].y : vreg[1].x,
+                     c = w ? vreg[2].y : vreg[2].x, d = w ? vreg[3].y : vreg[3].x;
+      const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u),   // a0 b0 a1 b1
+                     cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u),
+                     ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u),   // a2 b2 a3 b3
+                     cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint32_t ab = p ? ab1 : ab0, cd = p ? cd1 : cd0;
+        const half8 h = nd::codes_to_half(u32x2{__builtin_amdgcn_perm(cd, ab, 0x05040100u),
+                                                __builtin_amdgcn_perm(cd, ab, 0x07060302u)});
+        _Float16* at = vt + (4 * w + 2 * p) * kVtStrideH;
+        *reinterpret_cast<half4*>(at) = half4{h[0], h[1], h[2], h[3]};
+        *reinterpret_cast<half4*>(at + kVtStrideH) = half4{h[4], h[5], h[6], h[7]};
+      }
     }
     if (tg < kPfKeys) {
       B.ks[tg] = ksr * ks_mul;
@@ -352,18 +372,15 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     }
   };
   const uint32_t steps = (nblocks + kPfGroups - 1) / kPfGroups;  // the groups step together
-  if (grp < nblocks) {
-    load_block(grp);
-    store_block(s_buf[grp][0]);
-  }
+  if (grp < nblocks) store_block(s_buf[grp]);
   nd::lds_barrier();
 
-  float m = -INFINITY, l = 0.f;  // m in base 2
+  float m = -INFINITY, l = 0.f;  // m in base 2, over qup
   float4v o[4] = {};
   for (uint32_t i = 0; i < steps; ++i) {
     const uint32_t b = kPfGroups * i + grp;
     const bool has = b < nblocks, has_next = b + kPfGroups < nblocks;
-    PfBuf& B = s_buf[grp][i & 1];
+    PfBuf& B = s_buf[grp];
     if (has_next) load_block(b + kPfGroups);
     if (has) {
       const uint32_t k0 = block_key(b);
@@ -388,22 +405,31 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
         const float ksv[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          float v = (sc[j][c] * ksv[c]) * qup;
-          if (masked) {
-            const uint32_t key = k0 + 16 * j + 4 * kb + c;
-            v = (q_ok && key <= pos && (!WIN || key >= row_low || key < sink)) ? v : -INFINITY;
-          }
-          sc[j][c] = v;
-          bmax = fmaxf(bmax, v);
+          sc[j][c] *= ksv[c];
         }
       }
+      if (masked) {
+        asm volatile("; masked block");  // a branch: not selects on every block
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const uint32_t key = k0 + 16 * j + 4 * kb + c;
+            const bool in = q_ok && key <= pos && (!WIN || key >= row_low || key < sink);
+            sc[j][c] = in ? sc[j][c] : -INFINITY;
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) bmax = fmaxf(bmax, sc[j][c]);
       bmax = nd::max_xor<16>(bmax);
       bmax = nd::max_xor<32>(bmax);
       const float m_new = fmaxf(m, bmax);
       // While no key has been visible m_new is -inf: subtract 0 instead, so
       // that masked scores give exp2(-inf) = 0 and alpha = 1.
       const float m_sub = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m - m_sub);
+      const float alpha = __builtin_amdgcn_exp2f((m - m_sub) * qup), mq = -m_sub * qup;
       m = m_new;
       l *= alpha;
 #pragma unroll
@@ -412,7 +438,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const float e = __builtin_amdgcn_exp2f(sc[j][c] - m_sub);
+          const float e = __builtin_amdgcn_exp2f(fmaf(sc[j][c], qup, mq));
           sc[j][c] = e;
           l += e;
         }
@@ -439,27 +465,29 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
         }
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-          const _Float16* vt = &B.vt[(16 * d + r16) * kVtStrideH + 32 * s2 + 4 * kb];
-          const half4 lo4 = *reinterpret_cast<const half4*>(vt);
-          const half4 hi4 = *reinterpret_cast<const half4*>(vt + 16);
-          const half8 va8 = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+          const half8 va8 =
+              *reinterpret_cast<const half8*>(&B.vt[(16 * d + r16) * kVtStrideH + 32 * s2 + 8 * kb]);
           o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ph, o[d], 0, 0, 0);
           o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, pl, o[d], 0, 0, 0);
         }
       }
     }
-    if (has_next) store_block(s_buf[grp][(i + 1) & 1]);
+    if (i + 1 == steps) break;
+    nd::lds_barrier();  // the group's waves are done with the block
+    if (has_next) store_block(s_buf[grp]);
     nd::lds_barrier();
   }
+  nd::lds_barrier();
+  m *= qup;
   // l over the row's four lanes; o[d][c] is dim 16 d + 4 kb + c of the row.
   l = nd::sum_xor<16>(l);
   l = nd::sum_xor<32>(l);
   // Merge: groups 1.. leave (m, l, o) in LDS (the key buffers are free),
   // group 0 combines them with its own and stores the row.
-  float* xm = reinterpret_cast<float*>(&s_buf[0][0]);  // [group - 1][wq][18][64]
-  static_assert((kPfGroups - 1) * 4 * 18 * 64 * 4 <= sizeof(PfBuf) * kPfGroups * 2, "merge fits");
+  float* xm = reinterpret_cast<float*>(&s_buf[0]);  // [group - 1][wq][18][64]
+  static_assert((kPfGroups - 1) * 2 * 18 * 64 * 4 <= sizeof(PfBuf) * kPfGroups, "merge fits");
   if (grp > 0) {
-    float* dst = xm + ((grp - 1) * 4 + wq) * 18 * 64 + lane;
+    float* dst = xm + ((grp - 1) * 2 + wq) * 18 * 64 + lane;
     dst[0] = m;
     dst[64] = l;
 #pragma unroll
@@ -476,7 +504,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     float mt = m;
 #pragma unroll
     for (uint32_t g = 1; g < kPfGroups; ++g) {
-      const float* src = xm + ((g - 1) * 4 + wq) * 18 * 64 + lane;
+      const float* src = xm + ((g - 1) * 2 + wq) * 18 * 64 + lane;
       mg[g] = src[0];
       lg[g] = src[64];
       mt = fmaxf(mt, mg[g]);
@@ -489,7 +517,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_attention_mfma_kernel(
     for (int d = 0; d < 4; ++d) o[d] *= ag[0];
 #pragma unroll
     for (uint32_t g = 1; g < kPfGroups; ++g) {
-      const float* src = xm + ((g - 1) * 4 + wq) * 18 * 64 + lane;
+      const float* src = xm + ((g - 1) * 2 + wq) * 18 * 64 + lane;
       l += lg[g] * ag[g];
 #pragma unroll
       for (int d = 0; d < 4; ++d)
@@ -531,11 +559,11 @@ hipError_t launch_attention(const AttnLaunch& a, hipStream_t s) {
       const uint32_t window = nd_kv_linear(a.kv) ? a.kv->window : 0u;
       hipLaunchKernelGGL(window ? prefill_attention_mfma_kernel<true>
                                 : prefill_attention_mfma_kernel<false>,
-                         dim3((a.batch + kPfRows - 1) / kPfRows, a.seq_kv_heads * REP),
+                         dim3((a.batch + kPfRows - 1) / kPfRows * a.seq_kv_heads * REP),
                          dim3(kPfThreads), 0, s, reinterpret_cast<const int8_t*>(a.kv->k),
                          reinterpret_cast<const int8_t*>(a.kv->v), a.kv->ks, a.kv->vs, a.q, a.out,
                          a.gate, a.gate_ld, a.layer, a.kv->kv_heads, a.kv->alloc, a.kv->sink,
-                         window, a.positions, a.batch, a.seq_kv_heads * REP, (uint32_t)REP,
+                         window, a.first_position, a.batch, a.seq_kv_heads * REP, (uint32_t)REP,
                          0.125f);
       return hipGetLastError();
     }
@@ -748,8 +776,9 @@ hipError_t nd_launch_attention(const nd_kv* kv, uint32_t layer, uint32_t positio
 
 // Batched form: query row z reads cache heads [z * kv_stride_z, +seq_kv_heads)
 // (kv_stride_z = seq_kv_heads for a batch of sequences, 0 for the positions of
-// one prefill) with queries q[z][seq_kv_heads * rep][64] at position
-// positions[z] (device memory), at most max_position.
+// one prefill, consecutive and ending at max_position) with queries
+// q[z][seq_kv_heads * rep][64] at position positions[z] (device memory), at
+// most max_position.
 hipError_t nd_launch_attention_batch(const nd_kv* kv, uint32_t layer, const uint32_t* positions,
                                      uint32_t batch, uint32_t seq_kv_heads, uint32_t kv_stride_z,
                                      uint32_t rep, uint32_t max_position, const float* q,
@@ -772,6 +801,7 @@ hipError_t nd_launch_attention_batch(const nd_kv* kv, uint32_t layer, const uint
   a.rep = rep;
   a.batch = batch;
   a.max_count = nv.count;
+  a.first_position = max_position + 1 - batch;
   // Positions sit in their own slots while no window is outgrown (they then
   // also see all of [0, position]) and in a linear cache.
   a.qblock = kv_stride_z == 0 && (nd_kv_linear(kv) || max_position < kv->window) &&
