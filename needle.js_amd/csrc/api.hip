@@ -471,6 +471,18 @@ nd_status nd_stream_read_d(nd_ctx* ctx, const void* src, uint64_t bytes, uint32_
   return ND_OK;
 }
 
+// Small host-buffer products go through pinned memory: x by a copy kernel
+// (which the product then reads from HBM, as many times as it has workgroups),
+// y written there by the product itself.  The runtime's copies of pageable
+// buffers cost more than the product: 512 x 512, 30 us a call with them.
+static constexpr size_t kDirectBytes = 32 << 10;
+
+static __global__ __launch_bounds__(256) void copy_in_kernel(const float* __restrict__ src,
+                                                             float* __restrict__ dst, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 nd_status nd_matvec(nd_ctx* ctx, const nd_mat* m, const float* x, uint32_t batch,
                     uint32_t row_start, uint32_t row_count, float* y) {
   if (!ctx) return nd_fail(nullptr, ND_ERR_BACKEND, "context is NULL");
@@ -484,6 +496,21 @@ nd_status nd_matvec(nd_ctx* ctx, const nd_mat* m, const float* x, uint32_t batch
   if (st != ND_OK) return st;
   float* dx = reinterpret_cast<float*>(ctx->stage);
   float* dy = reinterpret_cast<float*>(reinterpret_cast<char*>(ctx->stage) + align256(xb));
+  if (xb <= kDirectBytes && yb <= kDirectBytes) {
+    st = ensure_host_stage(ctx, 2 * kDirectBytes);
+    if (st != ND_OK) return st;
+    float* hx = reinterpret_cast<float*>(ctx->host_stage);
+    float* hy = hx + kDirectBytes / sizeof(float);
+    std::memcpy(hx, x, xb);
+    const uint32_t n = batch * m->k;
+    hipLaunchKernelGGL(copy_in_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, hx, dx, n);
+    ND_HIP(ctx, hipGetLastError());
+    ND_HIP(ctx, launch_matvec_any(ctx, m, dx, batch, row_start, row_count, hy, row_count,
+                                  ctx->stream, ctx->mv_split));
+    ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(y, hy, yb);
+    return ND_OK;
+  }
   ND_HIP(ctx, hipMemcpyAsync(dx, x, xb, hipMemcpyHostToDevice, ctx->stream));
   ND_HIP(ctx, launch_matvec_any(ctx, m, dx, batch, row_start, row_count, dy, row_count,
                                 ctx->stream, ctx->mv_split));
