@@ -621,6 +621,11 @@ nd_status nd_matmul_d(nd_ctx* ctx, const nd_mat* m, const float* x, uint32_t row
   if (st != ND_OK) return st;
   if (rows == 0) return ND_OK;
   if (!x || !y) return nd_fail(ctx, ND_ERR_INVALID, "x or y is NULL");
+  if (nd_gemm_rows_fits(m, x, m->k, false, rows)) {
+    ND_HIP(ctx, nd_launch_gemm_rows(m, x, m->k, nullptr, y, m->n, rows, accumulate ? 1 : 0,
+                                    nd_pick_stream(ctx, stream)));
+    return ND_OK;
+  }
   const size_t dbytes = align256((size_t)3 * rows * m->k);
   st = ensure_mm_scratch(ctx, dbytes + align256((size_t)rows * 4));
   if (st != ND_OK) return st;

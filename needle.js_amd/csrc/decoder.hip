@@ -797,20 +797,22 @@ static nd_status enqueue_prefill(nd_ctx* ctx, nd_prefill* p, nd_kv* kv, hipStrea
                      p->position0, M, p->rope);
   ND_HIP(ctx, hipGetLastError());
   ND_HIP(ctx, mark(O));
-  // Wo and Wdown as whole-row products that digitize their own inputs and
-  // leave the next norm's digits, or as digitize and GEMM launches.
-  const bool wide_o = nd_gemm_wide_fits(dec->wo[0], D, D, M);
-  const bool wide_d = nd_gemm_wide_fits(dec->wdown[0], F, D, M);
-  bool have = false;  // p->digits hold the next product's rows
-  for (uint32_t l = 0; l < dec->layers; ++l) {
-    const float* attn_norm = dec->norms + dec->attn_off + (size_t)l * D;
-    const float* ffn_norm = dec->norms + dec->ffn_off + (size_t)l * D;
-    if (!have) {
-      ND_HIP(ctx, nd_launch_digitize(p->x, D, attn_norm, nullptr, p->digits, p->fm, M, D, s));
-      ND_HIP(ctx, mark(O));
+  // y (op)= w (norm(x)): one launch for prompt-sized M, else digitize and GEMM.
+  auto product = [&](const nd_mat* w, const float* x, uint32_t ldx, const float* norm, float* y,
+                     uint32_t ldy, int epilogue) -> hipError_t {
+    hipError_t e;
+    if (nd_gemm_rows_fits(w, x, ldx, norm != nullptr, M)) {
+      e = nd_launch_gemm_rows(w, x, ldx, norm, y, ldy, M, epilogue, s);
+    } else {
+      e = nd_launch_digitize(x, ldx, norm, nullptr, p->digits, p->fm, M, w->k, s);
+      if (e == hipSuccess) e = mark(O);
+      if (e == hipSuccess) e = nd_launch_gemm(w, p->digits, p->fm, y, ldy, M, epilogue, s);
     }
-    ND_HIP(ctx, nd_launch_gemm(&dec->wqkv[l], p->digits, p->fm, p->qkv, qkv_rows, M, 0, s));
-    ND_HIP(ctx, mark(G));
+    return e == hipSuccess ? mark(G) : e;
+  };
+  for (uint32_t l = 0; l < dec->layers; ++l) {
+    ND_HIP(ctx, product(&dec->wqkv[l], p->x, D, dec->norms + dec->attn_off + (size_t)l * D, p->qkv,
+                        qkv_rows, 0));
     const nd::RopeStore rs{dec->heads, dec->kv_heads, dec->norms + dec->q_off + (size_t)l * kHd,
                            dec->norms + dec->k_off + (size_t)l * kHd, p->rope, nullptr, p->q,
                            (int8_t*)kv->k, (int8_t*)kv->v, kv->ks, kv->vs, l, kv->kv_heads,
@@ -822,29 +824,9 @@ static nd_status enqueue_prefill(nd_ctx* ctx, nd_prefill* p, nd_kv* kv, hipStrea
     ND_HIP(ctx, nd_launch_attention_batch(kv, l, p->positions, M, dec->kv_heads, 0u, rep, last,
                                           p->q, p->o, p->partials, p->counters, s));
     ND_HIP(ctx, mark(A));
-    if (wide_o) {
-      ND_HIP(ctx, nd_launch_gemm_wide(dec->wo[l], p->o, D, p->x, D, M, ffn_norm, p->digits, p->fm, s));
-      ND_HIP(ctx, mark(G));
-    } else {
-      ND_HIP(ctx, nd_launch_digitize(p->o, D, nullptr, nullptr, p->digits, p->fm, M, D, s));
-      ND_HIP(ctx, mark(O));
-      ND_HIP(ctx, nd_launch_gemm(dec->wo[l], p->digits, p->fm, p->x, D, M, 1, s));
-      ND_HIP(ctx, mark(G));
-      ND_HIP(ctx, nd_launch_digitize(p->x, D, ffn_norm, nullptr, p->digits, p->fm, M, D, s));
-      ND_HIP(ctx, mark(O));
-    }
-    ND_HIP(ctx, nd_launch_gemm(dec->wup[l], p->digits, p->fm, p->h, F, M, 2, s));
-    ND_HIP(ctx, mark(G));
-    have = wide_d && l + 1 < dec->layers;
-    if (wide_d) {
-      ND_HIP(ctx, nd_launch_gemm_wide(dec->wdown[l], p->h, F, p->x, D, M,
-                                      have ? attn_norm + D : nullptr, p->digits, p->fm, s));
-    } else {
-      ND_HIP(ctx, nd_launch_digitize(p->h, F, nullptr, nullptr, p->digits, p->fm, M, F, s));
-      ND_HIP(ctx, mark(O));
-      ND_HIP(ctx, nd_launch_gemm(dec->wdown[l], p->digits, p->fm, p->x, D, M, 1, s));
-    }
-    ND_HIP(ctx, mark(G));
+    ND_HIP(ctx, product(dec->wo[l], p->o, D, nullptr, p->x, D, 1));
+    ND_HIP(ctx, product(dec->wup[l], p->x, D, dec->norms + dec->ffn_off + (size_t)l * D, p->h, F, 2));
+    ND_HIP(ctx, product(dec->wdown[l], p->h, F, nullptr, p->x, D, 1));
   }
   ND_HIP(ctx, nd_launch_digitize(p->x + (size_t)(M - 1) * D, D, dec->norms + dec->final_off,
                                  nullptr, p->digits, p->fm, 1, D, s));

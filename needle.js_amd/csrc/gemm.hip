@@ -33,7 +33,6 @@ constexpr int kKChunk = 256;             // k per LDS stage
 constexpr int kLdsRow = kKChunk + 16;    // padded row stride (bank spread)
 constexpr int kMaxSplit = 8;             // k slices of a split launch
 constexpr uint32_t kMaxNormK = 1024;     // rows the fused norm reads whole
-constexpr uint32_t kWideMinRows = 256;
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.f + __expf(-v)); }
 
@@ -642,175 +641,53 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
   }
 }
 
-// Prompt-sized product with the activations stationary (M >= 1024, K in
-// {128, 256, 512}, N % 128 == 0): workgroup (column group g, row tile m) copies the
-// three digit planes of its 64 rows over all of K into LDS once (LDS DMA,
-// global_load_lds_dwordx4, no registers) and then streams 128-column weight
-// strips through them.  Every weight strip is read by the M / 64 row tiles
-// and every digit plane by the N / NG column groups, against one read of
-// each per 32 x 64 tile pair for the tiled kernel above -- about a quarter
-// of its L2 traffic at 2048 x 2048 x 512.  8 waves in two groups take the
-// strips alternately (group h: strips h, h + 2, ...), so one group's weight
-// loads overlap the other's products; wave w % 4 of a group takes the
-// strip's columns [32 (w % 4), +32).  The integer sums are exact and the
-// epilogue is the tiled kernel's, so both give the same bits.
+// Prompt-sized product on fp32 rows: the workgroup digitizes its 16 rows
+// itself (with NORM after the zero-centred RMS norm of math.ts:16-32, as
+// digitize_rows_kernel: the same bits) into LDS and multiplies them by 128 NS
+// columns over all of K.  A digitize launch of its own cost 5.6 us at 2048 rows
+// of 512, a write and three reads of the digits; redone by each column group
+// it is a wave's work on two rows while the first weights arrive.
 //
-// LDS layout: 16-byte units, plane j, row r, unit slot p (U = K / 16 per
-// row); slot p holds k-unit p ^ (4 (r % 4) & (U - 1)).  A wave's 16-byte
-// read takes k-units 4 q + (l / 16) of rows 16 b + l % 16: the rows' four
-// residues mod 4 move those units to four different 64-byte bank groups, so
-// the 64 lanes fall on all 16 groups of the 64 banks, four lanes each (the
-// minimum of four passes for 1 KiB).
-constexpr uint32_t kAsRows = 64, kAsMaxK = 512, kAsStrip = 128;
-__device__ __forceinline__ uint32_t as_slot(uint32_t u, uint32_t r, uint32_t U) {
-  return u ^ ((4u * (r & 3u)) & (U - 1u));
-}
-template <int EPI>
-__global__ __launch_bounds__(512) void gemm_i8_astat_kernel(
-    const int8_t* __restrict__ W, const float* __restrict__ sw, const int8_t* __restrict__ D,
-    const float* __restrict__ fm, float* __restrict__ Y, uint32_t M, uint32_t N, uint32_t K,
-    uint32_t ldy, uint32_t group_cols) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[3 * kAsRows * kAsMaxK];
-  const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const uint32_t half = wave >> 2, wq = wave & 3;
-  const uint32_t m0 = blockIdx.y * kAsRows;
-  const uint32_t c0 = blockIdx.x * group_cols;
-  const uint32_t U = K / 16;  // units per row
-  const size_t plane = (size_t)M * K;
-
-  // Stage the tile: 3 * 64 * U units in chunks of 64 (one wave load each).
-  {
-    const uint32_t chunks = 3 * kAsRows * U / 64;
-    for (uint32_t c = wave; c < chunks; c += 8) {
-      const uint32_t L = c * 64 + lane;
-      const uint32_t j = L / (kAsRows * U), r = (L / U) % kAsRows, pslot = L % U;
-      const uint32_t u = as_slot(pslot, r, U);  // the slot map is its own inverse
-      const uint32_t row = m0 + r < M ? m0 + r : M - 1;  // rows past M feed only rows past M
-      __builtin_amdgcn_global_load_lds(D + j * plane + (size_t)row * K + u * 16,
-                                       (__attribute__((address_space(3))) void*)(lds + c * 1024),
-                                       16, 0, 0);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-
-  const uint32_t lrow = lane & 15, lk = lane >> 4;
-  const uint32_t steps = K / 64;
-  for (uint32_t s0 = half * kAsStrip; s0 < group_cols; s0 += 2 * kAsStrip) {
-    const uint32_t nb = c0 + s0 + 32 * wq;  // this wave's 32 columns
-    // The strip's weights for both 16-column tiles and every k step.
-    v4i wa[kAsMaxK / 64][2];
-#pragma unroll
-    for (int q = 0; q < (int)(kAsMaxK / 64); ++q)
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const uint32_t n = nb + 16 * a;
-        const uint32_t qs = (uint32_t)q < steps ? q : 0;
-        wa[q][a] = *reinterpret_cast<const v4i*>(
-            W + ((size_t)((n < N ? n : N - 1) / 16) * steps + qs) * 1024 + lane * 16);
-      }
-    v4i acc[2][4][3];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) acc[a][b][j] = v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < (int)(kAsMaxK / 64); ++q) {
-      if ((uint32_t)q >= steps) break;
-      const uint32_t u = 4 * q + lk;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t r = 16 * b + lrow;
-        const uint32_t pslot = as_slot(u, r, U);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const v4i db = *reinterpret_cast<const v4i*>(
-              &lds[((j * kAsRows + r) * U + pslot) * 16]);
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-            acc[a][b][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[q][a], db, acc[a][b][j], 0, 0, 0);
-        }
-      }
-    }
-    // Output (a, b, i) of lane l: n = nb + 16 a + 4 (l / 16) + i, m = m0 + 16 b + l % 16.
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const uint32_t n = nb + 16 * a + 4 * lk;
-      if (n >= N) continue;
-      const float4 s4 = *reinterpret_cast<const float4*>(sw + n);
-      const float swv[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t m = m0 + 16 * b + lrow;
-        if (m >= M) continue;
-        const float f = fm[m];
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float c = (float)acc[a][b][0][i] + 256.f * (float)acc[a][b][1][i] +
-                          65536.f * (float)acc[a][b][2][i];
-          v[i] = swv[i] * (f * c);
-        }
-        float4* dst = reinterpret_cast<float4*>(Y + (size_t)m * ldy + n);
-        if constexpr (EPI == 1) {
-          const float4 o = *dst;
-          *dst = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
-        } else if constexpr (EPI == 2) {
-          *dst = make_float4(silu_f(v[0]), silu_f(v[1]), silu_f(v[2]), silu_f(v[3]));
-        } else {
-          *dst = make_float4(v[0], v[1], v[2], v[3]);
-        }
-      }
-    }
-  }
-}
-
-// Prompt-sized product whose outputs are whole rows (N = 128 NS <= 512
-// columns, M rows in tiles of 16): y += A W^T on fp32 rows A that the
-// workgroup digitizes itself, and, with DOUT, the zero-centred RMS norm of the
-// new rows and their digits for the next product.  A tile of all N columns
-// digitizes each row once and has the row's sum of squares and maximum at
-// hand, so the two digitize launches around such a product (5.4 and 7.7 us at
-// 2048 rows of 512 and 2048) and the fp32 round trips between them go away;
-// 16 rows keep 2048 of them on 128 workgroups.
-//
-// 8 waves: wave w digitizes rows 2 w and 2 w + 1 (digitize_rows_kernel's
-// split, the same bits) into LDS, then takes columns [16 NS w, +16 NS) over
-// all of K: weights straight from memory to registers, 256 k ahead of the
-// products (the first 256 k and the addends issued at entry), digits from LDS
-// (row stride K + 16 bytes: 16 rows cover all banks).  Lane l holds columns 4
-// (l / 16) + i of row l % 16.  Bound by the weights entering each CU: N K
-// bytes a workgroup.
-template <int NS, int KMAX, bool DOUT>
-__global__ __launch_bounds__(512) void gemm_i8_wide_kernel(
+// 8 waves: wave w digitizes rows 2 w and 2 w + 1, then takes columns [16 NS w,
+// +16 NS) of the group: weights straight from memory to registers (operand
+// order, one KiB a load), 256 k ahead of the products, the first issued behind
+// the rows; digits from LDS (row stride K + 16 bytes: 16 rows cover all
+// banks).  A = digits, B = weights: lane l holds column l % 16 of rows 4 (l /
+// 16) + i, so a store writes whole 64-byte runs.  Bound by the weights entering
+// each CU (128 NS K bytes a workgroup), the digitizing and the stores of y.
+// 2000 rows x (2048 x 512): 15.6 us, against 20.6 for the digitize launch and a
+// product with 64 rows of digits stationary in LDS.
+template <int NS, int KMAX, int EPI, bool NORM>
+__global__ __launch_bounds__(512) void gemm_i8_rows_kernel(
     const int8_t* __restrict__ W, const float* __restrict__ sw, const float* __restrict__ X,
-    uint32_t ldx, float* __restrict__ Y, uint32_t ldy, uint32_t M, uint32_t K,
-    const float* __restrict__ norm, int8_t* __restrict__ Dout, float* __restrict__ fm_out) {
-  constexpr uint32_t N = 128 * NS;
-  constexpr int VEC = KMAX / 256;
+    uint32_t ldx, const float* __restrict__ norm, float* __restrict__ Y, uint32_t ldy, uint32_t M,
+    uint32_t N, uint32_t K) {
+  constexpr int VEC = KMAX / 256, kR = 2, kRows = 16;
   constexpr int kQ = 4;  // 64-wide k steps per weight stage
-  constexpr uint32_t kOutLd = N + 16;
-  __shared__ __attribute__((aligned(16))) int8_t lds[3 * 16 * (KMAX + 16)];
-  static_assert(sizeof(lds) >= 3 * 16 * kOutLd, "the output digits fit");
-  __shared__ float s_fm[16], s_red[2][8][16];
+  __shared__ __attribute__((aligned(16))) int8_t lds[3 * kRows * (KMAX + 16)];
+  __shared__ __attribute__((aligned(16))) float s_fm[kRows];
   const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const uint32_t lrow = lane & 15, lk = lane >> 4;
-  const uint32_t m0 = blockIdx.x * 16, n0 = wave * 16 * NS;
-  const uint32_t kld = K + 16;
-  const uint32_t steps = K / 64;
+  const uint32_t m0 = blockIdx.x * kRows, n0 = (blockIdx.y * 8 + wave) * 16 * NS;
+  const uint32_t kld = K + 16, steps = K / 64, units = K / 4;
 
-  // The rows, then the first weights, then the addends.
-  float4 v[2][VEC];
+  float4 v[kR][VEC];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const uint32_t m = m0 + 2 * wave + r;
+  for (int r = 0; r < kR; ++r) {
+    const uint32_t m = m0 + kR * wave + r;
     const float4* x = reinterpret_cast<const float4*>(X + (size_t)(m < M ? m : M - 1) * ldx);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       const uint32_t u = lane + 64 * i;
-      v[r][i] = x[u < K / 4 ? u : 0];
+      v[r][i] = x[u < units ? u : 0];
+    }
+  }
+  float4 nw[NORM ? VEC : 1];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const uint32_t u = lane + 64 * i;
+      nw[i] = reinterpret_cast<const float4*>(norm)[u < units ? u : 0];
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -821,28 +698,53 @@ __global__ __launch_bounds__(512) void gemm_i8_wide_kernel(
 #pragma unroll
       for (int a = 0; a < NS; ++a) {
         const uint32_t qs = q0 + q < steps ? q0 + q : 0;  // clamped, never used
-        wn[q][a] = *reinterpret_cast<const v4i*>(W + ((size_t)(n0 / 16 + a) * steps + qs) * 1024 +
-                                                 lane * 16);
+        const uint32_t tile = (n0 < N ? n0 / 16 : 0) + a;
+        wn[q][a] = *reinterpret_cast<const v4i*>(
+            W + ((size_t)(tile < (N + 15) / 16 ? tile : 0) * steps + qs) * 1024 + lane * 16);
       }
   };
   load_w(0);
-  const uint32_t mo = m0 + lrow;
-  const float* yrow = Y + (size_t)(mo < M ? mo : M - 1) * ldy + n0 + 4 * lk;
-  float4 add[NS];
+  float swv[NS];
 #pragma unroll
-  for (int a = 0; a < NS; ++a) add[a] = *reinterpret_cast<const float4*>(yrow + 16 * a);
+  for (int a = 0; a < NS; ++a) swv[a] = sw[min(n0 + 16 * a + lrow, N - 1)];
+  // Epilogue 1's addends, with the operands.
+  float add[EPI == 1 ? NS : 1][4];
+  if constexpr (EPI == 1) {
+#pragma unroll
+    for (int a = 0; a < NS; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        add[a][i] = Y[(size_t)min(m0 + 4 * lk + i, M - 1) * ldy + min(n0 + 16 * a + lrow, N - 1)];
+  }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const uint32_t lr = 2 * wave + r;
+  for (int r = 0; r < kR; ++r) {
+    const uint32_t lr = kR * wave + r;
     const bool live = m0 + lr < M;  // rows past M multiply as zeros
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      if (!live || lane + 64 * i >= units) v[r][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (NORM) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        ss = fmaf(v[r][i].x, v[r][i].x, fmaf(v[r][i].y, v[r][i].y, fmaf(v[r][i].z, v[r][i].z,
+             fmaf(v[r][i].w, v[r][i].w, ss))));
+      ss = nd::wave_sum(ss);
+      const float inv = 1.f / sqrtf(ss / (float)K + 1e-6f);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        v[r][i].x = (1.f + nw[i].x) * v[r][i].x * inv;
+        v[r][i].y = (1.f + nw[i].y) * v[r][i].y * inv;
+        v[r][i].z = (1.f + nw[i].z) * v[r][i].z * inv;
+        v[r][i].w = (1.f + nw[i].w) * v[r][i].w * inv;
+      }
+    }
     float amax = 0.f;
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      if (!live || lane + 64 * i >= K / 4) v[r][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < VEC; ++i)
       amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[r][i].x), fabsf(v[r][i].y)),
                                fmaxf(fabsf(v[r][i].z), fabsf(v[r][i].w))));
-    }
     amax = nd::row_max(amax);
     amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
                  fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
@@ -855,14 +757,14 @@ __global__ __launch_bounds__(512) void gemm_i8_wide_kernel(
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       const uint32_t u = lane + 64 * i;
-      if (u >= K / 4) continue;
+      if (u >= units) continue;
       uint32_t d0, d1, d2;
       digit_words(digit_bias(v[r][i].x, up), digit_bias(v[r][i].y, up),
                   digit_bias(v[r][i].z, up), digit_bias(v[r][i].w, up), d0, d1, d2);
       int8_t* at = lds + lr * kld + 4 * u;
       *reinterpret_cast<uint32_t*>(at) = d0;
-      *reinterpret_cast<uint32_t*>(at + 16 * kld) = d1;
-      *reinterpret_cast<uint32_t*>(at + 32 * kld) = d2;
+      *reinterpret_cast<uint32_t*>(at + kRows * kld) = d1;
+      *reinterpret_cast<uint32_t*>(at + 2 * kRows * kld) = d2;
     }
     if (lane == 0) s_fm[lr] = ldexpf(1.f, e - 21);
   }
@@ -882,89 +784,35 @@ __global__ __launch_bounds__(512) void gemm_i8_wide_kernel(
     if (q0 + kQ < steps) load_w(q0 + kQ);
 #pragma unroll
     for (int q = 0; q < kQ; ++q) {
-      const uint32_t qs = q0 + q;
-      if (qs >= steps) break;
+      if (q0 + q >= steps) break;
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const v4i db = *reinterpret_cast<const v4i*>(lds + (j * 16 + lrow) * kld + qs * 64 + lk * 16);
+        const v4i da = *reinterpret_cast<const v4i*>(lds + (j * 16 + lrow) * kld + (q0 + q) * 64 +
+                                                     lk * 16);
 #pragma unroll
         for (int a = 0; a < NS; ++a)
-          acc[a][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[q][a], db, acc[a][j], 0, 0, 0);
+          acc[a][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(da, w[q][a], acc[a][j], 0, 0, 0);
       }
     }
   }
-
-  const float f = s_fm[lrow];
-  float y[NS][4];
-  float ss = 0.f;
+  const float4 f4 = *reinterpret_cast<const float4*>(&s_fm[4 * lk]);
+  const float f[4] = {f4.x, f4.y, f4.z, f4.w};
 #pragma unroll
-  for (int a = 0; a < NS; ++a) {
-    const float4 s4 = *reinterpret_cast<const float4*>(sw + n0 + 16 * a + 4 * lk);
-    const float swv[4] = {s4.x, s4.y, s4.z, s4.w};
-    const float o[4] = {add[a].x, add[a].y, add[a].z, add[a].w};
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t m = m0 + 4 * lk + i;
+    if (m >= M) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int a = 0; a < NS; ++a) {
+      const uint32_t n = n0 + 16 * a + lrow;
+      if (n >= N) continue;
       const float c = (float)acc[a][0][i] + 256.f * (float)acc[a][1][i] +
                       65536.f * (float)acc[a][2][i];
-      y[a][i] = o[i] + swv[i] * (f * c);
-      ss = fmaf(y[a][i], y[a][i], ss);
+      const float y = swv[a] * (f[i] * c);
+      float* dst = Y + (size_t)m * ldy + n;
+      if constexpr (EPI == 1) *dst = add[a][i] + y;
+      else if constexpr (EPI == 2) *dst = silu_f(y);
+      else *dst = y;
     }
-    if (mo < M)
-      *reinterpret_cast<float4*>(Y + (size_t)mo * ldy + n0 + 16 * a + 4 * lk) =
-          make_float4(y[a][0], y[a][1], y[a][2], y[a][3]);
-  }
-  if constexpr (!DOUT) return;
-  // The new rows' norm and digits: row sums and maxima over the lanes of a
-  // row and the waves.
-  ss = nd::sum_xor<16>(ss);
-  ss = nd::sum_xor<32>(ss);
-  if (lk == 0) s_red[0][wave][lrow] = ss;
-  nd::lds_barrier();  // also: every wave is done with the digits
-  float total = 0.f;
-#pragma unroll
-  for (int w = 0; w < 8; ++w) total += s_red[0][w][lrow];
-  const float inv = 1.f / sqrtf(total / (float)N + 1e-6f);
-  float amax = 0.f;
-#pragma unroll
-  for (int a = 0; a < NS; ++a) {
-    const float4 w4 = *reinterpret_cast<const float4*>(norm + n0 + 16 * a + 4 * lk);
-    const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      y[a][i] = (1.f + wv[i]) * y[a][i] * inv;
-      amax = fmaxf(amax, fabsf(y[a][i]));
-    }
-  }
-  amax = nd::max_xor<16>(amax);
-  amax = nd::max_xor<32>(amax);
-  if (lk == 0) s_red[1][wave][lrow] = amax;
-  nd::lds_barrier();
-#pragma unroll
-  for (int w = 0; w < 8; ++w) amax = fmaxf(amax, s_red[1][w][lrow]);
-  int e = 0;
-  if (amax > 0.f) {
-    frexpf(amax, &e);
-    e -= 1;
-  }
-  const float up = ldexpf(1.f, 21 - e);
-#pragma unroll
-  for (int a = 0; a < NS; ++a) {
-    uint32_t d0, d1, d2;
-    digit_words(digit_bias(y[a][0], up), digit_bias(y[a][1], up), digit_bias(y[a][2], up),
-                digit_bias(y[a][3], up), d0, d1, d2);
-    int8_t* at = lds + lrow * kOutLd + n0 + 16 * a + 4 * lk;
-    *reinterpret_cast<uint32_t*>(at) = d0;
-    *reinterpret_cast<uint32_t*>(at + 16 * kOutLd) = d1;
-    *reinterpret_cast<uint32_t*>(at + 32 * kOutLd) = d2;
-  }
-  if (wave == 0 && lk == 0 && mo < M) fm_out[mo] = ldexpf(1.f, e - 21);
-  nd::lds_barrier();
-  const size_t plane = (size_t)M * N;
-  for (uint32_t u = t; u < 3 * 16 * N / 16; u += 512) {
-    const uint32_t j = u / N, r = u % N / (N / 16), c = u % (N / 16) * 16;
-    if (m0 + r < M)
-      *reinterpret_cast<uint4*>(Dout + j * plane + (size_t)(m0 + r) * N + c) =
-          *reinterpret_cast<const uint4*>(lds + (j * 16 + r) * kOutLd + c);
   }
 }
 
@@ -1060,29 +908,6 @@ hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm
                           uint32_t ldy, uint32_t M, int epilogue, hipStream_t s,
                           const nd_gemm_split* split) {
   if (M == 0) return hipSuccess;
-  // Prompt-sized M with K <= 512: the activation tile stays in LDS.  Column
-  // groups of whole 128-column strips, as many as give the row tiles 256
-  // workgroups (or fewer when N has fewer strips).
-  if (M >= 1024 && (w->k == 128 || w->k == 256 || w->k == 512) && w->n % kAsStrip == 0 &&
-      ldy % 4 == 0 &&
-      (reinterpret_cast<uintptr_t>(y) & 15) == 0 && (reinterpret_cast<uintptr_t>(digits) & 15) == 0) {
-    const uint32_t mt = (M + kAsRows - 1) / kAsRows, strips = w->n / kAsStrip;
-    uint32_t groups = (256 + mt - 1) / mt;
-    if (groups > strips) groups = strips;
-    while (strips % groups) --groups;
-    const uint32_t gc = (strips / groups) * kAsStrip;
-    const dim3 grid(groups, mt);
-    if (epilogue == 0)
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<0>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
-                         fm, y, M, w->n, w->k, ldy, gc);
-    else if (epilogue == 1)
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<1>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
-                         fm, y, M, w->n, w->k, ldy, gc);
-    else
-      hipLaunchKernelGGL(gemm_i8_astat_kernel<2>, grid, dim3(512), 0, s, w->wt, w->scales, digits,
-                         fm, y, M, w->n, w->k, ldy, gc);
-    return hipGetLastError();
-  }
   // A wide product at decode M (the 32768-row lm head of a 64-row batch)
   // takes 32 x 128 tiles: 16.1 us with digitize, against 21.2 for 16 x 128
   // tiles with the k prefetch.
@@ -1116,37 +941,56 @@ hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm
   return hipGetLastError();
 }
 
-// The whole-row product above: true when it takes (w, M).  Prompts through 8
-// layers of 512 x 512 and 512 x 2048, whole-row against tiled products with
-// their digitize launches: 496 and 513 us at 256 rows, 557 and 598 at 512, 695
-// and 838 at 1024.
-bool nd_gemm_wide_fits(const nd_mat* w, uint32_t ldx, uint32_t ldy, uint32_t M) {
-  return M >= kWideMinRows && (w->n == 128 || w->n == 256 || w->n == 512) && w->k % 64 == 0 &&
-         w->k <= 2048 && ldx % 4 == 0 && ldy % 4 == 0;
+// Column groups of the row product: 512 columns, 256 or 128 for a narrow
+// matrix, and 256 when the 512-column workgroups (one to a CU by their
+// registers) would leave their last round less than 3/5 full -- two of the
+// smaller share a CU (1500 rows x (2048 x 512), 1.5 rounds: 11.9 us against
+// 14.0; 2000 rows, nearly two rounds: 16.8 against 15.6).
+static uint32_t rows_subtiles(const nd_mat* w, uint32_t M) {
+  const uint32_t ns = w->n > 256 ? 4 : w->n > 128 ? 2 : 1;
+  const uint64_t wgs = (uint64_t)((M + 15) / 16) * ((w->n + 511) / 512);
+  const uint32_t last = (uint32_t)(wgs % 256);
+  return ns == 4 && w->k <= 512 && wgs > 256 && last > 0 && last <= 154 ? 2 : ns;
 }
 
-hipError_t nd_launch_gemm_wide(const nd_mat* w, const float* x, uint32_t ldx, float* y,
-                               uint32_t ldy, uint32_t M, const float* norm, int8_t* digits,
-                               float* fm, hipStream_t s) {
-  if (!nd_gemm_wide_fits(w, ldx, ldy, M) ||
-      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
-        reinterpret_cast<uintptr_t>(norm) | reinterpret_cast<uintptr_t>(digits)) & 15))
+// Whether the row product takes (w, M): from 128 rows (the tiled kernels with
+// their digitize launch: 6.8 against 7.3 us at 512 x 512, 7.1 against 7.4 at
+// 2048 x 512; at 64 rows they are level), and past k = 512, where a workgroup's
+// weights take longer than the tiled kernels' split ones, from 36 workgroups
+// (512 x 2048: 15.3 against 15.2 us at 400 rows, 15.6 against 19.9 at 700).
+bool nd_gemm_rows_fits(const nd_mat* w, const float* x, uint32_t ldx, bool norm, uint32_t M) {
+  const uint32_t cols = 128 * rows_subtiles(w, M);
+  return M >= 128 && w->k % 64 == 0 && w->k <= 2048 && (!norm || w->k <= 512) &&
+         (w->k <= 512 || (uint64_t)((M + 15) / 16) * ((w->n + cols - 1) / cols) >= 36) &&
+         ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+}
+
+hipError_t nd_launch_gemm_rows(const nd_mat* w, const float* x, uint32_t ldx, const float* norm,
+                               float* y, uint32_t ldy, uint32_t M, int epilogue, hipStream_t s) {
+  if (!nd_gemm_rows_fits(w, x, ldx, norm != nullptr, M) ||
+      (reinterpret_cast<uintptr_t>(norm) & 15) || epilogue < 0 || epilogue > 2)
     return hipErrorInvalidValue;
-  using Fn = void (*)(const int8_t*, const float*, const float*, uint32_t, float*, uint32_t,
-                      uint32_t, uint32_t, const float*, int8_t*, float*);
-  auto pick = [&](auto ns, auto k) -> Fn {
-    constexpr int NS = decltype(ns)::value, KM = decltype(k)::value;
-    return norm ? &gemm_i8_wide_kernel<NS, KM, true> : &gemm_i8_wide_kernel<NS, KM, false>;
+  using Fn = void (*)(const int8_t*, const float*, const float*, uint32_t, const float*, float*,
+                      uint32_t, uint32_t, uint32_t, uint32_t);
+  auto pick = [&](auto ns, auto km, auto nm) -> Fn {
+    constexpr int NS = decltype(ns)::value, KM = decltype(km)::value;
+    constexpr bool NM = decltype(nm)::value;
+    return epilogue == 0   ? &gemm_i8_rows_kernel<NS, KM, 0, NM>
+           : epilogue == 1 ? &gemm_i8_rows_kernel<NS, KM, 1, NM>
+                           : &gemm_i8_rows_kernel<NS, KM, 2, NM>;
   };
+  using std::integral_constant;
   auto pick_k = [&](auto ns) -> Fn {
-    return w->k <= 512 ? pick(ns, std::integral_constant<int, 512>())
-                       : pick(ns, std::integral_constant<int, 2048>());
+    const integral_constant<int, 512> k512;
+    if (w->k > 512) return pick(ns, integral_constant<int, 2048>(), std::false_type());
+    return norm ? pick(ns, k512, std::true_type()) : pick(ns, k512, std::false_type());
   };
-  const Fn f = w->n == 512   ? pick_k(std::integral_constant<int, 4>())
-               : w->n == 256 ? pick_k(std::integral_constant<int, 2>())
-                             : pick_k(std::integral_constant<int, 1>());
-  hipLaunchKernelGGL(f, dim3((M + 15) / 16), dim3(512), 0, s, w->wt, w->scales, x, ldx, y, ldy, M,
-                     w->k, norm, digits, fm);
+  const uint32_t ns = rows_subtiles(w, M);
+  const Fn f = ns == 4   ? pick_k(integral_constant<int, 4>())
+               : ns == 2 ? pick_k(integral_constant<int, 2>())
+                         : pick_k(integral_constant<int, 1>());
+  hipLaunchKernelGGL(f, dim3((M + 15) / 16, (w->n + 128 * ns - 1) / (128 * ns)), dim3(512), 0, s,
+                     w->wt, w->scales, x, ldx, norm, y, ldy, M, w->n, w->k);
   return hipGetLastError();
 }
 

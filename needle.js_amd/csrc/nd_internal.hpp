@@ -266,14 +266,12 @@ struct nd_gemm_split {
 hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm, float* y,
                           uint32_t ldy, uint32_t M, int epilogue, hipStream_t s,
                           const nd_gemm_split* split = nullptr);
-// y += x W^T for prompt-sized M and n of 128, 256 or 512 (nd_gemm_wide_fits) on
-// fp32 rows x [M][ldx], digitized inside the launch; with `norm`, the new rows
-// of y are then RMS-normalized (math.ts:16-32) and their digits and factors
-// written for the next nd_launch_gemm.  Pointers 16-byte aligned.
-bool nd_gemm_wide_fits(const nd_mat* w, uint32_t ldx, uint32_t ldy, uint32_t M);
-hipError_t nd_launch_gemm_wide(const nd_mat* w, const float* x, uint32_t ldx, float* y,
-                               uint32_t ldy, uint32_t M, const float* norm, int8_t* digits,
-                               float* fm, hipStream_t s);
+// The same product for prompt-sized M (nd_gemm_rows_fits) on fp32 rows x
+// [M][ldx], 16-byte aligned, optionally RMS-normalized with `norm`
+// (math.ts:16-32; k <= 512), digitized inside the launch.
+bool nd_gemm_rows_fits(const nd_mat* w, const float* x, uint32_t ldx, bool norm, uint32_t M);
+hipError_t nd_launch_gemm_rows(const nd_mat* w, const float* x, uint32_t ldx, const float* norm,
+                               float* y, uint32_t ldy, uint32_t M, int epilogue, hipStream_t s);
 // The same product on fp32 rows x [M][ldx] (optionally RMS-normalized with
 // `norm`, math.ts:16-32), digitized per 256-wide chunk inside the launch;
 // only for the shapes nd_gemm_f32_fits accepts.  Epilogue 3 (the q/k/v

@@ -3399,6 +3399,8 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
                      uint32_t y_ld) -> hipError_t {
     if (w->bits)
       return nd_launch_cq_matvec(w, x, M, x_ld, nullptr, 0, w->n, y, y_ld, s);
+    if (nd_gemm_rows_fits(w, x, x_ld, false, M))
+      return nd_launch_gemm_rows(w, x, x_ld, nullptr, y, y_ld, M, 0, s);
     hipError_t r = nd_launch_digitize(x, x_ld, nullptr, nullptr, n->pf_digits, n->pf_fm, M, k, s);
     if (r != hipSuccess) return r;
     return nd_launch_gemm(w, n->pf_digits, n->pf_fm, y, y_ld, M, 0, s);

@@ -28,7 +28,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import (assert_close, assert_codes_or_boundary_flips, read_device,
+from helpers import (DeviceArray, assert_close, assert_codes_or_boundary_flips, read_device,
                      storekv_of_projections)
 from needle_hip import Int8Matrix, NeedleError, synth
 from needle_hip import lib as L
@@ -274,3 +274,35 @@ def test_batch_rejects_bad_state(hip):
         b.step(16)
     b.free()
     dec.free()
+
+
+@pytest.mark.parametrize("n,k,rows", [(96, 256, 130), (300, 128, 128), (512, 512, 129),
+                                      (2048, 512, 200), (2500, 512, 1000), (700, 2048, 640),
+                                      (512, 1024, 600)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_matmul_prompt_rows(hip, n, k, rows, accumulate):
+    """Prompt-sized products (digitized inside the launch): column groups of
+    128, 256 and 512 with ragged ends, a row past a tile, the narrower groups
+    of a launch past 256 workgroups, K past 512, rows of zeros and of very
+    different magnitudes; plain and added into y.  Bound per output: the
+    digits keep 2^-22 of the row's largest element, the factors and the sum
+    round a few times: 2^-21 of the row maximum times the absolute weights
+    plus 2^-21 of the values."""
+    say("matmul prompt rows", n, k, rows, accumulate)
+    w, s = synth.int8_matrix(71, f"rows{n}x{k}", n, k, k)
+    x = synth.Stream(71, f"rx{k}r{rows}").normal((rows, k))
+    x[0] = 0.0
+    x[1] *= np.float32(1e-30)
+    x[2] *= np.float32(1e25)
+    y0 = synth.Stream(72, f"ry{n}r{rows}").normal((rows, n))
+    dx, dy = DeviceArray(x), DeviceArray(y0)
+    hip._check(hip.lib.nd_matmul_d(hip.ctx, hip.upload(Int8Matrix(w, s, k)), dx.ptr, rows, dy.ptr,
+                                   accumulate, None))
+    hip._check(hip.lib.nd_sync(hip.ctx))
+    got = dy.read().astype(np.float64)
+    full = w.astype(np.float64) * s.astype(np.float64)
+    y = x.astype(np.float64) @ full.T
+    want = y + y0 if accumulate else y
+    top = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
+    bound = 2.0 ** -21 * (top * np.abs(full).sum(axis=1)[None] + np.abs(y) + np.abs(want)) + 1e-40
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
