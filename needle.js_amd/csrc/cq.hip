@@ -341,6 +341,221 @@ __global__ __launch_bounds__(kCqThreads) void cq_matvec_kernel(
   }
 }
 
+// One activation row times a large matrix (g >= 32, at most 64 units a row):
+// workgroups that stay for many rows, so that the rotation of x and a wider
+// lookup table are set up once.  The table holds a copy of every entry for each
+// lane of an LDS access phase (32 copies of 8-byte entries, 16 of 16-byte
+// ones), laid out so that a lane's copy lies in banks of its own: a lookup of 64
+// random codes takes the minimum of cycles, where the one shared copy of
+// cq_matvec_kernel, whose LDS reads bound it, took about three times that.
+// Bound by the weights: 32768 x 2048 in 4 bits (38 MB) 8.2 us a call against 10.5,
+// of which about 4.3 are the launch's.
+// The workgroup rotates x together (4 values a thread, the stages of
+// rotate_unit in the same order: the same bits) while the first rows arrive.
+// Wave w of the launch takes 64 / tpr rows at a time (tpr threads a row, one
+// 32-code unit each), kStreamRows such passes in flight, strided over the rows
+// by the launch's waves.  The same fp32 dots per unit, times the norm, as
+// cq_matvec_kernel; row sums by a butterfly over the row's lanes.
+constexpr uint32_t kStreamThreads = 512;
+constexpr int kStreamRows = 4;
+static_assert(kStreamThreads * 4 == 64 * 32, "a thread holds 4 of a row's values");
+
+template <int M>
+__device__ __forceinline__ void cross_lane_stage4(float (&v)[4]) {
+  const bool right = (__lane_id() & M) != 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float other = nd::lane_xor<M>(v[i]);
+    v[i] = right ? other - v[i] : v[i] + other;
+  }
+}
+
+template <int UB>
+__global__ __launch_bounds__(kStreamThreads) void cq_stream_kernel(
+    const uint8_t* __restrict__ packed, const uint16_t* __restrict__ norms, Codebook cb,
+    const float* __restrict__ x, bool vec, float* __restrict__ y, uint32_t k, uint32_t units,
+    uint32_t groups, uint32_t g_log2, uint32_t row_bytes, uint32_t row_start, uint32_t row_count,
+    uint32_t tpr_log2, float out_scale) {
+  constexpr int kPB = UB / 4, kE = lookup_codes(UB), kLB = kPB * kE;
+  constexpr uint32_t kEntries = 1u << kLB, kCopies = 64 / kE;  // an entry's copies: 64 words
+  constexpr int kLookups = 32 / kE, kW = UB / 4;
+  // x: 32 floats of a unit at 36 words, so that 16-byte reads of consecutive
+  // units cover all banks.
+  __shared__ __align__(16) float tab[kEntries * 64];
+  __shared__ __align__(16) float sx[64 * 36];
+  const uint32_t t = threadIdx.x, lane = t & 63;
+  const uint32_t tpr = 1u << tpr_log2, rpw = 64u >> tpr_log2;  // rows a wave pass
+  const uint32_t sub = lane >> tpr_log2, u = lane & (tpr - 1);
+  const bool active = u < units;
+  const uint32_t uc = active ? u : 0;
+  const uint32_t wave = blockIdx.x * (kStreamThreads / 64) + __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t step = gridDim.x * (kStreamThreads / 64) * rpw;  // rows between a wave's passes
+  float v[4];
+  if (vec) {
+    const float4 f = *reinterpret_cast<const float4*>(x + (4 * t < k ? 4 * t : 0));
+    v[0] = f.x;
+    v[1] = f.y;
+    v[2] = f.z;
+    v[3] = f.w;
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) v[i] = x[4 * t + i < k ? 4 * t + i : 0];
+  }
+  uint32_t raw[kStreamRows][kW], nb[kStreamRows];
+  const uint32_t own = wave * rpw;
+  // A pass beyond the rows re-reads the wave's first rows: loads without a
+  // branch, and no line that many waves would ask for at once.
+  auto load = [&](uint32_t first) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < kStreamRows; ++r) {
+      const uint32_t at = first + r * step < row_count ? first + r * step : own;
+      const uint32_t row = at + sub;
+      const size_t rr = row_start + (row < row_count ? row : row_count - 1);
+      const uint32_t* src =
+          reinterpret_cast<const uint32_t*>(packed + rr * row_bytes + (size_t)uc * UB);
+#pragma unroll
+      for (int w = 0; w < kW; ++w) raw[r][w] = __builtin_nontemporal_load(src + w);
+      nb[r] = norms[rr * groups + ((uc * 32) >> g_log2)];
+    }
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  load(own);
+  __builtin_amdgcn_sched_barrier(0);
+  // Copy c of entry e at words (e kCopies + c) kE.  Thread t writes the copies of
+  // entry t, in an order turned by its lane: a write's lanes lie in different banks.
+  for (uint32_t e = t; e < kEntries; e += kStreamThreads) {
+    float c[kE];
+#pragma unroll
+    for (int i = 0; i < kE; ++i)
+      c[i] = pick_code<(1 << kPB)>(cb, (e >> (i * kPB)) & ((1u << kPB) - 1));
+#pragma unroll
+    for (uint32_t q = 0; q < 16; ++q) {
+      float4* at = reinterpret_cast<float4*>(tab + e * 64) + ((q + e) & 15);
+      if constexpr (kE == 4)
+        *at = make_float4(c[0], c[1], c[2], c[3]);
+      else
+        *at = make_float4(c[0], c[1], c[0], c[1]);
+    }
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) v[i] = 4 * t + i < k ? v[i] : 0.f;
+  {
+    const float a = v[0] + v[1], b = v[0] - v[1], c = v[2] + v[3], d = v[2] - v[3];
+    v[0] = a + c;
+    v[1] = b + d;
+    v[2] = a - c;
+    v[3] = b - d;
+  }
+  cross_lane_stage4<1>(v);
+  cross_lane_stage4<2>(v);
+  cross_lane_stage4<4>(v);
+  if (g_log2 > 5) cross_lane_stage4<8>(v);
+  if (g_log2 > 6) cross_lane_stage4<16>(v);
+  if (g_log2 > 7) cross_lane_stage4<32>(v);
+  auto word_of = [](uint32_t c) { return (c >> 5) * 36 + (c & 31); };
+  *reinterpret_cast<float4*>(sx + word_of(4 * t)) = make_float4(v[0], v[1], v[2], v[3]);
+  nd::lds_barrier();
+  if (g_log2 > 8) {  // strides 256, 512, 1024: thread t's values are 256 apart
+    if (t < 256) {
+      float z[8];
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) z[i] = sx[word_of(t + 256 * i)];
+#pragma unroll
+      for (uint32_t st = 1; st < 8; st <<= 1) {
+        if ((256u * st) >> g_log2) continue;
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+          if ((i & st) == 0) {
+            const float a = z[i], b = z[i + st];
+            z[i] = a + b;
+            z[i + st] = a - b;
+          }
+        }
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) sx[word_of(t + 256 * i)] = z[i];
+    }
+    nd::lds_barrier();
+  }
+  float xv[32];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float4 f = *reinterpret_cast<const float4*>(sx + u * 36 + 4 * q);
+    xv[4 * q] = f.x;
+    xv[4 * q + 1] = f.y;
+    xv[4 * q + 2] = f.z;
+    xv[4 * q + 3] = f.w;
+  }
+
+  const char* mine = reinterpret_cast<const char*>(tab) + (lane % kCopies) * (kE * 4);
+  auto row_of = [&](const uint32_t (&codes)[kW], uint32_t norm, uint32_t row)
+      __attribute__((always_inline)) {
+    float d[kE];
+#pragma unroll
+    for (int e = 0; e < kE; ++e) d[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < kLookups; ++i) {
+      const int bit = kLB * i, w = bit >> 5, sh = bit & 31;
+      uint32_t b = codes[w] >> sh;
+      if constexpr (32 % kLB != 0) {
+        if (sh + kLB > 32) b |= codes[w + 1] << (32 - sh);
+      }
+      const char* at = mine + (b & (kEntries - 1u)) * 256u;
+      if constexpr (kE == 4) {
+        const float4 f = *reinterpret_cast<const float4*>(at);
+        d[0] = fmaf(f.x, xv[4 * i], d[0]);
+        d[1] = fmaf(f.y, xv[4 * i + 1], d[1]);
+        d[2] = fmaf(f.z, xv[4 * i + 2], d[2]);
+        d[3] = fmaf(f.w, xv[4 * i + 3], d[3]);
+      } else {
+        const float2 f = *reinterpret_cast<const float2*>(at);
+        d[0] = fmaf(f.x, xv[2 * i], d[0]);
+        d[1] = fmaf(f.y, xv[2 * i + 1], d[1]);
+      }
+    }
+    float dot = d[0] + d[1];
+    if constexpr (kE == 4) dot += d[2] + d[3];
+    float sum = active ? half_bits_to_float(norm) * dot : 0.f;
+    if (tpr > 32) sum = nd::sum_xor<32>(sum);
+    if (tpr > 16) sum = nd::sum_xor<16>(sum);
+    sum += nd::lane_xor<8>(sum);
+    sum += nd::lane_xor<4>(sum);
+    sum += nd::lane_xor<2>(sum);
+    sum += nd::lane_xor<1>(sum);
+    if (u == 0 && row < row_count) y[row] = sum * out_scale;
+  };
+  for (uint32_t first = own; first < row_count; first += kStreamRows * step) {
+    uint32_t cur[kStreamRows][kW], cn[kStreamRows];
+#pragma unroll
+    for (int r = 0; r < kStreamRows; ++r) {
+#pragma unroll
+      for (int w = 0; w < kW; ++w) cur[r][w] = raw[r][w];
+      cn[r] = nb[r];
+    }
+    if (first + kStreamRows * step < row_count) load(first + kStreamRows * step);
+    if (first + (kStreamRows - 1) * step < row_count) {
+#pragma unroll
+      for (int r = 0; r < kStreamRows; ++r) row_of(cur[r], cn[r], first + r * step + sub);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kStreamRows; ++r) {
+        if (first + r * step >= row_count) break;
+        row_of(cur[r], cn[r], first + r * step + sub);
+      }
+    }
+  }
+}
+
+using CqStreamFn = void (*)(const uint8_t*, const uint16_t*, Codebook, const float*, bool, float*,
+                            uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t,
+                            uint32_t, float);
+
+CqStreamFn pick_stream(const nd_mat* m) {
+  return m->bits == 4   ? &cq_stream_kernel<16>
+         : m->bits == 3 ? &cq_stream_kernel<12>
+                        : &cq_stream_kernel<8>;
+}
+
 Codebook codebook_of(const nd_mat* m) {
   Codebook c{};
   for (int i = 0; i < 16; ++i) c.v[i] = m->cb[i];
@@ -353,6 +568,8 @@ using CqFn = void (*)(const uint8_t*, const uint16_t*, Codebook, const float*, u
 
 constexpr int kRacc = 8;  // rows per thread: rpp * 8 <= 256 outputs per workgroup
 constexpr uint32_t kMaxRotateGroup = 2048;  // 64 lanes of 32 codes
+constexpr uint32_t kStreamBlocks = 512;     // two to a CU (64 KB of table each)
+constexpr uint64_t kStreamUnits = 131072;
 
 template <int UB, int RACC, bool ROTATE, bool VEC>
 CqFn pick_ng(uint32_t g) {
@@ -426,6 +643,24 @@ hipError_t nd_launch_cq_matvec(const nd_mat* m, const float* x, uint32_t batch, 
   uint32_t g_log2 = 0;
   while ((1u << g_log2) < m->g) ++g_log2;
   const uint32_t lanes_per_group = m->g > 32 ? m->g / 32 : 1;
+  // The streaming form from 131072 units (8192 x 512: level at 4.9 us, 4096 x
+  // 2048: 7.0 against 4.8, 32768 x 2048: 10.5 against 8.2 in 4 bits and 10.7
+  // against 8.1 in 2; below, 4096 x 512: 4.7 against 4.9), when the row's threads
+  // are at least two thirds in use or x needs scalar loads, which it makes once a
+  // workgroup (32768 x 300, 10 of 16: 5.1 against 5.3; 40001 x 777: 13.9 against
+  // 7.5).
+  uint32_t row_log2 = 4;  // its row sum spans at least 16 lanes
+  while ((1u << row_log2) < units) ++row_log2;
+  if (batch == 1 && m->g >= 32 && units > 8 && units <= 64 &&
+      (uint64_t)row_count * units >= kStreamUnits && (!vec || units * 3 >= 2u << row_log2)) {
+    const uint32_t rows_per_block = (kStreamThreads >> row_log2);
+    const uint32_t want = (row_count + rows_per_block - 1) / rows_per_block;
+    hipLaunchKernelGGL(pick_stream(m), dim3(want < kStreamBlocks ? want : kStreamBlocks),
+                       dim3(kStreamThreads), 0, s, m->packed, m->norms, codebook_of(m), x, vec, y,
+                       m->k, units, m->kpad >> g_log2, g_log2, m->row_bytes, row_start, row_count,
+                       row_log2, (float)(1.0 / std::sqrt((double)m->g)));
+    return hipGetLastError();
+  }
   if (m->g <= kMaxRotateGroup) {
     const CqFn f = vec ? pick<true, true>(m, racc) : pick<true, false>(m, racc);
     hipLaunchKernelGGL(f, dim3(blocks, batch), dim3(kCqThreads), 0, s, m->packed,

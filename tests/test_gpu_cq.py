@@ -245,3 +245,27 @@ def test_cq_many_rows(hip, bits, n, k, g, batch):
         want = rot @ w[lo:lo + count].T
         bound = 2.0 ** -18 * (spread @ np.abs(w[lo:lo + count]).T) + 1e-43
         assert np.all(np.abs(got - want) <= bound), (lo, np.max(np.abs(got - want) / bound))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+@pytest.mark.parametrize("n,k,g", [(13200, 290, 32), (5301, 777, 128), (4113, 1024, 1024),
+                                   (2803, 1501, 512), (2053, 2048, 2048), (16411, 512, 256),
+                                   (4111, 2045, 64)])
+def test_cq_one_row_of_a_large_matrix(hip, bits, n, k, g):
+    """Matrices large enough for the streaming form: 16, 32 and 64 threads a row
+    with and without idle ones, x of any alignment, groups up to the row, fewer
+    rows than a launch's waves and several passes of them.  Bound: the
+    rotation's at most 11 stages round the norm of x by 2^-24 each, the at most
+    53 products and additions of a row's sum by 2^-24 of |w| |x| each: 2^-18."""
+    say("cq one row", n, k, g, bits)
+    m = cq(11, n, k, g, bits)
+    x = np.random.default_rng(n + k).standard_normal(k).astype(np.float32)
+    top = 1.2240064 / np.sqrt(g) if bits == TERNARY else float(np.max(np.abs(BOOKS[bits])))
+    groups = -(-k // g)
+    norms = np.asarray(m.norms).view(np.float16).astype(np.float64).reshape(n, -1)[:, :groups]
+    size = top * np.sqrt(g) * np.linalg.norm(norms, axis=1) * np.linalg.norm(x.astype(np.float64))
+    want = np.asarray(ref_matvec(m, x), np.float64)
+    for lo, count in ((0, n), (1, n - 1), (3, n - 3)):
+        got = hip.matvec(m, x, MatrixRowRange(lo, count)).astype(np.float64)
+        worst = np.max(np.abs(got - want[lo:lo + count]) / size[lo:lo + count])
+        assert worst <= 2.0 ** -18, (lo, worst)
