@@ -30,11 +30,6 @@ __device__ __forceinline__ uint64_t sm64_at(uint64_t seed, uint64_t i) {
   return sm64_mix(seed + (i + 1) * 0x9E3779B97F4A7C15ull);
 }
 
-// Wave reductions on DPP and readlane (every lane gets the same value).
-__device__ __forceinline__ double wave_sum_d(double v) { return nd::wave_sum(v); }
-
-__device__ __forceinline__ float wave_absmax_js(float v) { return nd::wave_max_js(fabsf(v)); }
-
 // x[m][:] = f32(f32(W[tok][:] * s[tok]) * sqrt(d)), the row() gather and
 // embedding scale of runtime.ts:305-309, in float64 like the reference.
 __global__ void embed_kernel(const int8_t* __restrict__ W, const float* __restrict__ S,

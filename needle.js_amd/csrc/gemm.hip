@@ -831,17 +831,10 @@ using GemmFn = void (*)(const int8_t*, const float*, const int8_t*, const float*
                         uint32_t, uint32_t, uint32_t, uint32_t, float*, uint32_t*);
 
 template <int EPI>
-GemmFn pick(uint32_t ms, uint32_t ns, bool pf) {
-  if (ms == 4) {
-    if (pf) return ns == 2 ? &gemm_i8_digits_kernel<4, 2, EPI, true> : &gemm_i8_digits_kernel<4, 1, EPI, true>;
-    return ns == 2 ? &gemm_i8_digits_kernel<4, 2, EPI, false> : &gemm_i8_digits_kernel<4, 1, EPI, false>;
-  }
-  if (ms == 2) {
-    if (pf) return ns == 2 ? &gemm_i8_digits_kernel<2, 2, EPI, true> : &gemm_i8_digits_kernel<2, 1, EPI, true>;
-    return ns == 2 ? &gemm_i8_digits_kernel<2, 2, EPI, false> : &gemm_i8_digits_kernel<2, 1, EPI, false>;
-  }
-  if (pf) return ns == 2 ? &gemm_i8_digits_kernel<1, 2, EPI, true> : &gemm_i8_digits_kernel<1, 1, EPI, true>;
-  return ns == 2 ? &gemm_i8_digits_kernel<1, 2, EPI, false> : &gemm_i8_digits_kernel<1, 1, EPI, false>;
+GemmFn pick(uint32_t ms, uint32_t ns) {
+  return ms == 1   ? &gemm_i8_digits_kernel<1, 1, EPI, true>
+         : ns == 2 ? &gemm_i8_digits_kernel<2, 2, EPI, false>
+                   : &gemm_i8_digits_kernel<2, 1, EPI, false>;
 }
 
 }  // namespace
@@ -897,7 +890,8 @@ hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, f
 }
 
 // Tile choice: decode-sized M (<= 64) uses 16-row m tiles so that even
-// N = 512 spreads over 32+ workgroups; prefill-sized M uses 32 x 64 tiles
+// N = 512 spreads over 32+ workgroups; larger M (what the row product does not
+// take: too few rows, k past 2048, unaligned x) uses 32 x 64 tiles
 // (measured at M = 2048 with digitize: 24.2 / 45.3 / 15.7 / 27.9 us for N x K
 // = 1536 x 512, 4096 x 512, 512 x 512, 512 x 2048, against 38.9 / 65.3 /
 // 21.6 / 43.9 for 64 x 128 tiles and 30.6 / 58.9 / 16.3 / 33.3 for 16 x 64).
@@ -920,11 +914,9 @@ hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm
   if (((w->n + 64 * ns - 1) / (64 * ns)) * ((M + 16 * ms - 1) / (16 * ms)) < 256) ms = ns = 1;
   // The prefetch of the next k chunk pays on the 16-row tiles (split-k
   // decode shapes: 31.2 vs 33.3 us at 512 x 2048); the larger tiles run more
-  // workgroups per CU without it.
-  const bool pf = ms == 1;
+  // workgroups per CU without it (pick).
   const uint32_t tm = 16 * ms, tn = 64 * ns;
-  GemmFn f = epilogue == 0 ? pick<0>(ms, ns, pf) : epilogue == 1 ? pick<1>(ms, ns, pf)
-                                                 : pick<2>(ms, ns, pf);
+  GemmFn f = epilogue == 0 ? pick<0>(ms, ns) : epilogue == 1 ? pick<1>(ms, ns) : pick<2>(ms, ns);
   dim3 grid((w->n + tn - 1) / tn, (M + tm - 1) / tm, 1);
   const uint32_t tiles = grid.x * grid.y;
   if (split && ms == 1 && ns == 1 && w->k % kKChunk == 0 && tiles <= split->counter_count) {

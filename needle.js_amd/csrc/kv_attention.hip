@@ -83,7 +83,7 @@ __global__ __launch_bounds__(64) void kv_store_kernel(void* __restrict__ Kc, voi
 
 // The attention launches' kernel: attention_body with its workgroup
 // (chunk, KV head, row) taken from the grid.
-template <int REP, bool F32, bool QB = false, int KW = 4, int TILES = 0, bool XL = false,
+template <int REP, bool F32, int KW = 4, int TILES = 0, bool XL = false,
           bool STAMP = false>
 __global__ __launch_bounds__(64 * KW) void attention_kernel(
     const void* __restrict__ Kc, const void* __restrict__ Vc, const float* __restrict__ Ks,
@@ -93,11 +93,11 @@ __global__ __launch_bounds__(64 * KW) void attention_kernel(
     uint32_t kv_heads, uint32_t alloc, uint32_t sink, uint32_t window, Visible vis,
     const uint32_t* __restrict__ positions, uint32_t slot_space, uint32_t seq_kv_heads,
     uint32_t kv_stride_z, uint32_t chunk_positions, uint32_t max_chunks, float score_scale,
-    uint32_t qrows, uint32_t qgroup, uint64_t* __restrict__ stamps) {
-  attention_body<REP, F32, QB, KW, TILES, XL, STAMP, true>(
+    uint32_t rows, uint64_t* __restrict__ stamps) {
+  attention_body<REP, F32, KW, TILES, XL, STAMP, true>(
       0, 0, 0, Kc, Vc, Ks, Vs, Q, out, gate, gate_ld, part_acc, part_ml, counters, layer,
       kv_heads, alloc, sink, window, vis, positions, slot_space, seq_kv_heads, kv_stride_z,
-      chunk_positions, max_chunks, score_scale, qrows, qgroup, stamps);
+      chunk_positions, max_chunks, score_scale, rows, stamps);
 }
 
 // Positions per chunk: the whole visible range when the (row, kv head) pairs
@@ -545,12 +545,12 @@ hipError_t launch_attention(const AttnLaunch& a, hipStream_t s) {
     // workgroups, the instance the resident Needle 2 step's fused layer
     // launch runs (the same bits either way).
     if (a.slot_space && a.batch == 1 && a.max_count <= kGatedChunk && !a.stamps) {
-      hipLaunchKernelGGL((attention_kernel<2, false, false, 8, 1, false>),
+      hipLaunchKernelGGL((attention_kernel<2, false, 8, 1, false>),
                          dim3(1, a.seq_kv_heads, 1), dim3(64 * 8), 0, s, a.kv->k, a.kv->v,
                          a.kv->ks, a.kv->vs, a.q, a.out, a.gate, a.gate_ld, a.partials,
                          a.partials, a.counters, a.layer, a.kv->kv_heads, a.kv->alloc, a.kv->sink,
                          a.kv->window, a.vis, a.positions, a.slot_space, a.seq_kv_heads,
-                         a.kv_stride_z, kGatedChunk, 1u, 0.125f, a.batch, 1u, nullptr);
+                         a.kv_stride_z, kGatedChunk, 1u, 0.125f, a.batch, nullptr);
       return hipGetLastError();
     }
   }
@@ -597,32 +597,32 @@ hipError_t launch_attention(const AttnLaunch& a, hipStream_t s) {
       if (a.stamps) return hipErrorInvalidValue;  // no measurement form of the two-wave kernel
       float* pm2 = a.partials + (size_t)a.batch * hq * mc2 * kHeadDim;
       const uint32_t gpx = (a.batch * a.seq_kv_heads + 7) / 8;
-      hipLaunchKernelGGL((attention_kernel<REP, F32, false, 2, 1, true>), dim3(8 * gpx * mc2),
+      hipLaunchKernelGGL((attention_kernel<REP, F32, 2, 1, true>), dim3(8 * gpx * mc2),
                          dim3(64 * 2), 0, s, a.kv->k, a.kv->v, a.kv->ks, a.kv->vs, a.q, a.out,
                          a.gate, a.gate_ld, part_acc, pm2, a.counters, a.layer, a.kv->kv_heads,
                          a.kv->alloc, a.kv->sink, a.kv->window, a.vis, a.positions,
                          a.slot_space, a.seq_kv_heads, a.kv_stride_z, cp2, mc2, 0.125f, a.batch,
-                         1u, nullptr);
+                         nullptr);
       return hipGetLastError();
     }
   }
   if (xcd && max_chunks > 1) {
     // Rows split into chunks: the XCD-local merge (grid laid out per XCD,
     // see attention_kernel).
-    auto kernel = tiles == 1   ? attention_kernel<REP, F32, false, kWaves, 1, true>
-                  : tiles == 2 ? attention_kernel<REP, F32, false, kWaves, 2, true>
-                               : attention_kernel<REP, F32, false, kWaves, 0, true>;
+    auto kernel = tiles == 1   ? attention_kernel<REP, F32, kWaves, 1, true>
+                  : tiles == 2 ? attention_kernel<REP, F32, kWaves, 2, true>
+                               : attention_kernel<REP, F32, kWaves, 0, true>;
     const uint32_t gpx = (a.batch * a.seq_kv_heads + 7) / 8;
     if (a.stamps) {  // the measurement form of the same launch (one tile per wave)
       if (tiles != 1 || 8 * gpx * max_chunks > a.stamp_capacity) return hipErrorInvalidValue;
-      kernel = attention_kernel<REP, F32, false, kWaves, 1, true, true>;
+      kernel = attention_kernel<REP, F32, kWaves, 1, true, true>;
       *a.stamp_workgroups = 8 * gpx * max_chunks;
     }
     hipLaunchKernelGGL(kernel, dim3(8 * gpx * max_chunks), dim3(64 * kWaves), 0, s, a.kv->k,
                        a.kv->v, a.kv->ks, a.kv->vs, a.q, a.out, a.gate, a.gate_ld, part_acc,
                        part_ml, a.counters, a.layer, a.kv->kv_heads, a.kv->alloc, a.kv->sink,
                        a.kv->window, a.vis, a.positions, a.slot_space, a.seq_kv_heads,
-                       a.kv_stride_z, cp, max_chunks, 0.125f, a.batch, 1u, a.stamps);
+                       a.kv_stride_z, cp, max_chunks, 0.125f, a.batch, a.stamps);
     return hipGetLastError();
   }
   if (a.stamps) return hipErrorInvalidValue;
@@ -630,24 +630,24 @@ hipError_t launch_attention(const AttnLaunch& a, hipStream_t s) {
     if (max_chunks == 1 && tiles == 2) {
       // One 512-position chunk per (row, KV head): eight waves of one tile
       // each instead of four of two.
-      hipLaunchKernelGGL((attention_kernel<REP, F32, false, 8, 1>),
+      hipLaunchKernelGGL((attention_kernel<REP, F32, 8, 1>),
                          dim3(1, a.seq_kv_heads, a.batch), dim3(64 * 8), 0, s, a.kv->k, a.kv->v,
                          a.kv->ks, a.kv->vs, a.q, a.out, a.gate, a.gate_ld, part_acc, part_ml,
                          a.counters, a.layer, a.kv->kv_heads, a.kv->alloc, a.kv->sink,
                          a.kv->window, a.vis, a.positions, a.slot_space, a.seq_kv_heads,
-                         a.kv_stride_z, cp, max_chunks, 0.125f, a.batch, 1u, nullptr);
+                         a.kv_stride_z, cp, max_chunks, 0.125f, a.batch, nullptr);
       return hipGetLastError();
     }
   }
-  auto kernel = tiles == 1   ? attention_kernel<REP, F32, false, kWaves, 1>
-                : tiles == 2 ? attention_kernel<REP, F32, false, kWaves, 2>
-                             : attention_kernel<REP, F32, false, kWaves, 0>;
+  auto kernel = tiles == 1   ? attention_kernel<REP, F32, kWaves, 1>
+                : tiles == 2 ? attention_kernel<REP, F32, kWaves, 2>
+                             : attention_kernel<REP, F32, kWaves, 0>;
   hipLaunchKernelGGL(kernel, dim3(max_chunks, a.seq_kv_heads, a.batch),
                      dim3(64 * kWaves), 0, s, a.kv->k, a.kv->v, a.kv->ks, a.kv->vs, a.q, a.out,
                      a.gate, a.gate_ld, part_acc, part_ml, a.counters, a.layer, a.kv->kv_heads, a.kv->alloc,
                      a.kv->sink, a.kv->window, a.vis, a.positions, a.slot_space, a.seq_kv_heads,
                      a.kv_stride_z,
-                     cp, max_chunks, 0.125f, a.batch, 1u, nullptr);
+                     cp, max_chunks, 0.125f, a.batch, nullptr);
   return hipGetLastError();
 }
 

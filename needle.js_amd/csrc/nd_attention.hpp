@@ -144,12 +144,6 @@ __device__ __forceinline__ void unpack(const Tile<F32>& tl, int k, bool is_v, fl
 // Output gate of gated attention (model/runtime.ts:503-507): sigmoid(g).
 __device__ __forceinline__ float gate_factor(float g) { return 1.f / (1.f + __expf(-g)); }
 
-// QB (a prefill whose positions all see [0, position]: no sliding window,
-// or a window no position outgrows): the REP rows are REP / G consecutive
-// query positions x the G = qgroup query heads of KV head blockIdx.y --
-// row r is query z0 + r / G (z0 = (REP / G) blockIdx.z, rows at or past
-// `qrows` absent), head G blockIdx.y + r % G, with its own causal limit --
-// so every K/V tile is read once for all of them.
 // STAMP (measurement only): thread 0 reads the 100 MHz constant clock at
 // entry, after its wave's tiles, after the waves' combine, once the chunk's
 // partials are published, once its arrival is counted and (the last chunk)
@@ -175,7 +169,7 @@ struct NoHook {
 // the grid (the arguments of those names are ignored); otherwise from the
 // arguments (a caller that runs one workgroup per (chunk, KV head, row) of
 // its own).
-template <int REP, bool F32, bool QB = false, int KW = 4, int TILES = 0, bool XL = false,
+template <int REP, bool F32, int KW = 4, int TILES = 0, bool XL = false,
           bool STAMP = false, bool GRID = true, class Hook = NoHook>
 __device__ __forceinline__ void attention_body(
     uint32_t chunk_arg, uint32_t kvh_arg, uint32_t z_arg, const void* Kc, const void* Vc, const float* Ks,
@@ -186,9 +180,9 @@ __device__ __forceinline__ void attention_body(
     uint32_t alloc, uint32_t sink, uint32_t window, Visible vis,
     const uint32_t* positions, uint32_t slot_space, uint32_t seq_kv_heads,
     uint32_t kv_stride_z,
-    uint32_t chunk_positions, uint32_t max_chunks, float score_scale, uint32_t qrows,
-    uint32_t qgroup, uint64_t* stamps, const Hook& hook = Hook()) {
-  static_assert(!Hook::kActive || (TILES == 1 && !F32 && !QB),
+    uint32_t chunk_positions, uint32_t max_chunks, float score_scale, uint32_t rows,
+    uint64_t* stamps, const Hook& hook = Hook()) {
+  static_assert(!Hook::kActive || (TILES == 1 && !F32),
                 "the hook serves the one-tile int8 single-row form");
   uint64_t stamp[6] = {};
   if constexpr (STAMP) stamp[0] = wall_clock64();
@@ -213,7 +207,7 @@ __device__ __forceinline__ void attention_body(
     // L % 8, so pair g = 8 (L / 8 / max_chunks) + L % 8 (row g /
     // seq_kv_heads) and chunk L / 8 % max_chunks -- on each XCD a pair's
     // chunks are dispatched one after another.
-    const uint32_t pairs = qrows * seq_kv_heads;
+    const uint32_t pairs = rows * seq_kv_heads;
     const uint32_t L = blockIdx.x, sl = L >> 3, g = 8 * (sl / max_chunks) + (L & 7);
     chunk = sl % max_chunks;
     if (g >= pairs) return;
@@ -240,19 +234,7 @@ __device__ __forceinline__ void attention_body(
   // holds a visible position iff slot <= position or the ring is full
   // (position >= alloc).  Otherwise the visible range of the row's position.
   uint32_t spos = 0;
-  uint32_t rlim[QB ? REP : 1];  // QB: row r sees cache positions < rlim[r]
-  if constexpr (QB) {
-    uint32_t top = 0;
-#pragma unroll
-    for (int r = 0; r < REP; ++r) {
-      const uint32_t zr = z * (REP / qgroup) + r / qgroup;
-      const uint32_t pr = zr < qrows ? positions[zr] : 0;
-      if (zr < qrows && pr >= alloc) return;  // validated on entry; stay in bounds
-      rlim[r] = zr < qrows ? pr + 1 : 0;
-      top = max(top, rlim[r]);
-    }
-    vis = Visible{top, top, top};
-  } else if (slot_space) {
+  if (slot_space) {
     spos = positions[z];
   } else if (positions) {
     if (window == 0 && positions[z] >= alloc) return;  // validated on entry; stay in bounds
@@ -263,28 +245,15 @@ __device__ __forceinline__ void attention_body(
   if (chunk >= nchunks) return;
   const uint32_t c_begin = chunk * chunk_positions;
   const uint32_t c_end = min(vis.count, c_begin + chunk_positions);
-  if constexpr (!QB) {
-    Q += (size_t)z * hq * kHeadDim;
-    out += (size_t)z * hq * kHeadDim;
-  }
+  Q += (size_t)z * hq * kHeadDim;
+  out += (size_t)z * hq * kHeadDim;
   const size_t head_base = ((size_t)layer * kv_heads + kvh) * alloc;
-  // Query row h: head h of this KV head, or (QB) query z REP + h (absent
-  // rows read query 0; they are never stored).
-  auto qrow = [&](int h) -> size_t {
-    if constexpr (QB) {
-      const uint32_t zr = z * (REP / qgroup) + h / qgroup;
-      return ((size_t)(zr < qrows ? zr : 0) * seq_kv_heads * qgroup + kvh_local * qgroup +
-              h % qgroup) * kHeadDim;
-    } else {
-      return (size_t)(kvh_local * REP + h) * kHeadDim;
-    }
-  };
-
   float q[REP][16];
   auto load_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
-      const float4* qp = reinterpret_cast<const float4*>(Q + qrow(h) + quad * 16);
+      const float4* qp = reinterpret_cast<const float4*>(
+          Q + (size_t)(kvh_local * REP + h) * kHeadDim + quad * 16);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const float4 f = qp[c];
@@ -330,9 +299,7 @@ __device__ __forceinline__ void attention_body(
 #pragma unroll
         for (int i = 0; i < 16; ++i) d = fmaf(q[h][i], kc[i], d);
         d = nd::quad_sum(d);
-        bool ok = valid[k];
-        if constexpr (QB) ok = ok && t0 + trow + 16 * k < rlim[h];
-        p[h][k] = ok ? d * cur.ks[k] * score_scale : -INFINITY;
+        p[h][k] = valid[k] ? d * cur.ks[k] * score_scale : -INFINITY;
       }
     }
 #pragma unroll
@@ -354,9 +321,7 @@ __device__ __forceinline__ void attention_body(
       for (int i = 0; i < 16; ++i) acc[h][i] *= alpha;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        bool ok = valid[k];
-        if constexpr (QB) ok = ok && t0 + trow + 16 * k < rlim[h];
-        const float e = ok ? __expf(p[h][k] - m_new) : 0.f;
+        const float e = valid[k] ? __expf(p[h][k] - m_new) : 0.f;
         p[h][k] = e;
         l[h] += e;
       }
@@ -542,20 +507,6 @@ __device__ __forceinline__ void attention_body(
   const size_t row0 = (size_t)z * hq + (size_t)kvh_local * REP;
   float* const out_z = out;  // already offset to row z
   const float* const gate_z = gate ? gate + (size_t)z * gate_ld : nullptr;
-  if constexpr (QB) {  // one chunk (the launch guarantees it)
-    if (part == 0) {
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const uint32_t r = w_o[u] / kHeadDim, zr = z * (REP / qgroup) + r / qgroup;
-        if (zr >= qrows) continue;
-        const uint32_t oi = (kvh_local * qgroup + r % qgroup) * kHeadDim + w_o[u] % kHeadDim;
-        float v = w_a[u] / w_l[u];
-        if (gate) v *= gate_factor(gate[(size_t)zr * gate_ld + oi]);
-        out[(size_t)zr * seq_kv_heads * qgroup * kHeadDim + oi] = v;
-      }
-    }
-    return;
-  }
   if (nchunks == 1) {
     if (part == 0) {
 #pragma unroll

@@ -1584,11 +1584,11 @@ __device__ __forceinline__ void attention_role(const MixArgs& a, uint32_t ah,
   const AttArgs& g = a.att;
   const AttWaitT<STAMP> w{a.att_count + kAttStride * ah, a.status, &s_att_go, a.att_target,
                           a.spin, kv_slot(g.position[0], g.sink, g.window), marks};
-  nd::att::attention_body<2, false, false, kMixWg / 64, 1, false, false, false, AttWaitT<STAMP>>(
+  nd::att::attention_body<2, false, kMixWg / 64, 1, false, false, false, AttWaitT<STAMP>>(
       0u, ah, 0u, g.Kc, g.Vc, g.Ks, g.Vs, g.q, g.out, g.gate, 0u, nullptr, nullptr, nullptr,
       g.layer, g.kv_heads, g.alloc, g.sink, g.window,
       nd::att::Visible{g.alloc, g.alloc, g.alloc}, g.position, 1u, g.kv_heads, 0u,
-      nd::att::kGatedChunk, 1u, 0.125f, 1u, 1u, nullptr, w);
+      nd::att::kGatedChunk, 1u, 0.125f, 1u, nullptr, w);
   if constexpr (STAMP) {
     __builtin_amdgcn_s_waitcnt(0);
     if (threadIdx.x == 0) marks[4] = wall_clock64();
