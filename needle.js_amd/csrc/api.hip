@@ -621,7 +621,10 @@ nd_status nd_matmul_d(nd_ctx* ctx, const nd_mat* m, const float* x, uint32_t row
   if (st != ND_OK) return st;
   if (rows == 0) return ND_OK;
   if (!x || !y) return nd_fail(ctx, ND_ERR_INVALID, "x or y is NULL");
-  if (nd_gemm_rows_fits(m, x, m->k, false, rows)) {
+  // In one launch, unless y overlaps x: its workgroups read rows of x while
+  // others write y, where the digitize launch has read all of x first.
+  const bool apart = x + (size_t)rows * m->k <= y || y + (size_t)rows * m->n <= x;
+  if (apart && nd_gemm_rows_fits(m, x, m->k, false, rows)) {
     ND_HIP(ctx, nd_launch_gemm_rows(m, x, m->k, nullptr, y, m->n, rows, accumulate ? 1 : 0,
                                     nd_pick_stream(ctx, stream)));
     return ND_OK;

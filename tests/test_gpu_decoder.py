@@ -306,3 +306,22 @@ def test_matmul_prompt_rows(hip, n, k, rows, accumulate):
     top = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
     bound = 2.0 ** -21 * (top * np.abs(full).sum(axis=1)[None] + np.abs(y) + np.abs(want)) + 1e-40
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
+
+
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_matmul_into_its_input(hip, accumulate):
+    """y = x (n == k): every row of x is read before y is written, the same
+    results as into an array of its own, for every row on its own account."""
+    n, rows = 512, 300
+    say("matmul in place", accumulate)
+    w, s = synth.int8_matrix(73, "inplace", n, n, n)
+    x = synth.Stream(73, "inplace x").normal((rows, n))
+    mat = hip.upload(Int8Matrix(w, s, n))
+    dx, dy, dz = DeviceArray(x), DeviceArray(x), DeviceArray(x)
+    for _ in range(3):
+        hip._check(hip.lib.nd_matmul_d(hip.ctx, mat, dx.ptr, rows, dy.ptr, accumulate, None))
+        hip._check(hip.lib.nd_matmul_d(hip.ctx, mat, dz.ptr, rows, dz.ptr, accumulate, None))
+        hip._check(hip.lib.nd_sync(hip.ctx))
+        want = dy.read()
+        assert np.array_equal(dz.read(), want)
+        dx, dy = DeviceArray(want), DeviceArray(want)
