@@ -282,7 +282,14 @@ static nd_status upload(nd_ctx* ctx, const void* w, const void* s, uint32_t n, u
   if (e == hipSuccess) e = hipMalloc(&m->scales, sb);
   if (e == hipSuccess) e = hipMemcpyAsync(m->w, w, wb, kind, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->scales, s, sb, kind, ctx->stream);
-  if (e == hipSuccess) e = nd_tile_weights(m->w, n, k, &m->wt, ctx->stream);
+  if (e == hipSuccess) {
+    e = nd_tile_weights(m->w, n, k, &m->wt, ctx->stream);
+    if (e == hipErrorOutOfMemory) {  // matvecs go on without the copy, row by row
+      (void)hipGetLastError();
+      m->wt = nullptr;
+      e = hipSuccess;
+    }
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
     free_mat_buffers(m);
@@ -598,6 +605,9 @@ static nd_status check_matmul(nd_ctx* ctx, const nd_mat* m) {
     return nd_fail(ctx, ND_ERR_INVALID,
                    "nd_matmul needs per-row scales (g == k), k %% 64 == 0 and k <= 2048 "
                    "(got k=%u g=%u)", m->k, m->g);
+  if (!m->wt)
+    return nd_fail(ctx, ND_ERR_BACKEND,
+                   "the matrix was uploaded without memory for its operand-order copy");
   return ND_OK;
 }
 

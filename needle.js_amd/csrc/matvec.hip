@@ -695,6 +695,7 @@ hipError_t nd_launch_matvec(const nd_mat* m, const float* x, uint32_t batch, uin
                             uint32_t row_start, uint32_t row_count, float* y, uint32_t y_stride,
                             hipStream_t s, void* split) {
   if (row_count == 0 || batch == 0) return hipSuccess;
+  if (!m->wt) split = nullptr;  // no operand-order copy: the vector kernel
   // More than eight rows (the forms below then launch once for every eight:
   // 12 rows of 4096 x 4096, 15.8 us against 8.5), or more than 256 of the
   // fused form's workgroups, one to a CU (8 rows of 6000 x 2048, 9.3 against
