@@ -2693,8 +2693,10 @@ struct nd_needle {
   PoolState pool{};
   float *cells = nullptr, *pf_cells = nullptr;
   double *scores = nullptr, *pf_scores = nullptr, *conf_out = nullptr;
-  double* pf_pool = nullptr;  // the pass's slices: weighted sums [slice][8][d]
-  PoolSlice* pf_pool_slices = nullptr;
+  // Slices of a pool update past kStepCells cells (a pass, and a step of a
+  // model with that many layers): weighted sums [slice][8][d].
+  double* pool_part = nullptr;
+  PoolSlice* pool_slices = nullptr;
   // Which calls drive the runtime since the last reset: 0 none yet, 1 whole
   // steps (nd_needle_step, _prefill, _step_select, _generate), 2 the session
   // methods (ResidentExecutionSession, backends/backend.ts:65-80).
@@ -2739,6 +2741,7 @@ hipError_t enqueue_pool(nd_needle* n, const float* cells, uint32_t C, double* sc
                        scale, n->pool);
     return hipGetLastError();
   }
+  if (!n->pool_part || !n->pool_slices) return hipErrorInvalidValue;
   hipLaunchKernelGGL(n2_probe_scores_kernel, dim3((C + 3) / 4), dim3(256), 0, s, cells, C, D,
                      probes, n->probe_count, scale, scores);
   hipError_t e = hipGetLastError();
@@ -2747,9 +2750,9 @@ hipError_t enqueue_pool(nd_needle* n, const float* cells, uint32_t C, double* sc
   const uint32_t slices = (C + per - 1) / per;
   hipLaunchKernelGGL(n2_probe_pool_kernel, dim3(slices, (D + kPoolCols - 1) / kPoolCols),
                      dim3(kPoolThreads), 0, s, cells, C, D, n->probe_count, scores, per,
-                     n->pf_pool, n->pf_pool_slices);
+                     n->pool_part, n->pool_slices);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(n2_probe_merge_kernel, grid, dim3(256), 0, s, n->pf_pool, n->pf_pool_slices,
+  hipLaunchKernelGGL(n2_probe_merge_kernel, grid, dim3(256), 0, s, n->pool_part, n->pool_slices,
                      slices, D, n->pool);
   return hipGetLastError();
 }
@@ -3299,8 +3302,6 @@ nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
                           al((size_t)cap * d.kv_heads * kAttnCounterStride * 4),
                           n->conf ? al((size_t)cap * (d.layers + 1) * D * 4) : 0,
                           n->conf ? al((size_t)cap * (d.layers + 1) * kMaxProbes * 8) : 0,
-                          n->conf ? al((size_t)kPoolSlices * kMaxProbes * D * 8) : 0,
-                          n->conf ? al(kPoolSlices * sizeof(PoolSlice)) : 0,
                           al((size_t)cap * 32 * 16),
                           n->cq ? al((size_t)cap * (2 * d.engram_tables + 1) * 4) : 0};
   size_t total = 0;
@@ -3340,8 +3341,6 @@ nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
   take(&n->pf_counters);
   take(&n->pf_cells);
   take(&n->pf_scores);
-  take(&n->pf_pool);
-  take(&n->pf_pool_slices);
   take(&n->pf_rope);
   take(&n->pf_cq_lookup);
   n->pf_cap = cap;
@@ -3997,7 +3996,9 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
                             al((size_t)S * cat * 4), al((size_t)S * 2 * D * 4),
                             al((size_t)S * D * 4), al(pf * 4), al(20 * 4), al(64 * 8),
                             cb * al((size_t)(d.layers + 1) * D * 4),
-                            cb * al((size_t)(d.layers + 1) * P8), cb * al(64), al(32 * 4),
+                            cb * al((size_t)(d.layers + 1) * P8), cb * al(64),
+                            cb * al((size_t)kPoolSlices * P8 * D),
+                            cb * al(kPoolSlices * sizeof(PoolSlice)), al(32 * 4),
                             al((size_t)2 * S * D * 4),
                             al((size_t)(3 * D + ln * D + ln + ln * ln) * 4),
                             al((2 * 16 + 1) * 4)};
@@ -4054,6 +4055,8 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
     take(&n->cells);
     take(&n->scores);
     take(&n->conf_out);
+    take(&n->pool_part);
+    take(&n->pool_slices);
     take(&n->lookup);
     take(&n->host_eng);
     take(&n->fwd_in);

@@ -602,3 +602,36 @@ def test_prompt_that_outgrows_the_ring(hip, window, sink, prompts, mode, cq_bits
                     close(a, b, "float32 rows")
     finally:
         model.dispose()
+
+
+@pytest.mark.parametrize("layers", [31, 32, 40])
+def test_steps_of_a_deep_model_pool_without_a_prompt(hip, layers):
+    """A step pools layers + 1 confidence cells: up to 32 in one launch, more
+    through the slices a prompt's pass uses, whose memory a runtime that has
+    seen no prompt must have too.  Whole steps, the session's token and steps
+    after a prompt (graphs keep the addresses) against the oracle."""
+    say("needle2 deep model", layers)
+    g = Needle2Geometry(**{**SMALL.__dict__, "layers": layers, "sites": (0, layers - 1)})
+    w = Needle2Weights(g, 45)
+    model = NeedleModel(hip, w)
+    try:
+        rt = model.create_resident_runtime()
+        tokens = synth.Stream(14, "n2deep").integers(16, 0, g.vocab - 1)
+        ref = oracle.Needle2(w).runtime(g.max_length, 3)
+        rt.reset(g.max_length, 3)
+        for i, t in enumerate(tokens[:4]):
+            close(rt.step(int(t)), ref.step(int(t)), ("step", i))
+        alone = rt.resolve_confidence()
+        close_confidence(alone, ref.confidence(), "steps alone")
+        close(rt.prefill(tokens[4:10]), [ref.step(int(t)) for t in tokens[4:10]][-1], "prompt")
+        for i, t in enumerate(tokens[10:]):
+            close(rt.step(int(t)), ref.step(int(t)), ("step after the prompt", i))
+        close_confidence(rt.resolve_confidence(), ref.confidence(), "steps after a prompt")
+        session = model.create_runtime()
+        session.reset(g.max_length, 3)
+        for t in tokens[:4]:
+            session.step(int(t))
+        assert session.resolve_confidence() == alone
+        session.dispose()
+    finally:
+        model.dispose()
