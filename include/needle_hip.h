@@ -79,6 +79,14 @@ nd_status nd_test_xcd_local(nd_ctx* ctx, int32_t enable, uint32_t* probed);
 
 /* ------------------------------------------------------------- weights */
 
+/* Operand-order copies, no counterpart in the reference.  Besides its
+ * row-major codes a context keeps int8 matrices a second time in the order
+ * the matrix cores read.  A matrix that gets no copy (no memory for it, or
+ * past the context's limit) takes part in every call all the same, slower.
+ * Test hook: sets that limit, in bytes over all copies, for the matrices and
+ * models uploaded and created after the call. */
+nd_status nd_test_copy_limit(nd_ctx* ctx, uint64_t bytes);
+
 /* Uploads one int8 matrix: W int8 [n][k] row-major, scales f32 [n][k/g]
  * (one scale per row and group of g columns; g == k gives per-row scales).
  * Requires k % g == 0, g % 16 == 0, k % 16 == 0.  This is the int8 form of

@@ -128,9 +128,32 @@ void nd_xcd_override(bool off) {
   g_xcd_local = g_xcd_probed == 1 && !off;
 }
 
-static void free_mat_buffers(nd_mat* m) {
-  hipFree(m->w);
+static size_t copy_size(const nd_mat* m) { return ((size_t)m->n + 15) / 16 * 16 * m->k; }
+
+hipError_t nd_make_copy(nd_ctx* ctx, nd_mat* m) {
+  const size_t bytes = copy_size(m);
+  if (bytes > ctx->copy_limit || ctx->copy_bytes > ctx->copy_limit - bytes) return hipSuccess;
+  const hipError_t e = hipMalloc(&m->wt, bytes);
+  if (e != hipSuccess) {
+    m->wt = nullptr;
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    return hipSuccess;
+  }
+  ctx->copy_bytes += bytes;
+  return nd_tile_weights(m->w, m->n, m->k, m->wt, ctx->stream);
+}
+
+void nd_drop_copy(nd_ctx* ctx, nd_mat* m) {
+  if (!m->wt) return;
   hipFree(m->wt);
+  m->wt = nullptr;
+  ctx->copy_bytes -= copy_size(m);
+}
+
+static void free_mat_buffers(nd_ctx* ctx, nd_mat* m) {
+  nd_drop_copy(ctx, m);
+  hipFree(m->w);
   hipFree(m->scales);
   hipFree(m->packed);
   hipFree(m->norms);
@@ -202,7 +225,7 @@ nd_status nd_destroy(nd_ctx* ctx) {
   if (!ctx) return ND_OK;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->stream);
-  for (nd_mat* m : ctx->mats) free_mat_buffers(m);
+  for (nd_mat* m : ctx->mats) free_mat_buffers(ctx, m);
   for (nd_kv* kv : ctx->kvs) {
     hipFree(kv->k);
     delete kv;
@@ -253,6 +276,12 @@ nd_status nd_test_xcd_local(nd_ctx* ctx, int32_t enable, uint32_t* probed) {
 
 // ------------------------------------------------------------- matrices
 
+nd_status nd_test_copy_limit(nd_ctx* ctx, uint64_t bytes) {
+  if (!ctx) return nd_fail(nullptr, ND_ERR_BACKEND, "context is NULL");
+  ctx->copy_limit = (size_t)bytes;
+  return ND_OK;
+}
+
 static nd_status check_mat_shape(nd_ctx* ctx, uint32_t n, uint32_t k, uint32_t g) {
   if (n == 0 || k == 0 || g == 0)
     return nd_fail(ctx, ND_ERR_INVALID, "matrix shape %ux%u with group %u is empty", n, k, g);
@@ -282,17 +311,10 @@ static nd_status upload(nd_ctx* ctx, const void* w, const void* s, uint32_t n, u
   if (e == hipSuccess) e = hipMalloc(&m->scales, sb);
   if (e == hipSuccess) e = hipMemcpyAsync(m->w, w, wb, kind, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->scales, s, sb, kind, ctx->stream);
-  if (e == hipSuccess) {
-    e = nd_tile_weights(m->w, n, k, &m->wt, ctx->stream);
-    if (e == hipErrorOutOfMemory) {  // matvecs go on without the copy, row by row
-      (void)hipGetLastError();
-      m->wt = nullptr;
-      e = hipSuccess;
-    }
-  }
+  if (e == hipSuccess) e = nd_make_copy(ctx, m);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
-    free_mat_buffers(m);
+    free_mat_buffers(ctx, m);
     return nd_hip_fail(ctx, e, "matrix upload");
   }
   ctx->mats.insert(m);
@@ -315,7 +337,7 @@ nd_status nd_mat_free(nd_ctx* ctx, nd_mat* m) {
   if (!m) return ND_OK;
   if (!ctx->mats.erase(m)) return nd_fail(ctx, ND_ERR_INVALID, "matrix does not belong to context");
   ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  free_mat_buffers(m);
+  free_mat_buffers(ctx, m);
   return ND_OK;
 }
 
@@ -387,7 +409,7 @@ nd_status nd_mat_upload_cq(nd_ctx* ctx, const uint8_t* packed, const uint16_t* n
   if (e == hipSuccess) e = hipMemcpyAsync(m->norms, nsrc, nbytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
-    free_mat_buffers(m);
+    free_mat_buffers(ctx, m);
     return nd_hip_fail(ctx, e, "CQ matrix upload");
   }
   ctx->mats.insert(m);
@@ -605,9 +627,6 @@ static nd_status check_matmul(nd_ctx* ctx, const nd_mat* m) {
     return nd_fail(ctx, ND_ERR_INVALID,
                    "nd_matmul needs per-row scales (g == k), k %% 64 == 0 and k <= 2048 "
                    "(got k=%u g=%u)", m->k, m->g);
-  if (!m->wt)
-    return nd_fail(ctx, ND_ERR_BACKEND,
-                   "the matrix was uploaded without memory for its operand-order copy");
   return ND_OK;
 }
 

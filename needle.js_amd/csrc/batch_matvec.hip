@@ -628,7 +628,7 @@ Plan plan_batch(uint32_t width, uint32_t row_count, uint32_t batch, bool split) 
 bool nd_batch_matvec_fits(const nd_mat* m, uint32_t batch) {
   if (batch < 3) return false;
   if (m->bits) return m->g >= 32 && m->g <= kChunk && m->k >= 4 && m->cb_factor > 0.0;
-  return m->g % 32 == 0 && m->k % 128 == 0;
+  return m->wt && m->g % 32 == 0 && m->k % 128 == 0;
 }
 
 float nd_batch_matvec_us(const nd_mat* m, uint32_t row_count, uint32_t batch) {

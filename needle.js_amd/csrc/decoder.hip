@@ -313,7 +313,7 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
                            ctx->stream);
       row += p->n;
     }
-    if (e == hipSuccess) e = nd_tile_weights(m.w, m.n, m.k, &m.wt, ctx->stream);
+    if (e == hipSuccess) e = nd_make_copy(ctx, &m);
     dec->wo.push_back(d->wo[l]);
     dec->wup.push_back(d->wup[l]);
     dec->wdown.push_back(d->wdown[l]);
@@ -349,8 +349,8 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
     for (auto& m : dec->wqkv) {
+      nd_drop_copy(ctx, &m);
       hipFree(m.w);
-      hipFree(m.wt);
       hipFree(m.scales);
     }
     hipFree(dec->norms);
@@ -367,8 +367,8 @@ nd_status nd_decoder_free(nd_ctx* ctx, nd_decoder* dec) {
   if (!dec) return ND_OK;
   ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
   for (auto& m : dec->wqkv) {
+    nd_drop_copy(ctx, &m);
     hipFree(m.w);
-    hipFree(m.wt);
     hipFree(m.scales);
   }
   hipFree(dec->norms);

@@ -17,7 +17,8 @@
 // l%16 of each operand, k in [16*(l/16), +16) of the 64-wide step; the
 // accumulator's element i of lane l is row 4*(l/16)+i (weight row n) and
 // column l%16 (activation row m).  Weights come from the matrix's copy in that
-// order (nd_tile_weights), one contiguous KiB a load.
+// order (nd_tile_weights), one contiguous KiB a load; a matrix without a copy
+// runs on the digit-plane product's row-major form.
 #include <type_traits>
 
 #include "nd_internal.hpp"
@@ -67,7 +68,9 @@ __device__ __forceinline__ void digit_words(uint32_t a, uint32_t b, uint32_t c, 
 // the three exact integer sums) with agent-coherent stores, counts itself in
 // on the tile's counter, and the last of the S to arrive adds the partials in
 // slice order (deterministic), applies the epilogue and resets the counter.
-template <int MS, int NS, int EPI, bool PF>
+// ROWMAJOR: W is the row-major codes (same products, same bits without a
+// split).
+template <int MS, int NS, int EPI, bool PF, bool ROWMAJOR = false>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_digits_kernel(
     const int8_t* __restrict__ W, const float* __restrict__ sw, const int8_t* __restrict__ D,
     const float* __restrict__ fm, float* __restrict__ Y, uint32_t M, uint32_t N, uint32_t K,
@@ -111,9 +114,11 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_digits_kernel(
       const uint32_t ks = (uint32_t)q * 64 < kw ? q * 64 : 0;  // clamped past kw, never used
 #pragma unroll
       for (int a = 0; a < NS; ++a) {
-        const uint32_t n = n0 + a * 16;
-        wa[q][a] = *reinterpret_cast<const v4i*>(
-            W + ((size_t)((n < N ? n : N - 1) / 16) * (K / 64) + (kc + ks) / 64) * 1024 + lane * 16);
+        const uint32_t n = n0 + a * 16 + (ROWMAJOR ? lrow : 0), nn = n < N ? n : N - 1;
+        const size_t at = ROWMAJOR
+                              ? (size_t)nn * K + kc + ks + lk
+                              : ((size_t)(nn / 16) * (K / 64) + (kc + ks) / 64) * 1024 + lane * 16;
+        wa[q][a] = *reinterpret_cast<const v4i*>(W + at);
       }
     }
 #pragma unroll
@@ -853,12 +858,10 @@ __global__ __launch_bounds__(256) void tile_weights_kernel(const int8_t* __restr
 }
 }  // namespace
 
-hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t** wt, hipStream_t s) {
+hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t* wt, hipStream_t s) {
   const uint64_t units = ((uint64_t)n + 15) / 16 * k;
-  hipError_t e = hipMalloc(wt, units * 16);
-  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(tile_weights_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, w,
-                     n, k, units, reinterpret_cast<uint4*>(*wt));
+                     n, k, units, reinterpret_cast<uint4*>(wt));
   return hipGetLastError();
 }
 
@@ -897,11 +900,20 @@ hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, f
 // 21.6 / 43.9 for 64 x 128 tiles and 30.6 / 58.9 / 16.3 / 33.3 for 16 x 64).
 // With `split`, a grid of fewer than 256 tiles also splits k (K % 256 == 0)
 // into S = 2..8 slices until tiles * S reaches 256, within the workspace
-// (16 x 64 tiles only).
+// (16 x 64 tiles only).  A matrix without its operand-order copy takes 32 x 64
+// tiles of the row-major form, whole.
 hipError_t nd_launch_gemm(const nd_mat* w, const int8_t* digits, const float* fm, float* y,
                           uint32_t ldy, uint32_t M, int epilogue, hipStream_t s,
                           const nd_gemm_split* split) {
   if (M == 0) return hipSuccess;
+  if (!w->wt) {
+    const GemmFn f = epilogue == 0   ? &gemm_i8_digits_kernel<2, 1, 0, false, true>
+                     : epilogue == 1 ? &gemm_i8_digits_kernel<2, 1, 1, false, true>
+                                     : &gemm_i8_digits_kernel<2, 1, 2, false, true>;
+    hipLaunchKernelGGL(f, dim3((w->n + 63) / 64, (M + 31) / 32), dim3(kGemmThreads), 0, s, w->w,
+                       w->scales, digits, fm, y, M, w->n, w->k, ldy, w->k, nullptr, nullptr);
+    return hipGetLastError();
+  }
   // A wide product at decode M (the 32768-row lm head of a 64-row batch)
   // takes 32 x 128 tiles: 16.1 us with digitize, against 21.2 for 16 x 128
   // tiles with the k prefetch.
@@ -945,14 +957,15 @@ static uint32_t rows_subtiles(const nd_mat* w, uint32_t M) {
   return ns == 4 && w->k <= 512 && wgs > 256 && last > 0 && last <= 154 ? 2 : ns;
 }
 
-// Whether the row product takes (w, M): from 128 rows (the tiled kernels with
+// Whether the row product takes (w, M): a matrix with its operand-order copy,
+// from 128 rows (the tiled kernels with
 // their digitize launch: 6.8 against 7.3 us at 512 x 512, 7.1 against 7.4 at
 // 2048 x 512; at 64 rows they are level), and past k = 512, where a workgroup's
 // weights take longer than the tiled kernels' split ones, from 36 workgroups
 // (512 x 2048: 15.3 against 15.2 us at 400 rows, 15.6 against 19.9 at 700).
 bool nd_gemm_rows_fits(const nd_mat* w, const float* x, uint32_t ldx, bool norm, uint32_t M) {
   const uint32_t cols = 128 * rows_subtiles(w, M);
-  return M >= 128 && w->k % 64 == 0 && w->k <= 2048 && (!norm || w->k <= 512) &&
+  return w->wt && M >= 128 && w->k % 64 == 0 && w->k <= 2048 && (!norm || w->k <= 512) &&
          (w->k <= 512 || (uint64_t)((M + 15) / 16) * ((w->n + cols - 1) / cols) >= 36) &&
          ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
 }
@@ -988,14 +1001,14 @@ hipError_t nd_launch_gemm_rows(const nd_mat* w, const float* x, uint32_t ldx, co
 
 // Decode-shaped product on fp32 activations (optionally RMS-normalized with
 // `norm`): one launch instead of digitize + GEMM, for the shapes
-// nd_gemm_f32_fits accepts (M <= 64, K % 256 == 0 with K / 256 <= kMaxSplit
+// nd_gemm_f32_fits accepts (the matrix's operand-order copy, M <= 64, K % 256 == 0 with K / 256 <= kMaxSplit
 // slices, K <= kMaxNormK with a norm, the slices' partials and counters
 // within the workspace, 16-byte aligned rows).
 bool nd_gemm_f32_fits(const nd_mat* w, const float* x, uint32_t ldx, bool norm, uint32_t M,
                       const nd_gemm_split* split) {
   const uint32_t S = w->k / kKChunk;
   const uint32_t tiles = ((w->n + 63) / 64) * ((M + 15) / 16);
-  return M >= 1 && M <= 64 && w->k % kKChunk == 0 && S <= (uint32_t)kMaxSplit &&
+  return w->wt && M >= 1 && M <= 64 && w->k % kKChunk == 0 && S <= (uint32_t)kMaxSplit &&
          (!norm || w->k <= kMaxNormK) && split &&
          (S == 1 || (tiles <= split->counter_count &&
                      (size_t)tiles * S * 1024 <= split->partial_floats)) &&

@@ -22,7 +22,7 @@ constexpr size_t kCqSlack = 16;
 
 struct nd_mat {
   int8_t* w = nullptr;      // [n][k] int8 codes, row-major
-  int8_t* wt = nullptr;     // the same codes in MFMA operand order (nd_tile_weights)
+  int8_t* wt = nullptr;     // the same codes in MFMA operand order, or null (nd_make_copy)
   float* scales = nullptr;  // [n][k / g]
   uint32_t n = 0, k = 0, g = 0;
   // Cactus-Quant form (bits != 0; w and scales unused): packed codes
@@ -76,6 +76,8 @@ struct nd_ctx {
   // Row records and counters of split selection (grown on demand, zeroed).
   void* sel_split = nullptr;
   size_t sel_split_bytes = 0;
+  size_t copy_limit = ~size_t(0);  // bytes the operand-order copies may take (nd_make_copy)
+  size_t copy_bytes = 0;           // and take now
   std::set<nd_mat*> mats;
   std::set<nd_kv*> kvs;
   std::set<nd_pieces*> pieces;
@@ -242,14 +244,21 @@ hipError_t nd_launch_select_mask(const float* logits, uint32_t batch, uint32_t v
 // digitize.
 hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, float* norm_out,
                               int8_t* digits, float* fm, uint32_t M, uint32_t K, hipStream_t s);
-// The codes w [n][k] (k % 64 == 0) in MFMA operand order, allocated into *wt:
-// 1 KiB blocks [row / 16][k / 64], lane l of a block holding row l % 16, k
-// [16 (l / 16), +16).  Consecutive lanes of an MFMA operand are different rows,
-// and a wave's load is served four adjacent lanes (64 contiguous bytes) a
-// cycle: read from row-major memory every lane is a request of its own, 34
-// KB/us into a CU against 105-117 from this order (a 1 MB matrix read by 64 to
-// 256 workgroups).  Rows past n are zero.
-hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t** wt, hipStream_t s);
+// The codes w [n][k] (k % 64 == 0) in MFMA operand order: 1 KiB blocks [row /
+// 16][k / 64], lane l of a block holding row l % 16, k [16 (l / 16), +16).
+// Consecutive lanes of an MFMA operand are different rows, and a wave's load
+// is served four adjacent lanes (64 contiguous bytes) a cycle: read from
+// row-major memory every lane is a request of its own, 34 KB/us into a CU
+// against 105-117 from this order (a 1 MB matrix read by 64 to 256
+// workgroups).  Rows past n are zero.
+hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t* wt, hipStream_t s);
+// Gives an int8 matrix its copy in that order, wt, enqueued on the context's
+// stream.  Past the context's limit, or without memory, the matrix stays
+// without one and this still succeeds: its products then run on the vector
+// matvec and on nd_launch_gemm's row-major form (the *_fits functions refuse
+// it).  nd_drop_copy frees the copy.
+hipError_t nd_make_copy(nd_ctx* ctx, nd_mat* m);
+void nd_drop_copy(nd_ctx* ctx, nd_mat* m);
 inline __host__ __device__ size_t nd_tile_row(uint32_t row, uint32_t k) {
   return (size_t)(row >> 4) * (k / 64) * 1024 + (row & 15) * 16;
 }

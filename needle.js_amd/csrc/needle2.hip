@@ -3826,7 +3826,7 @@ nd_status nd_needle_create(nd_ctx* ctx, const nd_needle_desc* d, nd_needle** out
                            hipMemcpyDeviceToDevice, ctx->stream);
       row += p->n;
     }
-    if (e == hipSuccess) e = nd_tile_weights(m.w, m.n, m.k, &m.wt, ctx->stream);
+    if (e == hipSuccess) e = nd_make_copy(ctx, &m);
   };
   // Parts of one format are concatenated; a Cactus-Quant model also keeps
   // every part as a matrix of its own (a view into the concatenation, or an
@@ -3944,8 +3944,8 @@ nd_status nd_needle_free(nd_ctx* ctx, nd_needle* n) {
   if (n->pf_kv_arena) hipFree(n->pf_kv_arena);
   for (auto* v : {&n->wqkvg, &n->ekv, &n->owned_parts})
     for (auto& m : *v) {
+      nd_drop_copy(ctx, &m);
       if (m.w) hipFree(m.w);
-      if (m.wt) hipFree(m.wt);
       if (m.scales) hipFree(m.scales);
       if (m.packed) hipFree(m.packed);
       if (m.norms) hipFree(m.norms);

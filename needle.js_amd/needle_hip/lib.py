@@ -59,6 +59,7 @@ SIGNATURES = {
     "nd_sync": (I32, [P]),
     "nd_stream": (P, [P]),
     "nd_test_xcd_local": (I32, [P, I32, PU32]),
+    "nd_test_copy_limit": (I32, [P, C.c_uint64]),
     "nd_mat_upload_i8": (I32, [P, P, P, U32, U32, U32, PP]),
     "nd_mat_upload_i8_d": (I32, [P, P, P, U32, U32, U32, PP]),
     "nd_mat_free": (I32, [P, P]),
