@@ -81,9 +81,10 @@ nd_status nd_test_xcd_local(nd_ctx* ctx, int32_t enable, uint32_t* probed);
 
 /* Operand-order copies, no counterpart in the reference.  Besides its
  * row-major codes a context keeps int8 matrices a second time in the order
- * the matrix cores read.  A matrix that gets no copy (no memory for it, or
- * past the context's limit) takes part in every call all the same, slower.
- * Test hook: sets that limit, in bytes over all copies, for the matrices and
+ * the matrix cores read, as long as the copies take no more than an eighth
+ * of the GPU's memory and leave an eighth of it free.  A matrix that gets no
+ * copy takes part in every call all the same, slower.
+ * Test hook: sets the limit of the copies, in bytes over all copies, for the matrices and
  * models uploaded and created after the call. */
 nd_status nd_test_copy_limit(nd_ctx* ctx, uint64_t bytes);
 

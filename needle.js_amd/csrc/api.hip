@@ -128,12 +128,19 @@ void nd_xcd_override(bool off) {
   g_xcd_local = g_xcd_probed == 1 && !off;
 }
 
+constexpr size_t kCopyShare = 8;  // of the GPU's memory: at most one part in copies, one left free
+
 static size_t copy_size(const nd_mat* m) { return ((size_t)m->n + 15) / 16 * 16 * m->k; }
 
 hipError_t nd_make_copy(nd_ctx* ctx, nd_mat* m) {
   const size_t bytes = copy_size(m);
+  if (m->g % 32 != 0) return hipSuccess;
+  size_t free_now = 0, total = 0;
+  hipError_t e = hipMemGetInfo(&free_now, &total);
+  if (e != hipSuccess) return e;
+  if (free_now < bytes || free_now - bytes < total / kCopyShare) return hipSuccess;
   if (bytes > ctx->copy_limit || ctx->copy_bytes > ctx->copy_limit - bytes) return hipSuccess;
-  const hipError_t e = hipMalloc(&m->wt, bytes);
+  e = hipMalloc(&m->wt, bytes);
   if (e != hipSuccess) {
     m->wt = nullptr;
     if (e != hipErrorOutOfMemory) return e;
@@ -184,6 +191,7 @@ nd_status nd_create(int32_t device, nd_ctx** out) {
                    device, prop.gcnArchName);
   nd_ctx* ctx = new nd_ctx();
   ctx->device = device;
+  ctx->copy_limit = prop.totalGlobalMem / kCopyShare;
   e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete ctx;

@@ -295,12 +295,17 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
   const uint32_t qkv_rows = (d->heads + 2 * d->kv_heads) * kHd;
   dec->wqkv.resize(d->layers);
   hipError_t e = hipSuccess;
+  // The products read a layer's joined codes in operand order; the row-major
+  // ones stay only where a layer has no copy, else the next layer's follow
+  // them in the same memory (in stream order).
+  int8_t* joined = nullptr;
   for (uint32_t l = 0; l < d->layers && e == hipSuccess; ++l) {
     nd_mat& m = dec->wqkv[l];
     m.n = qkv_rows;
     m.k = d->dim;
     m.g = d->dim;
-    e = hipMalloc(&m.w, (size_t)qkv_rows * d->dim);
+    if (!joined) e = hipMalloc(&joined, (size_t)qkv_rows * d->dim);
+    m.w = joined;
     if (e == hipSuccess) e = hipMalloc(&m.scales, (size_t)qkv_rows * 4);
     const nd_mat* parts[3] = {d->wq[l], d->wk[l], d->wv[l]};
     size_t row = 0;
@@ -314,6 +319,8 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
       row += p->n;
     }
     if (e == hipSuccess) e = nd_make_copy(ctx, &m);
+    if (m.wt) m.w = nullptr;
+    else joined = nullptr;
     dec->wo.push_back(d->wo[l]);
     dec->wup.push_back(d->wup[l]);
     dec->wdown.push_back(d->wdown[l]);
@@ -347,6 +354,7 @@ nd_status nd_decoder_create(nd_ctx* ctx, const nd_decoder_desc* d, nd_decoder** 
     e = hipMemcpyAsync(dec->inv_freq, freq.data(), freq.size() * 8, hipMemcpyHostToDevice,
                        ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  hipFree(joined);
   if (e != hipSuccess) {
     for (auto& m : dec->wqkv) {
       nd_drop_copy(ctx, &m);

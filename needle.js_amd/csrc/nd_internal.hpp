@@ -76,8 +76,8 @@ struct nd_ctx {
   // Row records and counters of split selection (grown on demand, zeroed).
   void* sel_split = nullptr;
   size_t sel_split_bytes = 0;
-  size_t copy_limit = ~size_t(0);  // bytes the operand-order copies may take (nd_make_copy)
-  size_t copy_bytes = 0;           // and take now
+  size_t copy_limit = 0;  // bytes the operand-order copies may take (nd_make_copy)
+  size_t copy_bytes = 0;  // and take now
   std::set<nd_mat*> mats;
   std::set<nd_kv*> kvs;
   std::set<nd_pieces*> pieces;
@@ -253,10 +253,14 @@ hipError_t nd_launch_digitize(const float* x, uint32_t ldx, const float* norm, f
 // workgroups).  Rows past n are zero.
 hipError_t nd_tile_weights(const int8_t* w, uint32_t n, uint32_t k, int8_t* wt, hipStream_t s);
 // Gives an int8 matrix its copy in that order, wt, enqueued on the context's
-// stream.  Past the context's limit, or without memory, the matrix stays
-// without one and this still succeeds: its products then run on the vector
-// matvec and on nd_launch_gemm's row-major form (the *_fits functions refuse
-// it).  nd_drop_copy frees the copy.
+// stream.  A copy doubles what a matrix takes, so copies are made of memory
+// that is not scarce: up to an eighth of the GPU's for all of a context's (the
+// codes of a model of 36 GB), while another eighth stays free.  Past that, or
+// without memory, the matrix stays without one and this still succeeds: its
+// products then run on the vector matvec and on nd_launch_gemm's row-major
+// form (the *_fits functions refuse it).  Groups of columns that no
+// matrix-core kernel takes (g % 32 != 0) get none.  nd_drop_copy frees the
+// copy.
 hipError_t nd_make_copy(nd_ctx* ctx, nd_mat* m);
 void nd_drop_copy(nd_ctx* ctx, nd_mat* m);
 inline __host__ __device__ size_t nd_tile_row(uint32_t row, uint32_t k) {

@@ -6,14 +6,18 @@ their results equal those with the copy bit for bit; the models stay within
 the bars of the tests they are run through.
 """
 
+import ctypes as C
 import sys
 
 import numpy as np
 import pytest
 
 import oracle
+from helpers import hip_runtime
 from needle_hip import HipBackend, Int8Matrix, MatrixRowRange, NeedleModel, synth
-from needle_hip.models import ConstrainedWorkload, DecoderGeometry
+from needle_hip import lib as L
+from needle_hip.models import (ConstrainedWorkload, DecoderGeometry, DecoderWeights,
+                               HipDecoder)
 from needle_hip.needle2 import Needle2Geometry, Needle2Weights
 from test_gpu_decoder import matmul, run_case
 from test_gpu_needle2 import SMALL, check_kv, close
@@ -70,6 +74,52 @@ def test_batch_decode_from_row_major_codes(bare):
     g = DecoderGeometry(layers=2, vocab=4096)
     run_case(bare, g, ConstrainedWorkload(batch=3, steps=3, min_context=1, max_context=300,
                                           vocab=g.vocab), seed=11)
+
+
+def test_copies_take_their_share_and_no_more(hip):
+    """The copies counted through free memory: 64 MB more for 64 MB of codes, none
+    for groups that no matrix-core kernel reads or past the limit, and given
+    back with the matrix; a decoder keeps one form of its joined projections."""
+    say("memory of the copies")
+    lib, mb = hip_runtime(), 1 << 20
+    lib.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def now():
+        assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n, k = 16384, 4096
+    w = np.ones((n, k), np.int8)
+
+    def taken(backend, g):
+        s = np.ones((n, k // g), np.float32)
+        handle, before = C.c_void_p(), now()
+        backend._check(backend.lib.nd_mat_upload_i8(backend.ctx, L.ptr(w), L.ptr(s), n, k, g,
+                                                    C.byref(handle)))
+        grown = before - now()
+        backend._check(backend.lib.nd_mat_free(backend.ctx, handle))
+        assert abs(before - now()) < 4 * mb
+        return grown / mb
+
+    with HipBackend() as backend:
+        assert abs(taken(backend, 4096) - 128) < 8
+        assert abs(taken(backend, 16) - 80) < 8  # codes and 16 MB of scales
+        backend._check(backend.lib.nd_test_copy_limit(backend.ctx, 60 * mb))
+        assert abs(taken(backend, 4096) - 64) < 8
+    with HipBackend() as backend:
+        g = DecoderGeometry(layers=4, dim=2048, heads=32, kv_heads=32, ffn=2048, vocab=64)
+        weights = DecoderWeights(g, 1)
+        for role in ("wq", "wk", "wv", "wo", "wup", "wdown"):
+            for m in getattr(weights, role):
+                backend.upload(m)
+        backend.upload(weights.embedding)
+        before = now()
+        dec = HipDecoder(backend, weights)
+        # 4 layers of 6144 x 2048, and one more that the runtime may give back
+        # only with the stream's next work.
+        assert -8 < (before - now()) / mb - 4 * 12 < 12 + 8
+        dec.free()
 
 
 def test_needle_prompt_from_row_major_codes(bare):
