@@ -2126,8 +2126,8 @@ __global__ __launch_bounds__(kMixWg, ROWS ? 4 : 1) void n2_mix_kernel(MixArgs a)
 // While the prompt's cache slots do not wrap (positions < slots) the passes
 // work on the ring itself, which keeps every position a later query can see.
 // A prompt that outgrows the ring works on a linear prompt cache, one slot
-// per position and layer: the ring's rows are copied in once, every pass
-// appends to it and attends over each query's own window of it, and the rows
+// per position and layer (prompt_cache): the ring's rows are copied in once,
+// every pass appends to it and attends over each query's own window of it, and the rows
 // the ring keeps are copied back once after the last pass.
 
 // Per position: token from the prompt in `history`, engram hashes, scaled
@@ -2673,10 +2673,6 @@ struct nd_needle {
   uint32_t *pf_positions = nullptr, *pf_counters = nullptr;
   double2* pf_rope = nullptr;        // (sin, cos) of each position's RoPE angles [cap][32]
   uint32_t* pf_cq_lookup = nullptr;  // CQ model: each position's engram lookups and token
-  // The linear prompt cache (first prompt that outgrows its ring): max_length
-  // slots per layer and KV head, pf_kv.mode the widest row it holds so far.
-  char* pf_kv_arena = nullptr;
-  nd_kv pf_kv{};
   // Step graphs, valid for (graph_alloc, graph_sink).
   hipGraphExec_t graphs[3] = {nullptr, nullptr, nullptr};
   uint32_t graph_kernels[3] = {0, 0, 0};  // kernel launches each graph holds
@@ -3518,26 +3514,45 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
   return nd_launch_select_list(n->logits, d.vocab, nullptr, 0, n->sel_id, n->sel_lp, s);
 }
 
-// The linear prompt cache for this reset's cache mode.
-nd_status ensure_prompt_cache(nd_ctx* ctx, nd_needle* n) {
-  const nd_needle_desc& d = n->d;
-  const bool f32 = n->kv.mode == ND_KV_FLOAT32;
-  if (!n->pf_kv_arena || (f32 && n->pf_kv.mode != ND_KV_FLOAT32)) {
-    const size_t rows = (size_t)d.layers * d.kv_heads * d.max_length;
-    const size_t code_bytes = al(rows * kHd * (f32 ? 4 : 1)), scale_bytes = al(rows * 4);
-    if (n->pf_kv_arena) {  // earlier prompts may still read it
-      ND_HIP(ctx, hipStreamSynchronize(ctx->stream));
-      hipFree(n->pf_kv_arena);
-      n->pf_kv_arena = nullptr;
-    }
-    ND_HIP(ctx, hipMalloc(&n->pf_kv_arena, 2 * (code_bytes + scale_bytes)));
-    n->pf_kv.k = n->pf_kv_arena;
-    n->pf_kv.v = n->pf_kv_arena + code_bytes;
-    n->pf_kv.ks = reinterpret_cast<float*>(n->pf_kv_arena + 2 * code_bytes);
-    n->pf_kv.vs = reinterpret_cast<float*>(n->pf_kv_arena + 2 * code_bytes + scale_bytes);
-    n->pf_kv.mode = n->kv.mode;
+// Float32 cache rows that the reset's memory holds per layer and KV head: the
+// model's longest runtime and, for a model with a window, a ring of up to
+// kRingSinks sinks beside it (prompt_cache).
+constexpr uint32_t kRingSinks = 64;
+uint32_t cache_rows(const nd_needle_desc& d) {
+  const uint64_t ring = d.kv_window ? std::min((uint64_t)d.max_length,
+                                               (uint64_t)d.kv_window + kRingSinks) : 0;
+  return (uint32_t)std::min(d.max_length + ring, (uint64_t)~0u);
+}
+
+// The linear prompt cache of a prompt that ends at position `end` past the
+// ring, in the part of the reset's cache memory that the ring leaves unused:
+// a call allocates nothing.  An int8 ring takes at most the first quarter of
+// arrays sized for float32 rows, its prompt cache the second and the start of
+// the third.  A float32 ring's follows it; false when its rows do not reach
+// `end` (more than kRingSinks sinks and a prompt near the model's limit).
+bool prompt_cache(const nd_needle* n, uint32_t end, nd_kv* lin) {
+  const nd_kv& kv = n->kv;
+  const uint32_t rows = cache_rows(n->d);
+  const size_t heads = (size_t)n->d.layers * n->d.kv_heads;
+  *lin = kv;
+  if (kv.mode == ND_KV_FLOAT32) {
+    if (rows - kv.alloc < end) return false;
+    lin->alloc = rows - kv.alloc;
+    lin->k = reinterpret_cast<float*>(kv.k) + heads * kv.alloc * kHd;
+    lin->v = reinterpret_cast<float*>(kv.v) + heads * kv.alloc * kHd;
+    lin->ks = kv.ks + heads * kv.alloc;
+    lin->vs = kv.vs + heads * kv.alloc;
+    return true;
   }
-  return ND_OK;
+  lin->alloc = rows;
+  auto quarter = [&](void* base, size_t i) {
+    return reinterpret_cast<char*>(base) + i * heads * rows * kHd;
+  };
+  lin->k = quarter(kv.k, 1);
+  lin->v = quarter(kv.v, 1);
+  lin->ks = reinterpret_cast<float*>(quarter(kv.k, 2));
+  lin->vs = reinterpret_cast<float*>(quarter(kv.v, 2));
+  return true;
 }
 
 // Copies rows between the ring and the linear prompt cache lin: positions
@@ -3573,27 +3588,23 @@ nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits
   hipStream_t s = ctx->stream;
   uint32_t done = 0;
   const uint32_t fit = n->kv.alloc > n->position ? n->kv.alloc - n->position : 0;
-  if (count > fit && count - fit > kStepRest) {
-    if ((st = ensure_prompt_cache(ctx, n)) != ND_OK) return st;
-    nd_kv lin = n->kv;
-    lin.k = n->pf_kv.k;
-    lin.v = n->pf_kv.v;
-    lin.ks = n->pf_kv.ks;
-    lin.vs = n->pf_kv.vs;
-    // More than sink + window slots, the mark of a linear cache: the prompt
-    // outgrows the ring, so max_length does too.
-    lin.alloc = n->d.max_length;
+  nd_kv lin;  // more than sink + window slots, the mark of a linear cache
+  if (count > fit && count - fit > kStepRest && prompt_cache(n, n->position + count, &lin)) {
     const uint32_t first = n->position;
-    if (first) ND_HIP(ctx, enqueue_ring_copy(n, lin, 0, first, false, s));
+    hipError_t e = first ? enqueue_ring_copy(n, lin, 0, first, false, s) : hipSuccess;
     const uint32_t passes = (count + n->pf_cap - 1) / n->pf_cap;
-    for (uint32_t i = 0; i < passes; ++i) {  // even passes: no short last one
+    for (uint32_t i = 0; i < passes && e == hipSuccess; ++i) {  // even passes: no short last one
       const uint32_t chunk = (count - done + (passes - i) - 1) / (passes - i);
       const bool last = i + 1 == passes;
-      ND_HIP(ctx, enqueue_prefill(n, lin, chunk, last && want_logits, last && select, s));
+      e = enqueue_prefill(n, lin, chunk, last && want_logits, last && select, s);
+      if (e != hipSuccess) break;
       n->position += chunk;
       done += chunk;
     }
-    ND_HIP(ctx, enqueue_ring_copy(n, lin, first, n->position, true, s));
+    // The ring gets its rows of the passes that went through, whatever became
+    // of a later one.
+    const hipError_t back = enqueue_ring_copy(n, lin, first, n->position, true, s);
+    ND_HIP(ctx, e != hipSuccess ? e : back);
     return ND_OK;
   }
   while (done < count) {
@@ -3607,7 +3618,7 @@ nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits
       done += chunk;
       continue;
     }
-    // The few positions past the ring: one step per token.
+    // Positions past the ring, few or without a prompt cache: a step per token.
     const bool last = left == 1;
     if (graphs) {
       if ((st = launch_graph(ctx, n, last && (want_logits || select) ? kGraphPromptSelect
@@ -3941,7 +3952,6 @@ nd_status nd_needle_free(nd_ctx* ctx, nd_needle* n) {
   drop_graphs(n);
   if (n->arena) hipFree(n->arena);
   if (n->pf_arena) hipFree(n->pf_arena);
-  if (n->pf_kv_arena) hipFree(n->pf_kv_arena);
   for (auto* v : {&n->wqkvg, &n->ekv, &n->owned_parts})
     for (auto& m : *v) {
       nd_drop_copy(ctx, &m);
@@ -3974,7 +3984,7 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
   if (!n->arena) {
     // Sized for the model's max_length so that later resets never allocate.
     const uint32_t cap = d.max_length;
-    const size_t rows = (size_t)d.layers * d.kv_heads * cap;
+    const size_t rows = (size_t)d.layers * d.kv_heads * cache_rows(d);
     const size_t pf = nd_attention_batch_partial_floats(1, d.kv_heads, d.heads / d.kv_heads, cap);
     const uint32_t S = d.n_sites ? d.n_sites : 1;
     const uint32_t cat = d.n_sites ? d.engram_tables * d.engram_sub : 1;
@@ -3987,7 +3997,7 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
                             al((size_t)d.layers * 128), al(128),
                             cb * al(P8 * kMaxChunks), cb * al(P8 * kMaxChunks),
                             cb * al(P8 * D), al(64), al(64),
-                            // K and V sized for float32 rows (kvCache "float32")
+                            // K and V sized for float32 rows (kvCache "float32"; cache_rows)
                             al((size_t)d.vocab * 4), al((size_t)(d.vocab + 31) / 32 * 4), al(rows * kHd * 4), al(rows * kHd * 4),
                             al(rows * 4),
                             al(rows * 4), al((size_t)ln * D * 4), al(D * 4), al(D * 4), al(D * 4),

@@ -12,6 +12,7 @@ rounding) at most one code apart on at most 1% of a layer's codes, scales
 within 1e-3 relative.
 """
 
+import ctypes as C
 import dataclasses
 import sys
 
@@ -19,7 +20,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_codes_or_boundary_flips
+from helpers import assert_codes_or_boundary_flips, hip_runtime
 from needle_hip import NeedleError, NeedleModel, synth
 from needle_hip.needle2 import Needle2Geometry, Needle2Weights
 
@@ -633,5 +634,54 @@ def test_steps_of_a_deep_model_pool_without_a_prompt(hip, layers):
             session.step(int(t))
         assert session.resolve_confidence() == alone
         session.dispose()
+    finally:
+        model.dispose()
+
+
+@pytest.mark.parametrize("mode,window,sink,length", [("int8", 40, 5, 300), ("int8", 40, 5, 20000),
+                                                     ("float32", 40, 5, 300),
+                                                     ("float32", 40, 5, 20000),
+                                                     ("float32", 40, 90, 300)])
+def test_prompt_past_the_ring_takes_no_memory(hip, mode, window, sink, length):
+    """A prompt past the ring, up to the model's last position or of a model
+    whose cache takes 16 MB as int8 codes, works beside the ring in the reset's
+    own memory: nothing is allocated (free memory is the same), and logits and
+    cache rows are those of a step per token.  A float32 ring of more than 64
+    sinks leaves no room there for a prompt to the last position: the
+    positions past it run as steps."""
+    say("needle2 prompt cache", mode, window, sink, length)
+    total = 300
+    g = Needle2Geometry(**{**SMALL.__dict__, "kv_window": window, "max_length": length})
+    model = NeedleModel(hip, Needle2Weights(g, 44))
+    lib = hip_runtime()
+    free, whole = C.c_size_t(), C.c_size_t()
+
+    def now():
+        assert lib.hipDeviceSynchronize() == 0
+        assert lib.hipMemGetInfo(C.byref(free), C.byref(whole)) == 0
+        return free.value
+
+    def rows():
+        return [model.resident.kv_read(l, h) for l in range(g.layers) for h in range(g.kv_heads)]
+
+    try:
+        rt, resident = model.create_resident_runtime(), model.resident
+        tokens = synth.Stream(16, "n2mem").integers(total, 0, g.vocab - 1)
+        resident.reset(g.max_length, sink, mode)
+        for t in tokens:
+            want = rt.step(int(t))
+        stepped = rows()
+        resident.reset(g.max_length, sink, mode)
+        rt.prefill(tokens[:10])  # the prompt buffers
+        before = now()
+        close(rt.prefill(tokens[10:]), want, "prompt")
+        assert now() == before, (before, now())
+        for got, ref in zip(rows(), stepped):
+            if mode == "int8":
+                d = np.abs(got[0].astype(int) - ref[0].astype(int))
+                assert d.max() <= 1 and np.count_nonzero(d) <= 0.01 * d.size
+            else:
+                close(got[0], ref[0], "float32 keys")
+                close(got[1], ref[1], "float32 values")
     finally:
         model.dispose()
