@@ -3276,34 +3276,46 @@ nd_status launch_graph(nd_ctx* ctx, nd_needle* n, GraphKind kind) {
   return ND_OK;
 }
 
-// Buffers of the batched prefill, for up to pf_cap positions per pass.
+// Buffers of the batched prefill, for up to pf_cap positions per pass: the most
+// a pass takes or, without the memory for that many, half of it.
 nd_status ensure_prefill(nd_ctx* ctx, nd_needle* n) {
   if (n->pf_arena) return ND_OK;
   const nd_needle_desc& d = n->d;
-  const uint32_t cap = std::min<uint32_t>(d.max_length, kPrefillRows);
   const uint32_t D = d.dim, ln = d.lanes, qw = d.heads * kHd, kw = d.kv_heads * kHd;
   const uint32_t S = d.n_sites ? d.n_sites : 1, cat = d.n_sites ? d.engram_tables * d.engram_sub : 1;
   const uint32_t kmax = std::max(std::max(D, qw), cat);
-  const size_t pf = nd_attention_batch_partial_floats(cap, d.kv_heads, d.heads / d.kv_heads,
-                                                      d.max_length);
-  const size_t sizes[] = {al((size_t)cap * ln * D * 4), al((size_t)cap * D * 4),
-                          al((size_t)cap * D * 4),      al((size_t)cap * D * 4),
-                          al((size_t)cap * ln * 4),     al((size_t)cap * ln * ln * 4),
-                          al((size_t)cap * 20 * 4),     al((size_t)cap * (2 * qw + 2 * kw) * 4),
-                          al((size_t)cap * qw * 4),     al((size_t)cap * qw * 4),
-                          al((size_t)cap * D * 4),      al((size_t)cap * S * cat * 4),
-                          al((size_t)cap * S * 2 * D * 4), al((size_t)cap * S * D * 4),
-                          al((size_t)cap * 4),          al(pf * 4),
-                          al((size_t)3 * cap * kmax),   al((size_t)cap * 4),
-                          al((size_t)cap * d.kv_heads * kAttnCounterStride * 4),
-                          n->conf ? al((size_t)cap * (d.layers + 1) * D * 4) : 0,
-                          n->conf ? al((size_t)cap * (d.layers + 1) * kMaxProbes * 8) : 0,
-                          al((size_t)cap * 32 * 16),
-                          n->cq ? al((size_t)cap * (2 * d.engram_tables + 1) * 4) : 0};
-  size_t total = 0;
-  for (size_t v : sizes) total += v;
-  hipError_t e = hipMalloc(&n->pf_arena, total);
-  if (e == hipSuccess) e = hipMemsetAsync(n->pf_arena, 0, total, ctx->stream);
+  auto sizes_of = [&](uint32_t cap) {
+    const size_t pf = nd_attention_batch_partial_floats(cap, d.kv_heads, d.heads / d.kv_heads,
+                                                        d.max_length);
+    return std::vector<size_t>{
+        al((size_t)cap * ln * D * 4), al((size_t)cap * D * 4),
+        al((size_t)cap * D * 4),      al((size_t)cap * D * 4),
+        al((size_t)cap * ln * 4),     al((size_t)cap * ln * ln * 4),
+        al((size_t)cap * 20 * 4),     al((size_t)cap * (2 * qw + 2 * kw) * 4),
+        al((size_t)cap * qw * 4),     al((size_t)cap * qw * 4),
+        al((size_t)cap * D * 4),      al((size_t)cap * S * cat * 4),
+        al((size_t)cap * S * 2 * D * 4), al((size_t)cap * S * D * 4),
+        al((size_t)cap * 4),          al(pf * 4),
+        al((size_t)3 * cap * kmax),   al((size_t)cap * 4),
+        al((size_t)cap * d.kv_heads * kAttnCounterStride * 4),
+        n->conf ? al((size_t)cap * (d.layers + 1) * D * 4) : 0,
+        n->conf ? al((size_t)cap * (d.layers + 1) * kMaxProbes * 8) : 0,
+        al((size_t)cap * 32 * 16),
+        n->cq ? al((size_t)cap * (2 * d.engram_tables + 1) * 4) : 0};
+  };
+  std::vector<size_t> sizes;
+  uint32_t cap = 0;
+  hipError_t e = hipErrorOutOfMemory;
+  for (uint32_t rows = kPrefillRows; rows >= kPrefillRows / 2 && e == hipErrorOutOfMemory;
+       rows /= 2) {
+    cap = std::min<uint32_t>(d.max_length, rows);
+    sizes = sizes_of(cap);
+    size_t total = 0;
+    for (size_t v : sizes) total += v;
+    (void)hipGetLastError();
+    e = hipMalloc(&n->pf_arena, total);
+    if (e == hipSuccess) e = hipMemsetAsync(n->pf_arena, 0, total, ctx->stream);
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
     if (n->pf_arena) hipFree(n->pf_arena);

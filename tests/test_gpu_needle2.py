@@ -685,3 +685,29 @@ def test_prompt_past_the_ring_takes_no_memory(hip, mode, window, sink, length):
                 close(got[1], ref[1], "float32 values")
     finally:
         model.dispose()
+
+
+def test_prompt_passes_shrink_to_the_memory(hip):
+    """A model so long that the buffers of the largest prompt pass do not fit
+    the GPU (its attention's chunk partials grow with the length) and those of
+    half of it do: its prompts run all the same."""
+    lib = hip_runtime()
+    free, whole = C.c_size_t(), C.c_size_t()
+    assert lib.hipMemGetInfo(C.byref(free), C.byref(whole)) == 0
+    if free.value < 0.8 * whole.value:
+        pytest.skip("needs most of the GPU's memory")
+    rows, heads = 1024, SMALL.heads
+    length = int(1.02 * whole.value / (rows * heads * 66 * 4 / 128))
+    say("needle2 prompt passes", length)
+    g = Needle2Geometry(**{**SMALL.__dict__, "layers": 1, "sites": (0,), "max_length": length})
+    model = NeedleModel(hip, Needle2Weights(g, 47))
+    try:
+        rt = model.create_resident_runtime()
+        tokens = synth.Stream(17, "n2passes").integers(80, 0, g.vocab - 1)
+        rt.reset(200, 3)
+        for t in tokens:
+            want = rt.step(int(t))
+        rt.reset(200, 3)
+        close(rt.prefill(tokens), want, "prompt")
+    finally:
+        model.dispose()
