@@ -248,6 +248,10 @@ __device__ __forceinline__ void mfma_reduce_store(float4v acc, float* red, uint3
 // one group stays a permutation within each 256-byte block.
 constexpr uint32_t kFusedMaxK = 2048;
 constexpr uint32_t kMaxSlices = 16;  // k = 8192 in slices of 512
+// The smallest exponent a row is scaled by: 2^126 is the largest power of two
+// that brings a row of subnormals up without overflow, and what is left of
+// their bits (multiples of 2^-23) both halves hold exactly.
+constexpr int kMinExp = -126;
 constexpr int kXUnits = kFusedMaxK / 8 / 128;  // 8-value units of x per thread
 
 template <int NP>
@@ -351,6 +355,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void matvec_mfma_fused_kernel(
   const float amax = fmaxf(s_max[2 * xb], s_max[2 * xb + 1]);
   int ex = 0;
   if (amax > 0.f && amax <= 3.4028235e38f) frexpf(amax, &ex);  // amax < 2^ex
+  ex = ex < kMinExp ? kMinExp : ex;
   const float down = ldexpf(1.f, -ex);
   if (xj == 0) s_e[xb] = ex;
 #pragma unroll
@@ -496,6 +501,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves) void matvec_mfma_slice_kernel(
     for (uint32_t i = 0; i < kWpr; ++i) amax = fmaxf(amax, s_max[xb * kWpr + i]);
     int ex = 0;
     if (amax > 0.f && amax <= 3.4028235e38f) frexpf(amax, &ex);  // amax < 2^ex
+    ex = ex < kMinExp ? kMinExp : ex;
     const float down = ldexpf(1.f, -ex);
     if (u == 0) s_e[xb] = ex;
     half8 hv, lv;

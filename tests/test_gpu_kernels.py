@@ -417,3 +417,23 @@ def test_matvec_many_rows(hip, n, k, g, batch):
         want = x.astype(np.float64) @ full[lo:lo + count].T
         bound = 2.0 ** -18 * (np.abs(x).astype(np.float64) @ np.abs(full[lo:lo + count]).T) + 1e-43
         assert np.all(np.abs(got - want) <= bound), (lo, np.max(np.abs(got - want) / bound))
+
+
+@pytest.mark.parametrize("n,k,g,batch", [(70, 512, 32, 3), (33, 2048, 2048, 8), (130, 4096, 64, 5),
+                                         (96, 8192, 32, 8)])
+def test_matvec_rows_of_subnormals(hip, n, k, g, batch):
+    """Batches of 3 to 8 rows in one launch and in k slices: rows whose largest
+    element is subnormal, or normal and below 2^-120, among ordinary ones.  Their
+    scaled halves hold them exactly, so the bound is that of fp32 sums (2^-18
+    of the absolute sum, at most 57 + 16 additions) and, per output, the
+    rounding to the last bit of a subnormal."""
+    say("matvec subnormal rows", n, k, g, batch)
+    w, s = synth.int8_matrix(62, f"sub{n}x{k}", n, k, g)
+    x = synth.Stream(62, f"subx{k}b{batch}").normal((batch, k))
+    x[0] *= np.float32(1e-41)
+    x[1] *= np.float32(1e-37)
+    full = w.astype(np.float64) * np.repeat(s.astype(np.float64), g, axis=1)
+    got = hip.matvec(Int8Matrix(w, s, g), x).astype(np.float64)
+    want = x.astype(np.float64) @ full.T
+    bound = 2.0 ** -18 * (np.abs(x).astype(np.float64) @ np.abs(full).T) + 2.0 ** -148
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
