@@ -60,6 +60,25 @@ __device__ __forceinline__ void digit_words(uint32_t a, uint32_t b, uint32_t c, 
   w2 = __builtin_amdgcn_perm(cd2, ab2, 0x05040100u) ^ 0x80808080u;
 }
 
+// A row's digit scale: unit 2^(e - 21), up its reciprocal, for max |v| = amax
+// in [2^e, 2^(e+1)).  The unit is no smaller than the last bit of a subnormal
+// (which holds any row exactly), and for rows below 2^-106, whose reciprocal
+// unit is no float, lift is the part 2^64 of it that their values take first.
+struct DigitScale {
+  int e;
+  float lift, up;
+};
+__device__ __forceinline__ DigitScale digit_scale(float amax) {
+  int e = 0;
+  if (amax > 0.f) {
+    frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
+    e -= 1;
+  }
+  e = e < -128 ? -128 : e;
+  const bool small = e < -106;
+  return {e, small ? 0x1p64f : 1.f, ldexpf(1.f, (small ? -43 : 21) - e)};
+}
+
 // MS m-subtiles of 16 and NS n-subtiles of 16 per wave; 4 waves split n.
 // blockIdx.z selects the k slice [z * kslice, +kslice) (kslice = K without a
 // split).  Each 256-wide chunk issues its weight loads first and then stages
@@ -274,24 +293,23 @@ __global__ __launch_bounds__(256) void digitize_kernel(const float* __restrict__
   if ((t & 63) == 0) red[4 + (t >> 6)] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
-  int e = 0;
-  if (amax > 0.f) {
-    frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-    e -= 1;
+  const DigitScale sc = digit_scale(amax);
+  if (sc.lift != 1.f) {
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) v[i] *= sc.lift;
   }
-  const float up = ldexpf(1.f, 21 - e);
   const size_t plane = (size_t)M * K;
 #pragma unroll
   for (uint32_t i = 0; i < 8; ++i) {
     const uint32_t k = t + i * 256;
     if (i < per && k < K) {
-      const uint32_t u = digit_bias(v[i], up);
+      const uint32_t u = digit_bias(v[i], sc.up);
       D[(size_t)m * K + k] = (int8_t)(u ^ 0x80u);
       D[plane + (size_t)m * K + k] = (int8_t)((u >> 8) ^ 0x80u);
       D[2 * plane + (size_t)m * K + k] = (int8_t)((u >> 16) ^ 0x80u);
     }
   }
-  if (t == 0) fm[m] = ldexpf(1.f, e - 21);
+  if (t == 0) fm[m] = ldexpf(1.f, sc.e - 21);
 }
 
 // The same split with one wave per row (4 rows per workgroup): lane l holds
@@ -344,12 +362,16 @@ __global__ __launch_bounds__(256) void digitize_rows_kernel(const float* __restr
   amax = nd::row_max(amax);
   amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
                fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
-  int e = 0;
-  if (amax > 0.f) {
-    frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-    e -= 1;
+  const DigitScale sc = digit_scale(amax);
+  if (sc.lift != 1.f) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      v[i].x *= sc.lift;
+      v[i].y *= sc.lift;
+      v[i].z *= sc.lift;
+      v[i].w *= sc.lift;
+    }
   }
-  const float up = ldexpf(1.f, 21 - e);
   const size_t plane = (size_t)M * K;
   uint32_t* d0p = reinterpret_cast<uint32_t*>(D + (size_t)m * K);
   uint32_t* d1p = reinterpret_cast<uint32_t*>(D + plane + (size_t)m * K);
@@ -359,13 +381,13 @@ __global__ __launch_bounds__(256) void digitize_rows_kernel(const float* __restr
     const uint32_t u = lane + 64 * i;
     if (u >= units) continue;
     uint32_t w0, w1, w2;
-    digit_words(digit_bias(v[i].x, up), digit_bias(v[i].y, up), digit_bias(v[i].z, up),
-                digit_bias(v[i].w, up), w0, w1, w2);
+    digit_words(digit_bias(v[i].x, sc.up), digit_bias(v[i].y, sc.up), digit_bias(v[i].z, sc.up),
+                digit_bias(v[i].w, sc.up), w0, w1, w2);
     d0p[u] = w0;
     d1p[u] = w1;
     d2p[u] = w2;
   }
-  if (lane == 0) fm[m] = ldexpf(1.f, e - 21);
+  if (lane == 0) fm[m] = ldexpf(1.f, sc.e - 21);
 }
 
 // Decode-shaped product (M <= 64 rows per launch, 16 x 64 output tiles) that
@@ -515,12 +537,12 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[c][i]));
     amax = nd::row_max(amax);
-    int e = 0;
-    if (amax > 0.f) {
-      frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-      e -= 1;
+    const DigitScale sc = digit_scale(amax);
+    const float up = live ? sc.up : 0.f;
+    if (sc.lift != 1.f) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[c][i] *= sc.lift;
     }
-    const float up = live ? ldexpf(1.f, 21 - e) : 0.f;
     uint32_t d0w[4], d1w[4], d2w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -530,7 +552,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
     *reinterpret_cast<uint4*>(&lds[c][0][r][pc * 16]) = make_uint4(d0w[0], d0w[1], d0w[2], d0w[3]);
     *reinterpret_cast<uint4*>(&lds[c][1][r][pc * 16]) = make_uint4(d1w[0], d1w[1], d1w[2], d1w[3]);
     *reinterpret_cast<uint4*>(&lds[c][2][r][pc * 16]) = make_uint4(d2w[0], d2w[1], d2w[2], d2w[3]);
-    if (pc == 0) s_fm[c][r] = ldexpf(1.f, e - 21);
+    if (pc == 0) s_fm[c][r] = ldexpf(1.f, sc.e - 21);
   }
   __syncthreads();
 
@@ -753,25 +775,29 @@ __global__ __launch_bounds__(512) void gemm_i8_rows_kernel(
     amax = nd::row_max(amax);
     amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
                  fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
-    int e = 0;
-    if (amax > 0.f) {
-      frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-      e -= 1;
+    const DigitScale sc = digit_scale(amax);
+    if (sc.lift != 1.f) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        v[r][i].x *= sc.lift;
+        v[r][i].y *= sc.lift;
+        v[r][i].z *= sc.lift;
+        v[r][i].w *= sc.lift;
+      }
     }
-    const float up = ldexpf(1.f, 21 - e);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       const uint32_t u = lane + 64 * i;
       if (u >= units) continue;
       uint32_t d0, d1, d2;
-      digit_words(digit_bias(v[r][i].x, up), digit_bias(v[r][i].y, up),
-                  digit_bias(v[r][i].z, up), digit_bias(v[r][i].w, up), d0, d1, d2);
+      digit_words(digit_bias(v[r][i].x, sc.up), digit_bias(v[r][i].y, sc.up),
+                  digit_bias(v[r][i].z, sc.up), digit_bias(v[r][i].w, sc.up), d0, d1, d2);
       int8_t* at = lds + lr * kld + 4 * u;
       *reinterpret_cast<uint32_t*>(at) = d0;
       *reinterpret_cast<uint32_t*>(at + kRows * kld) = d1;
       *reinterpret_cast<uint32_t*>(at + 2 * kRows * kld) = d2;
     }
-    if (lane == 0) s_fm[lr] = ldexpf(1.f, e - 21);
+    if (lane == 0) s_fm[lr] = ldexpf(1.f, sc.e - 21);
   }
   nd::lds_barrier();
 

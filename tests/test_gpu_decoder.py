@@ -325,3 +325,34 @@ def test_matmul_into_its_input(hip, accumulate):
         want = dy.read()
         assert np.array_equal(dz.read(), want)
         dx, dy = DeviceArray(want), DeviceArray(want)
+
+
+@pytest.mark.parametrize("rows,n,k,offset", [(5, 70, 256, 0), (5, 70, 2048, 1), (130, 300, 512, 0),
+                                             (130, 300, 512, 1), (600, 512, 1024, 0)])
+def test_matmul_rows_of_small_values(hip, rows, n, k, offset):
+    """Rows whose largest element is subnormal or below 2^-106 (their digits'
+    reciprocal unit is no float), digitized apart (few rows, x off the 16-byte
+    grid) and inside the product, plain and added into y.  Bound: the digits
+    keep 2^-22 of the row's largest element or any subnormal exactly, the
+    factors and the sum round a few times: 2^-21 of the row maximum times the
+    absolute weights plus 2^-21 of the values, and 2^-147 for roundings to the
+    last bit of a subnormal."""
+    say("matmul small rows", rows, n, k, offset)
+    w, s = synth.int8_matrix(74, f"small{n}x{k}", n, k, k)
+    x = synth.Stream(74, f"sx{k}r{rows}").normal((rows, k))
+    for i, f in enumerate((1e-41, 1e-38, 1e-34, 1e-31)):
+        x[i] *= np.float32(f)
+    room = np.zeros(rows * k + offset, np.float32)
+    room[offset:] = x.reshape(-1)
+    dx, dy = DeviceArray(room), DeviceArray(np.zeros((rows, n), np.float32))
+    mat = hip.upload(Int8Matrix(w, s, k))
+    full = w.astype(np.float64) * s.astype(np.float64)
+    want = x.astype(np.float64) @ full.T
+    top = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
+    bound = 2.0 ** -21 * (top * np.abs(full).sum(axis=1)[None] + np.abs(want)) + 2.0 ** -147
+    for times in (1, 2):
+        hip._check(hip.lib.nd_matmul_d(hip.ctx, mat, dx.ptr.value + 4 * offset, rows, dy.ptr,
+                                       times - 1, None))
+        hip._check(hip.lib.nd_sync(hip.ctx))
+        err = np.abs(dy.read().astype(np.float64) - times * want)
+        assert np.all(err <= times * bound), (times, np.max(err / bound))
