@@ -60,23 +60,18 @@ __device__ __forceinline__ void digit_words(uint32_t a, uint32_t b, uint32_t c, 
   w2 = __builtin_amdgcn_perm(cd2, ab2, 0x05040100u) ^ 0x80808080u;
 }
 
-// A row's digit scale: unit 2^(e - 21), up its reciprocal, for max |v| = amax
-// in [2^e, 2^(e+1)).  The unit is no smaller than the last bit of a subnormal
-// (which holds any row exactly), and for rows below 2^-106, whose reciprocal
-// unit is no float, lift is the part 2^64 of it that their values take first.
+// A row's digit scale: unit 2^(e - 21) and up its reciprocal, for max |v| =
+// amax in [2^e, 2^(e+1)), straight from the exponent bits.  The unit ends at
+// 2^-126, whose reciprocal is still a float: values are carried to 2^-22 of
+// the row's largest, or to 2^-127 in a row below 2^-105 (bringing such rows
+// up first would keep their bits, and cost every product 1%: the waves wait
+// for their rows' scales).
 struct DigitScale {
-  int e;
-  float lift, up;
+  float unit, up;
 };
 __device__ __forceinline__ DigitScale digit_scale(float amax) {
-  int e = 0;
-  if (amax > 0.f) {
-    frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-    e -= 1;
-  }
-  e = e < -128 ? -128 : e;
-  const bool small = e < -106;
-  return {e, small ? 0x1p64f : 1.f, ldexpf(1.f, (small ? -43 : 21) - e)};
+  const uint32_t f = max((__float_as_uint(amax) >> 23) & 0xffu, 22u);
+  return {__uint_as_float((f - 21) << 23), __uint_as_float((275 - f) << 23)};
 }
 
 // MS m-subtiles of 16 and NS n-subtiles of 16 per wave; 4 waves split n.
@@ -294,10 +289,6 @@ __global__ __launch_bounds__(256) void digitize_kernel(const float* __restrict__
   __syncthreads();
   amax = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
   const DigitScale sc = digit_scale(amax);
-  if (sc.lift != 1.f) {
-#pragma unroll
-    for (uint32_t i = 0; i < 8; ++i) v[i] *= sc.lift;
-  }
   const size_t plane = (size_t)M * K;
 #pragma unroll
   for (uint32_t i = 0; i < 8; ++i) {
@@ -309,7 +300,7 @@ __global__ __launch_bounds__(256) void digitize_kernel(const float* __restrict__
       D[2 * plane + (size_t)m * K + k] = (int8_t)((u >> 16) ^ 0x80u);
     }
   }
-  if (t == 0) fm[m] = ldexpf(1.f, sc.e - 21);
+  if (t == 0) fm[m] = sc.unit;
 }
 
 // The same split with one wave per row (4 rows per workgroup): lane l holds
@@ -358,20 +349,12 @@ __global__ __launch_bounds__(256) void digitize_rows_kernel(const float* __restr
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < VEC; ++i)
-    amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+    amax = fmaxf(fmaxf(fmaxf(amax, fabsf(v[i].x)), fabsf(v[i].y)),
+                   fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
   amax = nd::row_max(amax);
   amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
-               fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
+                 fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
   const DigitScale sc = digit_scale(amax);
-  if (sc.lift != 1.f) {
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      v[i].x *= sc.lift;
-      v[i].y *= sc.lift;
-      v[i].z *= sc.lift;
-      v[i].w *= sc.lift;
-    }
-  }
   const size_t plane = (size_t)M * K;
   uint32_t* d0p = reinterpret_cast<uint32_t*>(D + (size_t)m * K);
   uint32_t* d1p = reinterpret_cast<uint32_t*>(D + plane + (size_t)m * K);
@@ -387,7 +370,7 @@ __global__ __launch_bounds__(256) void digitize_rows_kernel(const float* __restr
     d1p[u] = w1;
     d2p[u] = w2;
   }
-  if (lane == 0) fm[m] = ldexpf(1.f, sc.e - 21);
+  if (lane == 0) fm[m] = sc.unit;
 }
 
 // Decode-shaped product (M <= 64 rows per launch, 16 x 64 output tiles) that
@@ -539,10 +522,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
     amax = nd::row_max(amax);
     const DigitScale sc = digit_scale(amax);
     const float up = live ? sc.up : 0.f;
-    if (sc.lift != 1.f) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) v[c][i] *= sc.lift;
-    }
     uint32_t d0w[4], d1w[4], d2w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -552,7 +531,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
     *reinterpret_cast<uint4*>(&lds[c][0][r][pc * 16]) = make_uint4(d0w[0], d0w[1], d0w[2], d0w[3]);
     *reinterpret_cast<uint4*>(&lds[c][1][r][pc * 16]) = make_uint4(d1w[0], d1w[1], d1w[2], d1w[3]);
     *reinterpret_cast<uint4*>(&lds[c][2][r][pc * 16]) = make_uint4(d2w[0], d2w[1], d2w[2], d2w[3]);
-    if (pc == 0) s_fm[c][r] = ldexpf(1.f, sc.e - 21);
+    if (pc == 0) s_fm[c][r] = sc.unit;
   }
   __syncthreads();
 
@@ -770,21 +749,12 @@ __global__ __launch_bounds__(512) void gemm_i8_rows_kernel(
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < VEC; ++i)
-      amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[r][i].x), fabsf(v[r][i].y)),
-                               fmaxf(fabsf(v[r][i].z), fabsf(v[r][i].w))));
+      amax = fmaxf(fmaxf(fmaxf(amax, fabsf(v[r][i].x)), fabsf(v[r][i].y)),
+                     fmaxf(fabsf(v[r][i].z), fabsf(v[r][i].w)));
     amax = nd::row_max(amax);
     amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
-                 fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
+                   fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
     const DigitScale sc = digit_scale(amax);
-    if (sc.lift != 1.f) {
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        v[r][i].x *= sc.lift;
-        v[r][i].y *= sc.lift;
-        v[r][i].z *= sc.lift;
-        v[r][i].w *= sc.lift;
-      }
-    }
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       const uint32_t u = lane + 64 * i;
@@ -797,7 +767,7 @@ __global__ __launch_bounds__(512) void gemm_i8_rows_kernel(
       *reinterpret_cast<uint32_t*>(at + kRows * kld) = d1;
       *reinterpret_cast<uint32_t*>(at + 2 * kRows * kld) = d2;
     }
-    if (lane == 0) s_fm[lr] = ldexpf(1.f, sc.e - 21);
+    if (lane == 0) s_fm[lr] = sc.unit;
   }
   nd::lds_barrier();
 

@@ -333,10 +333,9 @@ def test_matmul_rows_of_small_values(hip, rows, n, k, offset):
     """Rows whose largest element is subnormal or below 2^-106 (their digits'
     reciprocal unit is no float), digitized apart (few rows, x off the 16-byte
     grid) and inside the product, plain and added into y.  Bound: the digits
-    keep 2^-22 of the row's largest element or any subnormal exactly, the
-    factors and the sum round a few times: 2^-21 of the row maximum times the
-    absolute weights plus 2^-21 of the values, and 2^-147 for roundings to the
-    last bit of a subnormal."""
+    keep 2^-22 of the row's largest element or 2^-127, the factors and the sum
+    round a few times: 2^-21 of the row maximum, and 2^-126, times the absolute
+    weights plus 2^-21 of the values."""
     say("matmul small rows", rows, n, k, offset)
     w, s = synth.int8_matrix(74, f"small{n}x{k}", n, k, k)
     x = synth.Stream(74, f"sx{k}r{rows}").normal((rows, k))
@@ -349,7 +348,8 @@ def test_matmul_rows_of_small_values(hip, rows, n, k, offset):
     full = w.astype(np.float64) * s.astype(np.float64)
     want = x.astype(np.float64) @ full.T
     top = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
-    bound = 2.0 ** -21 * (top * np.abs(full).sum(axis=1)[None] + np.abs(want)) + 2.0 ** -147
+    rows_of = (2.0 ** -21 * top + 2.0 ** -126) * np.abs(full).sum(axis=1)[None]
+    bound = rows_of + 2.0 ** -21 * np.abs(want)
     for times in (1, 2):
         hip._check(hip.lib.nd_matmul_d(hip.ctx, mat, dx.ptr.value + 4 * offset, rows, dy.ptr,
                                        times - 1, None))
