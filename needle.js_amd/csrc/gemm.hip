@@ -65,13 +65,26 @@ __device__ __forceinline__ void digit_words(uint32_t a, uint32_t b, uint32_t c, 
 // 2^-126, whose reciprocal is still a float: values are carried to 2^-22 of
 // the row's largest, or to 2^-127 in a row below 2^-105 (bringing such rows
 // up first would keep their bits, and cost every product 1%: the waves wait
-// for their rows' scales).
+// for their rows' scales).  A row with an infinity or a NaN (the maxima here
+// propagate it) has no digits: its unit is NaN, and so is every product with
+// it.
 struct DigitScale {
   float unit, up;
 };
 __device__ __forceinline__ DigitScale digit_scale(float amax) {
   const uint32_t f = max((__float_as_uint(amax) >> 23) & 0xffu, 22u);
-  return {__uint_as_float((f - 21) << 23), __uint_as_float((275 - f) << 23)};
+  return {f < 255 ? __uint_as_float((f - 21) << 23) : __builtin_nanf(""),
+          __uint_as_float((275 - f) << 23)};
+}
+__device__ __forceinline__ float nan_max(float a, float b) {
+  return __builtin_elementwise_maximum(a, b);
+}
+// Maximum over the lane's row of 16, on all of its lanes.
+__device__ __forceinline__ float row_nan_max(float v) {
+  v = nan_max(v, nd::dpp<nd::kQuadXor1>(v));
+  v = nan_max(v, nd::dpp<nd::kQuadXor2>(v));
+  v = nan_max(v, nd::dpp<nd::kHalfMirror>(v));
+  return nan_max(v, nd::dpp<nd::kRowMirror>(v));
 }
 
 // MS m-subtiles of 16 and NS n-subtiles of 16 per wave; 4 waves split n.
@@ -283,11 +296,11 @@ __global__ __launch_bounds__(256) void digitize_kernel(const float* __restrict__
   }
   float amax = 0.f;
 #pragma unroll
-  for (uint32_t i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-  for (int o = 32; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  for (uint32_t i = 0; i < 8; ++i) amax = nan_max(amax, fabsf(v[i]));
+  for (int o = 32; o >= 1; o >>= 1) amax = nan_max(amax, __shfl_xor(amax, o, 64));
   if ((t & 63) == 0) red[4 + (t >> 6)] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+  amax = nan_max(nan_max(red[4], red[5]), nan_max(red[6], red[7]));
   const DigitScale sc = digit_scale(amax);
   const size_t plane = (size_t)M * K;
 #pragma unroll
@@ -349,11 +362,11 @@ __global__ __launch_bounds__(256) void digitize_rows_kernel(const float* __restr
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < VEC; ++i)
-    amax = fmaxf(fmaxf(fmaxf(amax, fabsf(v[i].x)), fabsf(v[i].y)),
-                   fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
-  amax = nd::row_max(amax);
-  amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
-                 fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
+    amax = nan_max(nan_max(nan_max(amax, fabsf(v[i].x)), fabsf(v[i].y)),
+                   nan_max(fabsf(v[i].z), fabsf(v[i].w)));
+  amax = row_nan_max(amax);
+  amax = nan_max(nan_max(nd::readlane(amax, 0), nd::readlane(amax, 16)),
+                 nan_max(nd::readlane(amax, 32), nd::readlane(amax, 48)));
   const DigitScale sc = digit_scale(amax);
   const size_t plane = (size_t)M * K;
   uint32_t* d0p = reinterpret_cast<uint32_t*>(D + (size_t)m * K);
@@ -518,8 +531,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_f32a_kernel(
   for (int c = 0; c < CPW; ++c) {
     float amax = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[c][i]));
-    amax = nd::row_max(amax);
+    for (int i = 0; i < 16; ++i) amax = nan_max(amax, fabsf(v[c][i]));
+    amax = row_nan_max(amax);
     const DigitScale sc = digit_scale(amax);
     const float up = live ? sc.up : 0.f;
     uint32_t d0w[4], d1w[4], d2w[4];
@@ -749,11 +762,11 @@ __global__ __launch_bounds__(512) void gemm_i8_rows_kernel(
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < VEC; ++i)
-      amax = fmaxf(fmaxf(fmaxf(amax, fabsf(v[r][i].x)), fabsf(v[r][i].y)),
-                     fmaxf(fabsf(v[r][i].z), fabsf(v[r][i].w)));
-    amax = nd::row_max(amax);
-    amax = fmaxf(fmaxf(nd::readlane(amax, 0), nd::readlane(amax, 16)),
-                   fmaxf(nd::readlane(amax, 32), nd::readlane(amax, 48)));
+      amax = nan_max(nan_max(nan_max(amax, fabsf(v[r][i].x)), fabsf(v[r][i].y)),
+                     nan_max(fabsf(v[r][i].z), fabsf(v[r][i].w)));
+    amax = row_nan_max(amax);
+    amax = nan_max(nan_max(nd::readlane(amax, 0), nd::readlane(amax, 16)),
+                   nan_max(nd::readlane(amax, 32), nd::readlane(amax, 48)));
     const DigitScale sc = digit_scale(amax);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {

@@ -356,3 +356,24 @@ def test_matmul_rows_of_small_values(hip, rows, n, k, offset):
         hip._check(hip.lib.nd_sync(hip.ctx))
         err = np.abs(dy.read().astype(np.float64) - times * want)
         assert np.all(err <= times * bound), (times, np.max(err / bound))
+
+
+@pytest.mark.parametrize("rows,n,k", [(5, 70, 256), (64, 300, 2048), (130, 300, 512),
+                                      (600, 512, 1024)])
+def test_matmul_rows_that_are_not_finite(hip, rows, n, k):
+    """An infinity or a NaN anywhere in a row of x makes that row's products
+    NaN, and no other row's: those keep their bits."""
+    say("matmul non-finite rows", rows, n, k)
+    w, s = synth.int8_matrix(75, f"nan{n}x{k}", n, k, k)
+    x = synth.Stream(75, f"nanx{k}r{rows}").normal((rows, k))
+    m = Int8Matrix(w, s, k)
+    want = matmul(hip, m, x)
+    bad = {1: (np.nan, 0), 2: (np.inf, k - 1), 4: (-np.inf, k // 2 + 3), rows - 2: (np.nan, k - 66)}
+    for row, (value, col) in bad.items():
+        x[row, col] = value
+    got = matmul(hip, m, x)
+    for row in range(rows):
+        if row in bad:
+            assert np.isnan(got[row]).all(), row
+        else:
+            assert np.array_equal(got[row].view(np.uint32), want[row].view(np.uint32)), row
