@@ -279,6 +279,15 @@ nd_status nd_attention_static_d(nd_ctx* ctx, const nd_kv* kv, uint32_t layer, ui
                                 const float* q_dev, uint32_t q_heads, float* out_dev,
                                 void* stream);
 
+/* The prompt attention of nd_prefill_run and the Needle 2 prompts by itself:
+ * query rows q [rows][q_heads][64] of positions [position, position + rows),
+ * each over the positions it sees, to out (same shape).  Test hook: int8 caches
+ * whose positions sit in their own slots, 1 or 2 query heads per KV head, at
+ * least 64 rows (ND_ERR_INVALID otherwise). */
+nd_status nd_test_prompt_attention_d(nd_ctx* ctx, const nd_kv* kv, uint32_t layer,
+                                     uint32_t position, uint32_t rows, const float* q_dev,
+                                     uint32_t q_heads, float* out_dev, void* stream);
+
 /* ------------------------------------------- a4: masked argmax selection */
 
 /* selectToken (model/runtime.ts:880-899) with argmax (model/math.ts:140-151)

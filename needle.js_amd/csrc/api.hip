@@ -880,6 +880,27 @@ nd_status nd_attention_d(nd_ctx* ctx, const nd_kv* kv, uint32_t layer, uint32_t 
   return ND_OK;
 }
 
+nd_status nd_test_prompt_attention_d(nd_ctx* ctx, const nd_kv* kv, uint32_t layer,
+                                     uint32_t position, uint32_t rows, const float* q,
+                                     uint32_t q_heads, float* out, void* stream) {
+  if (!ctx) return nd_fail(nullptr, ND_ERR_BACKEND, "context is NULL");
+  if (rows == 0 || position + rows < rows)
+    return nd_fail(ctx, ND_ERR_INVALID, "%u rows from position %u", rows, position);
+  const uint32_t last = position + rows - 1;
+  nd_status st = check_attention(ctx, kv, layer, last, q_heads);
+  if (st != ND_OK) return st;
+  const uint32_t rep = q_heads / kv->kv_heads;
+  if (!q || !out || (reinterpret_cast<uintptr_t>(q) & 15) ||
+      (reinterpret_cast<uintptr_t>(out) & 15) || !nd_prompt_attention_fits(kv, rows, rep, last))
+    return nd_fail(ctx, ND_ERR_INVALID,
+                   "the prompt attention takes 16-byte aligned q and out, an int8 cache whose "
+                   "positions sit in their own slots, 1 or 2 query heads per KV head and 64 rows "
+                   "or more");
+  ND_HIP(ctx, nd_launch_attention_batch(kv, layer, nullptr, rows, kv->kv_heads, 0, rep, last, q,
+                                        out, nullptr, nullptr, nd_pick_stream(ctx, stream)));
+  return ND_OK;
+}
+
 nd_status nd_attention_stamped_d(nd_ctx* ctx, const nd_kv* kv, uint32_t layer, uint32_t position,
                                  const float* q, uint32_t q_heads, float* out, uint64_t* stamps,
                                  uint32_t capacity, uint32_t* workgroups, void* stream) {

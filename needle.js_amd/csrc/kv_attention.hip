@@ -171,17 +171,21 @@ struct AttnLaunch {
 // Bound by the LDS traffic and the vector ALU (softmax, the fp16 halves of p',
 // the conversion): a thread converts four keys of eight dimensions, 12 wide
 // stores, where one dimension of V at a time took 36.  And by the causal
-// triangle: the last row blocks walk every key and the first one block.  A CU holds two workgroups, so a launch of up to 512 goes out heavy
-// blocks first, then the light ones in the opposite order, and each CU's pair
-// has about the same work; 64-row workgroups, one to a CU, left half of the
-// CUs' time idle (2048 positions, 8 heads: 33.7 us).
+// triangle: the last row blocks walk every key and the first one block.  A CU
+// holds two workgroups, so a launch of up to 512 goes out heavy blocks first,
+// then the light ones in the opposite order, and each CU's pair has about the
+// same work; 64-row workgroups, one to a CU, left half of the CUs' time idle
+// (2048 positions, 8 heads: 33.7 us).
+// Error against 64 bits, 320 visible keys, q and K of unit variance: 1.63e-7,
+// the single-row kernel 1.68e-7 (2.54e-7 with the low halves of p' rounded
+// toward zero, those of q multiplied last and log2 e in the key scales).
 // Per block and wave:
 //   S^T = K Q^T on v_mfma_f32_16x16x32_f16: A = K codes (row = key, exact in
-//   fp16), B = Q^T split into fp16 halves hi + lo of q * 2^-e (e: the row's
-//   largest magnitude, < 2^e), which hold q to 2^-24 of the row maximum; the
-//   product lands as lane l holding keys 4 (l / 16) + c of each 16-key tile
-//   for its own row;
-//   scores in base 2: (S * (k_scale / 8 * log2 e)) * 2^e, causal mask,
+//   fp16), B = Q^T split into fp16 halves hi + lo of q' * 2^-e, q' = q / 8 *
+//   log2 e (e: the row's largest magnitude, < 2^e), which hold q' to 2^-23 of
+//   itself or 2^-25 of the row maximum; the product lands as lane l holding
+//   keys 4 (l / 16) + c of each 16-key tile for its own row;
+//   scores in base 2: (S * k_scale) * 2^e, causal mask,
 //   online softmax in fp32 with v_exp_f32 (2^x; results below 2^-126 flush
 //   to zero, as with __expf) -- NeedleRuntime.#attention
 //   (model/runtime.ts:719-786, softmaxInPlace model/math.ts:46-60) with its
@@ -199,7 +203,7 @@ constexpr uint32_t kVtStrideH = 72;  // halves per dim row of V^T in LDS
 struct PfBuf {
   _Float16 k[kPfKeys * kKStrideH];
   _Float16 vt[kHeadDim * kVtStrideH];
-  float ks[kPfKeys];  // k_scale / 8 * log2 e
+  float ks[kPfKeys];  // k_scale
   float vs[kPfKeys];  // v_scale * 2^f
 };
 
@@ -216,7 +220,9 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
   using nd::half8;
   using nd::float4v;
   using nd::u32x2;
+  using nd::half2v;
   typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+  typedef float float2v __attribute__((ext_vector_type(2)));
   __shared__ __align__(16) PfBuf s_buf[kPfGroups];
   __shared__ float s_vmax[kPfThreads / 64];
   const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
@@ -302,7 +308,14 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
       if (key[u] < top && seen(key[u])) vmax = fmaxf(vmax, vs[u]);
   }
 
-  // The split of q: the row maximum over the four lanes holding the row.
+  // The split of q, scaled for scores in base 2 (64 roundings of its elements
+  // weigh less in a score than one of the key's scale): the row maximum over
+  // the four lanes holding the row.
+  const float q_mul = score_scale * 1.4426950408889634f;
+#pragma unroll
+  for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qv[s2][e] *= q_mul;
   float qmax = 0.f;
 #pragma unroll
   for (int s2 = 0; s2 < 2; ++s2)
@@ -335,7 +348,6 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
   int fe = 0;
   if (vsmax > 0.f && vsmax <= 3.4028235e38f) frexpf(vsmax, &fe);  // vsmax < 2^fe
   const float pup = ldexpf(1.f, 15 - fe), pdown = ldexpf(1.f, fe - 15);
-  const float ks_mul = score_scale * 1.4426950408889634f;  // scores in base 2
 
   auto store_block = [&](PfBuf& B) {
 #pragma unroll
@@ -367,7 +379,7 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
       }
     }
     if (tg < kPfKeys) {
-      B.ks[tg] = ksr * ks_mul;
+      B.ks[tg] = ksr;
       B.vs[tg] = vsr * pup;
     }
   };
@@ -389,13 +401,18 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         sc[j] = float4v{0.f, 0.f, 0.f, 0.f};
+        half8 ka[2];
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const half8 ka =
+        for (int s2 = 0; s2 < 2; ++s2)
+          ka[s2] =
               *reinterpret_cast<const half8*>(&B.k[(16 * j + r16) * kKStrideH + 32 * s2 + 8 * kb]);
-          sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh[s2], sc[j], 0, 0, 0);
-          sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[s2], sc[j], 0, 0, 0);
-        }
+        // The low halves first: the sum is rounded at its full size only twice.
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+          sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[s2], ql[s2], sc[j], 0, 0, 0);
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+          sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[s2], qh[s2], sc[j], 0, 0, 0);
       }
       const bool masked = k0 + kPfKeys - 1 > wmin || (WIN && k0 < wlow);  // uniform over the wave
       float bmax = -INFINITY;
@@ -451,13 +468,14 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
                              sc[2 * s2][2] * va.z,     sc[2 * s2][3] * va.w,
                              sc[2 * s2 + 1][0] * vb.x, sc[2 * s2 + 1][1] * vb.y,
                              sc[2 * s2 + 1][2] * vb.z, sc[2 * s2 + 1][3] * vb.w};
-        // hi = pv rounded toward zero to fp16, lo = fp16 of the (exact f32)
-        // remainder: |pv - hi - lo| <= 2^-22 |pv| while lo is normal.
+        // hi = pv rounded to the nearest fp16, lo = that of the (exact f32)
+        // remainder: |pv - hi - lo| <= 2^-23 |pv| while lo is normal.
         half8 ph, pl;
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
-          const auto hv = __builtin_amdgcn_cvt_pkrtz(pv[e], pv[e + 1]);
-          const auto lv = __builtin_amdgcn_cvt_pkrtz(pv[e] - (float)hv[0], pv[e + 1] - (float)hv[1]);
+          const half2v hv = __builtin_convertvector(float2v{pv[e], pv[e + 1]}, half2v);
+          const half2v lv = __builtin_convertvector(
+              (float2v{pv[e] - (float)hv[0], pv[e + 1] - (float)hv[1]}), half2v);
           ph[e] = hv[0];
           ph[e + 1] = hv[1];
           pl[e] = lv[0];
@@ -774,6 +792,14 @@ hipError_t nd_launch_attention(const nd_kv* kv, uint32_t layer, uint32_t positio
   return kv->mode == ND_KV_FLOAT32 ? launch_rep<true>(a, s) : launch_rep<false>(a, s);
 }
 
+// Positions sit in their own slots while no window is outgrown (they then also
+// see all of [0, position]) and in a linear cache.
+bool nd_prompt_attention_fits(const nd_kv* kv, uint32_t rows, uint32_t rep,
+                              uint32_t max_position) {
+  return (nd_kv_linear(kv) || max_position < kv->window) && (rep == 1 || rep == 2) &&
+         kv->mode != ND_KV_FLOAT32 && rows >= 64;
+}
+
 // Batched form: query row z reads cache heads [z * kv_stride_z, +seq_kv_heads)
 // (kv_stride_z = seq_kv_heads for a batch of sequences, 0 for the positions of
 // one prefill, consecutive and ending at max_position) with queries
@@ -802,10 +828,7 @@ hipError_t nd_launch_attention_batch(const nd_kv* kv, uint32_t layer, const uint
   a.batch = batch;
   a.max_count = nv.count;
   a.first_position = max_position + 1 - batch;
-  // Positions sit in their own slots while no window is outgrown (they then
-  // also see all of [0, position]) and in a linear cache.
-  a.qblock = kv_stride_z == 0 && (nd_kv_linear(kv) || max_position < kv->window) &&
-             (rep == 1 || rep == 2) && kv->mode != ND_KV_FLOAT32 && batch >= 64;
+  a.qblock = kv_stride_z == 0 && nd_prompt_attention_fits(kv, batch, rep, max_position);
   return kv->mode == ND_KV_FLOAT32 ? launch_rep<true>(a, s) : launch_rep<false>(a, s);
 }
 

@@ -297,6 +297,9 @@ hipError_t nd_launch_gemm_f32(const nd_mat* w, const float* x, uint32_t ldx, con
                               float* y, uint32_t ldy, uint32_t M, int epilogue, hipStream_t s,
                               const nd_gemm_split* split,
                               const nd::RopeStore* rope = nullptr);
+// Whether `rows` consecutive positions ending at max_position take the prompt
+// attention (MFMA) of nd_launch_attention_batch.
+bool nd_prompt_attention_fits(const nd_kv* kv, uint32_t rows, uint32_t rep, uint32_t max_position);
 hipError_t nd_launch_attention_batch(const nd_kv* kv, uint32_t layer, const uint32_t* positions,
                                      uint32_t batch, uint32_t seq_kv_heads, uint32_t kv_stride_z,
                                      uint32_t rep, uint32_t max_position, const float* q,

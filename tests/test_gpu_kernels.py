@@ -16,6 +16,7 @@ import pytest
 import oracle
 from helpers import DeviceArray, assert_close
 from needle_hip import HipKvCache, Int8Matrix, MatrixRowRange, MatvecRequest, NeedleError
+from needle_hip import lib as L
 from needle_hip import synth
 
 pytestmark = pytest.mark.gpu
@@ -437,3 +438,43 @@ def test_matvec_rows_of_subnormals(hip, n, k, g, batch):
     want = x.astype(np.float64) @ full.T
     bound = 2.0 ** -18 * (np.abs(x).astype(np.float64) @ np.abs(full).T) + 2.0 ** -148
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
+
+
+@pytest.mark.parametrize("kv_heads,rep,length,size", [(4, 2, 320, 1.0), (4, 2, 320, 4.0),
+                                                      (4, 1, 200, 0.2)])
+def test_prompt_attention_is_as_exact_as_a_step(hip, kv_heads, rep, length, size):
+    """A prompt's attention against 64 bits, beside the single-row kernel that a
+    step of the same position runs: an error no larger over all rows (within
+    the 5% that 256 rows of 8 heads leave to chance) and no more bias."""
+    say("prompt attention error", kv_heads, rep, length, size)
+    rows, heads = min(256, length - 10), kv_heads * rep
+    first = length - rows
+    s = synth.Stream(63, f"pa{kv_heads}{rep}{length}{size}")
+    kv = HipKvCache(hip, 1, kv_heads, max_length=length)
+    kv.store(0, 0, s.normal((length, kv_heads, 64)), s.normal((length, kv_heads, 64)))
+    q = s.normal((rows, heads, 64)) * np.float32(size)
+    dq, dp, ds = DeviceArray(q), DeviceArray(np.zeros_like(q)), DeviceArray(np.zeros_like(q))
+    hip._check(hip.lib.nd_test_prompt_attention_d(hip.ctx, kv.handle, 0, first, rows, dq.ptr, heads,
+                                                  dp.ptr, None))
+    for r in range(rows):
+        at = 4 * r * heads * 64
+        hip._check(hip.lib.nd_attention_d(hip.ctx, kv.handle, 0, first + r, dq.ptr.value + at, heads,
+                                          ds.ptr.value + at, None))
+    hip._check(hip.lib.nd_sync(hip.ctx))
+    want = np.zeros((rows, heads, 64))
+    for h in range(kv_heads):
+        kc, vc, ks, vs = (np.asarray(a, np.float64) for a in kv.read(0, h))
+        k, v = kc * ks[:, None], vc * vs[:, None]
+        for g in range(h * rep, (h + 1) * rep):
+            sc = q[:, g].astype(np.float64) @ k.T / 8
+            sc[np.arange(length)[None] > first + np.arange(rows)[:, None]] = -np.inf
+            p = np.exp(sc - sc.max(axis=1, keepdims=True))
+            want[:, g] = (p @ v) / p.sum(axis=1, keepdims=True)
+    d = {name: a.read().astype(np.float64) - want for name, a in (("prompt", dp), ("step", ds))}
+    err = {name: np.linalg.norm(e) / np.linalg.norm(want) for name, e in d.items()}
+    bias = {name: abs((e * want).sum() / (want * want).sum()) for name, e in d.items()}
+    say(f"[measure] errors {err} bias {bias}")
+    assert err["prompt"] <= 1.05 * err["step"] and bias["prompt"] <= 3e-8, (err, bias)
+    assert hip.lib.nd_test_prompt_attention_d(hip.ctx, kv.handle, 0, 0, 63, dq.ptr, heads, dp.ptr,
+                                              None) == L.ND_ERR_INVALID
+    kv.free()
