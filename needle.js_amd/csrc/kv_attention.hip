@@ -325,6 +325,7 @@ __global__ __launch_bounds__(kPfThreads, 4) void prefill_attention_mfma_kernel(
   qmax = nd::max_xor<32>(qmax);
   int qe = 0;
   if (qmax > 0.f && qmax <= 3.4028235e38f) frexpf(qmax, &qe);  // qmax < 2^qe
+  qe = max(qe, -126);  // 2^-qe stays finite; such a row is left exact
   const float qdown = ldexpf(1.f, -qe), qup = ldexpf(1.f, qe);
   half8 qh[2], ql[2];
 #pragma unroll

@@ -478,3 +478,25 @@ def test_prompt_attention_is_as_exact_as_a_step(hip, kv_heads, rep, length, size
     assert hip.lib.nd_test_prompt_attention_d(hip.ctx, kv.handle, 0, 0, 63, dq.ptr, heads, dp.ptr,
                                               None) == L.ND_ERR_INVALID
     kv.free()
+
+
+def test_prompt_attention_rows_of_subnormals(hip):
+    """Query rows whose largest element is subnormal, all zeros or ordinary: the
+    first two weigh every position alike."""
+    say("prompt attention subnormal rows")
+    length, heads = 100, 2
+    s = synth.Stream(64, "pasub")
+    kv = HipKvCache(hip, 1, heads, max_length=length)
+    kv.store(0, 0, s.normal((length, heads, 64)), s.normal((length, heads, 64)))
+    q = s.normal((length, heads, 64))
+    q[::3] *= np.float32(1e-41)
+    q[1::3] = 0.0
+    dq, dp = DeviceArray(q), DeviceArray(np.zeros_like(q))
+    hip._check(hip.lib.nd_test_prompt_attention_d(hip.ctx, kv.handle, 0, 0, length, dq.ptr, heads,
+                                                  dp.ptr, None))
+    hip._check(hip.lib.nd_sync(hip.ctx))
+    got = dp.read()
+    for r in range(length):
+        want = kv.attention(0, r, q[r].reshape(-1)).reshape(heads, 64)
+        assert_close(got[r], want, 1e-5, 1e-6, f"row {r}")
+    kv.free()
