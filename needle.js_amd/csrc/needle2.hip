@@ -3400,12 +3400,18 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
   if (n->cq && (e = enqueue_cq_rows(n, n->pf_cq_lookup + lk - 1, n->pf_cq_lookup, s, M)) !=
                    hipSuccess)
     return e;
-  // The batch's products: digit-sliced int8 GEMMs, or for a Cactus-Quant
-  // model the CQ matvec over the M rows (the step's arithmetic per row).
+  // The batch's products: digit-sliced int8 GEMMs (22 bits of a row's largest
+  // element) or, over the prompt cache, whose positions would otherwise be
+  // steps, products that keep each element's own bits as the step's do; for a
+  // Cactus-Quant model the CQ matvec over the M rows.
+  const bool past_ring = kv.window && nd_kv_linear(&kv);
   auto product = [&](const nd_mat* w, const float* x, uint32_t x_ld, uint32_t k, float* y,
                      uint32_t y_ld) -> hipError_t {
     if (w->bits)
       return nd_launch_cq_matvec(w, x, M, x_ld, nullptr, 0, w->n, y, y_ld, s);
+    if (past_ring && nd_batch_matvec_fits(w, M))
+      return nd_launch_batch_matvec(w, x, M, x_ld, 0, w->n, y, y_ld, s, nullptr);
+    if (past_ring) return nd_launch_matvec(w, x, M, x_ld, 0, w->n, y, y_ld, s);
     if (nd_gemm_rows_fits(w, x, x_ld, false, M))
       return nd_launch_gemm_rows(w, x, x_ld, nullptr, y, y_ld, M, 0, s);
     hipError_t r = nd_launch_digitize(x, x_ld, nullptr, nullptr, n->pf_digits, n->pf_fm, M, k, s);

@@ -711,3 +711,32 @@ def test_prompt_passes_shrink_to_the_memory(hip):
         close(rt.prefill(tokens), want, "prompt")
     finally:
         model.dispose()
+
+
+@pytest.mark.parametrize("window", [8, 80])
+def test_prompt_past_the_ring_keeps_small_activations(hip, window):
+    """Positions past the ring were steps, whose products keep every element of
+    a row.  A normed activation of 1e5 that no weight takes up must not cost its
+    neighbours their bits when the prompt runs as a pass either (22 bits of the
+    row's largest would leave two digits of them)."""
+    say("needle2 small activations", window)
+    g = Needle2Geometry(**{**SMALL.__dict__, "kv_window": window, "max_length": 160})
+    w = Needle2Weights(g, 48)
+    w.norm_input[:, 5] = 1e5
+    for mats in (w.wq, w.wk, w.wv, w.wgate):
+        for m in mats:
+            m.codes[:, 5] = 0
+    model = NeedleModel(hip, w)
+    try:
+        rt = model.create_resident_runtime()
+        tokens = synth.Stream(18, "n2small").integers(150, 0, g.vocab - 1)
+        rt.reset(g.max_length, 3)
+        ref = oracle.Needle2(w).runtime(g.max_length, 3)
+        ref.capture_kv(0, g.max_length)
+        got = rt.prefill(tokens)
+        for t in tokens:
+            want = ref.step(int(t))
+        close(got, want, "prompt")
+        check_kv(model, ref, g, 150, 3, "prompt with a large activation")
+    finally:
+        model.dispose()
