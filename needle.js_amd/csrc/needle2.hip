@@ -3532,45 +3532,34 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
   return nd_launch_select_list(n->logits, d.vocab, nullptr, 0, n->sel_id, n->sel_lp, s);
 }
 
-// Float32 cache rows that the reset's memory holds per layer and KV head: the
-// model's longest runtime and, for a model with a window, a ring of up to
-// kRingSinks sinks beside it (prompt_cache).
-constexpr uint32_t kRingSinks = 64;
-uint32_t cache_rows(const nd_needle_desc& d) {
-  const uint64_t ring = d.kv_window ? std::min((uint64_t)d.max_length,
-                                               (uint64_t)d.kv_window + kRingSinks) : 0;
-  return (uint32_t)std::min(d.max_length + ring, (uint64_t)~0u);
-}
-
-// The linear prompt cache of a prompt that ends at position `end` past the
-// ring, in the part of the reset's cache memory that the ring leaves unused:
-// a call allocates nothing.  An int8 ring takes at most the first quarter of
-// arrays sized for float32 rows, its prompt cache the second and the start of
-// the third.  A float32 ring's follows it; false when its rows do not reach
-// `end` (more than kRingSinks sinks and a prompt near the model's limit).
-bool prompt_cache(const nd_needle* n, uint32_t end, nd_kv* lin) {
+// The linear prompt cache of prompts that outgrow the ring, in the part of the
+// reset's cache memory (float32 rows for the model's longest runtime) that the
+// ring leaves unused: a call allocates nothing.  An int8 ring takes at most the
+// first quarter of it, its prompt cache the second and the start of the third.
+// A float32 ring's follows it, so that its last positions are past it.  False
+// without more than sink + window slots, the mark of a linear cache.
+bool prompt_cache(const nd_needle* n, nd_kv* lin) {
   const nd_kv& kv = n->kv;
-  const uint32_t rows = cache_rows(n->d);
+  const uint32_t rows = n->d.max_length;
   const size_t heads = (size_t)n->d.layers * n->d.kv_heads;
   *lin = kv;
   if (kv.mode == ND_KV_FLOAT32) {
-    if (rows - kv.alloc < end) return false;
     lin->alloc = rows - kv.alloc;
     lin->k = reinterpret_cast<float*>(kv.k) + heads * kv.alloc * kHd;
     lin->v = reinterpret_cast<float*>(kv.v) + heads * kv.alloc * kHd;
     lin->ks = kv.ks + heads * kv.alloc;
     lin->vs = kv.vs + heads * kv.alloc;
-    return true;
+  } else {
+    lin->alloc = rows;
+    auto quarter = [&](void* base, size_t i) {
+      return reinterpret_cast<char*>(base) + i * heads * rows * kHd;
+    };
+    lin->k = quarter(kv.k, 1);
+    lin->v = quarter(kv.v, 1);
+    lin->ks = reinterpret_cast<float*>(quarter(kv.k, 2));
+    lin->vs = reinterpret_cast<float*>(quarter(kv.v, 2));
   }
-  lin->alloc = rows;
-  auto quarter = [&](void* base, size_t i) {
-    return reinterpret_cast<char*>(base) + i * heads * rows * kHd;
-  };
-  lin->k = quarter(kv.k, 1);
-  lin->v = quarter(kv.v, 1);
-  lin->ks = reinterpret_cast<float*>(quarter(kv.k, 2));
-  lin->vs = reinterpret_cast<float*>(quarter(kv.v, 2));
-  return true;
+  return kv.window && lin->alloc > kv.sink + kv.window;
 }
 
 // Copies rows between the ring and the linear prompt cache lin: positions
@@ -3606,14 +3595,17 @@ nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits
   hipStream_t s = ctx->stream;
   uint32_t done = 0;
   const uint32_t fit = n->kv.alloc > n->position ? n->kv.alloc - n->position : 0;
-  nd_kv lin;  // more than sink + window slots, the mark of a linear cache
-  if (count > fit && count - fit > kStepRest && prompt_cache(n, n->position + count, &lin)) {
+  nd_kv lin;
+  uint32_t past = 0;  // positions of the prompt that work on the prompt cache
+  if (count > fit && prompt_cache(n, &lin) && lin.alloc > n->position)
+    past = std::min(count, lin.alloc - n->position);
+  if (past > fit && past - fit > kStepRest) {
     const uint32_t first = n->position;
     hipError_t e = first ? enqueue_ring_copy(n, lin, 0, first, false, s) : hipSuccess;
-    const uint32_t passes = (count + n->pf_cap - 1) / n->pf_cap;
+    const uint32_t passes = (past + n->pf_cap - 1) / n->pf_cap;
     for (uint32_t i = 0; i < passes && e == hipSuccess; ++i) {  // even passes: no short last one
-      const uint32_t chunk = (count - done + (passes - i) - 1) / (passes - i);
-      const bool last = i + 1 == passes;
+      const uint32_t chunk = (past - done + (passes - i) - 1) / (passes - i);
+      const bool last = done + chunk == count;
       e = enqueue_prefill(n, lin, chunk, last && want_logits, last && select, s);
       if (e != hipSuccess) break;
       n->position += chunk;
@@ -3623,7 +3615,6 @@ nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits
     // of a later one.
     const hipError_t back = enqueue_ring_copy(n, lin, first, n->position, true, s);
     ND_HIP(ctx, e != hipSuccess ? e : back);
-    return ND_OK;
   }
   while (done < count) {
     const uint32_t left = count - done;
@@ -3636,7 +3627,7 @@ nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits
       done += chunk;
       continue;
     }
-    // Positions past the ring, few or without a prompt cache: a step per token.
+    // Positions past the ring, few or past the prompt cache: a step per token.
     const bool last = left == 1;
     if (graphs) {
       if ((st = launch_graph(ctx, n, last && (want_logits || select) ? kGraphPromptSelect
@@ -4002,7 +3993,7 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
   if (!n->arena) {
     // Sized for the model's max_length so that later resets never allocate.
     const uint32_t cap = d.max_length;
-    const size_t rows = (size_t)d.layers * d.kv_heads * cache_rows(d);
+    const size_t rows = (size_t)d.layers * d.kv_heads * cap;
     const size_t pf = nd_attention_batch_partial_floats(1, d.kv_heads, d.heads / d.kv_heads, cap);
     const uint32_t S = d.n_sites ? d.n_sites : 1;
     const uint32_t cat = d.n_sites ? d.engram_tables * d.engram_sub : 1;
@@ -4015,7 +4006,7 @@ nd_status nd_needle_reset(nd_ctx* ctx, nd_needle* n, uint32_t max_length, uint32
                             al((size_t)d.layers * 128), al(128),
                             cb * al(P8 * kMaxChunks), cb * al(P8 * kMaxChunks),
                             cb * al(P8 * D), al(64), al(64),
-                            // K and V sized for float32 rows (kvCache "float32"; cache_rows)
+                            // K and V sized for float32 rows (kvCache "float32")
                             al((size_t)d.vocab * 4), al((size_t)(d.vocab + 31) / 32 * 4), al(rows * kHd * 4), al(rows * kHd * 4),
                             al(rows * 4),
                             al(rows * 4), al((size_t)ln * D * 4), al(D * 4), al(D * 4), al(D * 4),

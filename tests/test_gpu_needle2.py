@@ -641,14 +641,15 @@ def test_steps_of_a_deep_model_pool_without_a_prompt(hip, layers):
 @pytest.mark.parametrize("mode,window,sink,length", [("int8", 40, 5, 300), ("int8", 40, 5, 20000),
                                                      ("float32", 40, 5, 300),
                                                      ("float32", 40, 5, 20000),
-                                                     ("float32", 40, 90, 300)])
+                                                     ("float32", 40, 90, 300),
+                                                     ("float32", 40, 120, 300)])
 def test_prompt_past_the_ring_takes_no_memory(hip, mode, window, sink, length):
     """A prompt past the ring, up to the model's last position or of a model
     whose cache takes 16 MB as int8 codes, works beside the ring in the reset's
     own memory: nothing is allocated (free memory is the same), and logits and
-    cache rows are those of a step per token.  A float32 ring of more than 64
-    sinks leaves no room there for a prompt to the last position: the
-    positions past it run as steps."""
+    cache rows are those of a step per token.  A float32 ring leaves no room
+    there for as many of the model's last positions as it has slots, and one
+    of more than half of the positions for none: those run as steps."""
     say("needle2 prompt cache", mode, window, sink, length)
     total = 300
     g = Needle2Geometry(**{**SMALL.__dict__, "kv_window": window, "max_length": length})
