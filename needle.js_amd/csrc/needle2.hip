@@ -3534,9 +3534,8 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
 
 // The linear prompt cache of prompts that outgrow the ring, in the part of the
 // reset's cache memory (float32 rows for the model's longest runtime) that the
-// ring leaves unused: a call allocates nothing.  An int8 ring takes at most the
-// first quarter of it, its prompt cache the second and the start of the third.
-// A float32 ring's follows it, so that its last positions are past it.  False
+// ring leaves unused: a call allocates nothing.  An int8 ring's keys take at
+// most the first quarter of theirs, its prompt cache the other three.  A float32 ring's follows it, so that its last positions are past it.  False
 // without more than sink + window slots, the mark of a linear cache.
 bool prompt_cache(const nd_needle* n, nd_kv* lin) {
   const nd_kv& kv = n->kv;
@@ -3551,13 +3550,11 @@ bool prompt_cache(const nd_needle* n, nd_kv* lin) {
     lin->vs = kv.vs + heads * kv.alloc;
   } else {
     lin->alloc = rows;
-    auto quarter = [&](void* base, size_t i) {
-      return reinterpret_cast<char*>(base) + i * heads * rows * kHd;
-    };
-    lin->k = quarter(kv.k, 1);
-    lin->v = quarter(kv.v, 1);
-    lin->ks = reinterpret_cast<float*>(quarter(kv.k, 2));
-    lin->vs = reinterpret_cast<float*>(quarter(kv.v, 2));
+    char* at = reinterpret_cast<char*>(kv.k) + heads * rows * kHd;
+    lin->k = at;
+    lin->v = at + heads * rows * kHd;
+    lin->ks = reinterpret_cast<float*>(at + 2 * heads * rows * kHd);
+    lin->vs = lin->ks + heads * rows;
   }
   return kv.window && lin->alloc > kv.sink + kv.window;
 }
