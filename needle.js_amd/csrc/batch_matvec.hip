@@ -28,8 +28,8 @@
 // row); 64 rows x (4096 x 4096, int8): 16.8 us (64.6 eight rows a launch).
 //
 // Split: a chunk's row is scaled by 2^(15 - e), e the exponent of its largest
-// magnitude, hi = f16(v), lo = f16(v - hi): v is kept to 2^-24 of itself, and
-// to 2^-40 of the chunk's largest where lo is subnormal.  int8 codes are
+// magnitude, hi = f16(v), lo = f16(v - hi): v is kept to 2^-23 of itself, and
+// to 2^-39 of the chunk's largest where lo is subnormal.  int8 codes are
 // exact in fp16; a codebook value is hi + lo too, after a factor that the
 // upload picks so that the whole book loses least (nd_split_codebook), and
 // all four products are taken.  fp16 products are exact in the fp32

@@ -181,8 +181,8 @@ __global__ __launch_bounds__(kThreads) void matvec_i8_stamped_kernel(
 // the fp32 inputs split exactly enough.  Each workgroup writes into LDS, per
 // batch row b with e_b = the exponent of max_k |x[b][k]| (max < 2^e_b),
 //   x[b][k] * 2^-e_b = hi + lo,  hi = f16(x * 2^-e_b),  lo = f16(x * 2^-e_b - hi),
-// which leaves at most 2^-24 of the row's largest element unrepresented
-// (fp32's own rounding step).  Weights are int8, exact in fp16, and fp16 x
+// which leaves at most 2^-24 2^e_b unrepresented (fp32's own rounding step for
+// the row's largest element).  Weights are int8, exact in fp16, and fp16 x
 // fp16 products are exact in the fp32 MFMA accumulator, so
 //   y[b][r] = 2^e_b * sum_g s[r][g] * (sum_{k in g} W[r][k] (hi + lo)[b][k])
 // differs from the fp32 dot product only by fp32 accumulation rounding.

@@ -3535,8 +3535,10 @@ hipError_t enqueue_prefill(nd_needle* n, const nd_kv& kv, uint32_t count, bool w
 // The linear prompt cache of prompts that outgrow the ring, in the part of the
 // reset's cache memory (float32 rows for the model's longest runtime) that the
 // ring leaves unused: a call allocates nothing.  An int8 ring's keys take at
-// most the first quarter of theirs, its prompt cache the other three.  A float32 ring's follows it, so that its last positions are past it.  False
-// without more than sink + window slots, the mark of a linear cache.
+// most the first quarter of theirs, its prompt cache the other three.  A
+// float32 ring's follows it and so ends that many positions before the model's
+// last.  False without more than sink + window slots, the mark of a linear
+// cache.
 bool prompt_cache(const nd_needle* n, nd_kv* lin) {
   const nd_kv& kv = n->kv;
   const uint32_t rows = n->d.max_length;
@@ -3579,11 +3581,11 @@ hipError_t enqueue_ring_copy(nd_needle* n, const nd_kv& lin, uint32_t first, uin
 // The last token produces logits (and a selection over all ids when select).
 // A prompt whose positions fit the ring's slots runs as passes over the ring;
 // one that outgrows it by more than kStepRest positions as passes over the
-// linear prompt cache, with the rows the ring keeps copied back at the end.
+// linear prompt cache (as far as that reaches), with the rows the ring keeps copied back at the end.
 // A rest of up to kStepRest positions takes steps: a pass costs its launches
 // and one trip through the layers however few its rows (about 1.5 ms at 27
 // layers, against 0.46-0.55 ms a step).  640 CQ4 tokens over a 256-position
-// window, 27 layers: 5.3 ms as one pass, 206 ms with the 384 positions past
+// window, 27 layers: 2.1 ms as one pass, 206 ms with the 384 positions past
 // the ring as steps.
 nd_status run_prompt(nd_ctx* ctx, nd_needle* n, uint32_t count, bool want_logits, bool select,
                      bool graphs) {

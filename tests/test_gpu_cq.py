@@ -216,9 +216,10 @@ def test_cq_many_rows(hip, bits, n, k, g, batch):
     """Batches that take the MFMA form: 16, 32 and 64 rows a tile, rows of x
     of any alignment, a last chunk of one unit, groups narrower than a chunk
     and as wide; a row of zeros, one of subnormals and one of large values.
-    Bound per output: x and the codebook keep 2^-24 and 2^-23 in their fp16
-    halves, the rotation's log2(g) additions and at most 57 more follow, each
-    2^-24 of the absolute sum over the rotation's absolute values: 2^-18."""
+    Bound per output: x and the codebook keep 2^-23 in their fp16 halves, the
+    rotation's at most 8 additions and at most 42 more follow (32 products, 5
+    for the units of a chunk, 5 chunks), each 2^-24 of the absolute sum over the
+    rotation's absolute values: 54 2^-24, within 2^-18."""
     say("cq many rows", n, k, g, bits, batch)
     m = cq(9, n, k, g, bits)
     x = np.random.default_rng(n + k + batch).standard_normal((batch, k)).astype(np.float32)

@@ -402,7 +402,7 @@ def test_matvec_many_rows(hip, n, k, g, batch):
     """Batches above eight (and three rows of a tall matrix) in one launch: a
     half chunk, one chunk, k slices, one row past a tile in each direction,
     batch rows of zeros, of subnormals and near the largest float, and a row
-    range.  Bound per output: the hi/lo split keeps x to 2^-24 and at most 57
+    range.  Bound per output: the hi/lo split keeps x to 2^-23 and at most 57
     fp32 additions follow (32 products, 8 units, up to 16 chunks of a group,
     a slice), each 2^-24 of the absolute sum: 2^-18 of it."""
     say("matvec many rows", n, k, g, batch)
